@@ -82,7 +82,7 @@ def build_driver() -> str:
 def build_oracle() -> None:
     d = os.path.join(ROOT, "oracle")
     _run(["make", "-C", d, "-s", "-B", "liboracle.so"])
-    if os.path.isdir("/root/reference"):
+    if os.path.exists("/root/reference/FD_function.cpp"):   # an empty folder: fixtures stay as committed
         _run(["make", "-C", d, "-s", "-B", "ref"])
 
 
