@@ -27,10 +27,11 @@
 // extractvel1 / extendvel1 (Velocity_function.cpp:2011-2073) as addressing,
 // continued into the field margins.
 // Damping factors are stored with the same margins (index -RTM_MXL.. of the
-// column arrays, -RTM_MZT.. of the row arrays; 1.0 outside the grid) as
-// a = c1/c2 and b = 1/c2 of the reference's c1 = 1 - dt*d/2, c2 = 2 - c1,
-// so that the damped update (c1*v - u)/c2 is fma(a, v, -(u*b)); a = b = 1
-// off the absorbing layer.
+// column arrays, -RTM_MZT.. of the row arrays) as a = c1/c2 and b = 1/c2 of
+// the reference's c1 = 1 - dt*d/2, c2 = 2 - c1, so that the damped update
+// (c1*v - u)/c2 is fma(a, v, -(u*b)); a = b = 1 off the absorbing layer.
+// Outside the velocity grid b = 0, which keeps the velocities there at +0
+// with no test in the kernels.
 // Imaging accumulators g1, illum: nzi x nxl, pitch nxl.
 // Boundary store: nt steps x strip_len values, packed per step as
 //   vx lr [2][nzi][10] | vz tb [2][10][nxl] | p lr [2][nzi][10] | p tb [2][10][nxl]
@@ -53,6 +54,7 @@ enum RtmTileFlag : int {
   TF_REC = 4,     // the tile holds receiver cells
   TF_GEN = 8,     // the tile or its halo leaves the undamped interior (per-cell rules)
   TF_INT = 16,    // reverse phase: the tile holds reconstructed cells (interior or strips)
+  TF_EDGE = 32,   // the tile or its halo holds cells of reduced radius (near the grid's edge)
 };
 
 enum RtmPhase : int { PH_IDLE = 0, PH_FWD = 1, PH_REV = 2 };

@@ -352,8 +352,8 @@ void shot_setup(const rtmh_params& P, const float* vp0, const float* colmax_vv, 
   damping(s.axv, s.bxv, nxp - 1, npml, s.vpmax, P.dx, true, P.dt);
   damping(s.az, s.bz, nzp, npml, s.vpmax, P.dz, false, P.dt);
   damping(s.azv, s.bzv, nzp - 1, npml, s.vpmax, P.dz, true, P.dt);
-  s.axv.push_back(1.0f); s.bxv.push_back(1.0f);              // pad to nxp / nzp
-  s.azv.push_back(1.0f); s.bzv.push_back(1.0f);
+  s.axv.push_back(1.0f); s.bxv.push_back(0.0f);              // pad to nxp / nzp: no velocity there
+  s.azv.push_back(1.0f); s.bzv.push_back(0.0f);
   // Gaussian source (kernel.cu:23-35): bounding box of its non-zero values.
   // expf(-a) is 0 in float for a > 104 (below half the smallest denormal), so
   // only the rectangle around the source where alp^2 dist <= 120 (plus two
@@ -634,7 +634,7 @@ static SmallLayout small_layout(const ShotSetup& s)
   SmallLayout L;
   size_t o = 0;
   // damping arrays carry the field margins: columns -RTM_MXL .. pitch-RTM_MXL-1,
-  // rows -RTM_MZT .. frows-RTM_MZT-1 (value 1 outside the grid)
+  // rows -RTM_MZT .. frows-RTM_MZT-1
   const size_t nx = Engine::pitch_of(s.g.nxp), nz = Engine::frows_of(s.g.nzp);
   const size_t n8[8] = {nx, nx, nx, nx, nz, nz, nz, nz};
   for (int i = 0; i < 8; i++) { L.c[i] = o; o += align256(n8[i] * 4); }
@@ -707,7 +707,9 @@ void Engine::layout_slot(const rtmh_params& P, const ShotSetup& s, int store_fmt
   const int len[8] = {d.pitch, d.pitch, d.pitch, d.pitch, d.frows, d.frows, d.frows, d.frows};
   for (int i = 0; i < 8; i++) {
     float* dst = (float*)(img.data() + L.c[i]);
-    for (int k = 0; k < len[i]; k++) dst[k] = 1.0f;
+    // outside the grid: a = 1, and b = 0 for the velocities (they stay +0)
+    const float out = i == 3 || i == 7 ? 0.0f : 1.0f;
+    for (int k = 0; k < len[i]; k++) dst[k] = out;
     memcpy(dst + pad[i], cv[i]->data(), cv[i]->size() * 4);
   }
   memcpy(img.data() + L.sa, s.sa.data(), s.sa.size() * 4);
@@ -909,6 +911,8 @@ void build_tiles(const std::vector<ShotDev>& ds, int tz, std::vector<Tile>& tile
         // (vx columns x0-10..x0+73, vz rows z0-10..z0+tz+8)
         const bool inside = x0 - 10 >= n && x1 + 10 <= nxp - n - 2 && z0 - 10 >= n && z1 + 9 <= nzp - n - 2;
         if (!inside) f |= TF_GEN;
+        // a stencil radius below 10 somewhere in those velocities or in p
+        if (x0 - 10 <= 9 || x1 + 10 >= nxp - 10 || z0 - 10 <= 9 || z1 + 9 >= nzp - 10) f |= TF_EDGE;
         // reverse phase: reconstructed cells (interior and strips)
         if (hit(0, 0, n - R, nzp - n + R - 1, n - R, nxp - n + R - 1)) f |= TF_INT;
         tiles.push_back(Tile{sid, x0, z0, f});
@@ -1498,6 +1502,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     last_tz = tz;
     last_tz_r = tz_r;
     if (rc) { for (void* p : mem) pool_.put(p); break; }
+    HIPCHK(rtm_launch_image(d_ds, d_slots, nb, 0, st_));
     HIPCHK(hipEventRecord(e2, st_));
     HIPCHK(hipStreamSynchronize(st_));
     if ((rc = guard_check(ds, shots, k0, "reverse")) != 0) { for (void* p : mem) pool_.put(p); break; }

@@ -47,6 +47,13 @@ typedef __attribute__((address_space(1))) unsigned int guint;
 typedef __attribute__((address_space(1))) unsigned short gushort;
 #define GF(p) ((gfloat*)(p))
 #define GCF(p) ((const gfloat*)(p))
+// wave-uniform reads of arrays that no kernel writes while a step runs
+// (damping, coefficients, wavelet, block scales): scalar loads
+#define CCF(p) ((const __attribute__((address_space(4))) float*)(p))
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) f4 gf4;
 
 namespace {
 
@@ -89,25 +96,14 @@ __device__ __forceinline__ int strip_vx(const ShotDev& s, int iz, int ix)
   if (ix >= c0 && ix < c0 + RTM_R) return RTM_R * s.nzi + r * RTM_R + ix - c0;
   return -1;
 }
-// The same offsets split into a row part (wave-uniform: the lanes of a wave
-// share their rows) and a column part (per lane, computed once per tile):
-// own-column cells then cost one add and a compare.
-struct StripCols {
-  int vx;    // vx lr column part, -1 off the vx strip columns
-  int plr;   // p lr column part, -1 off the p strip columns
-  int tb;    // ix - npml on the interior columns (vz / p tb blocks), -1 elsewhere
-};
-__device__ __forceinline__ StripCols strip_cols(const ShotDev& s, int ix)
+// The offsets of the other blocks split into a row part and a column part.
+// column part of the p lr block, -1 off its columns
+__device__ __forceinline__ int strip_col_plr(const ShotDev& s, int ix)
 {
-  const int n = s.npml;
-  const int blr = 2 * RTM_R * s.nzi + 2 * RTM_R * s.nxl;
-  StripCols c;
-  c.vx = (ix >= n - RTM_R && ix < n) ? ix - (n - RTM_R)
-       : ((ix >= s.nxp - n - 1 && ix < s.nxp - n - 1 + RTM_R) ? RTM_R * s.nzi + ix - (s.nxp - n - 1) : -1);
-  c.plr = (ix >= n - RTM_R && ix < n) ? blr + ix - (n - RTM_R)
-        : ((ix >= s.nxp - n && ix < s.nxp - n + RTM_R) ? blr + RTM_R * s.nzi + ix - (s.nxp - n) : -1);
-  c.tb = (ix >= n && ix < s.nxp - n) ? ix - n : -1;
-  return c;
+  const int n = s.npml, blr = 2 * RTM_R * s.nzi + 2 * RTM_R * s.nxl;
+  if (ix >= n - RTM_R && ix < n) return blr + ix - (n - RTM_R);
+  if (ix >= s.nxp - n && ix < s.nxp - n + RTM_R) return blr + RTM_R * s.nzi + ix - (s.nxp - n);
+  return -1;
 }
 // row part of the vz block offset (rows n-10..n-1 and nzp-n-1..nzp-n+8), -1
 __device__ __forceinline__ int strip_row_vz(const ShotDev& s, int iz)
@@ -132,28 +128,18 @@ __device__ __forceinline__ int strip_row_ptb(const ShotDev& s, int iz)
   if (iz >= r0 && iz < r0 + RTM_R) return b + RTM_R * s.nxl + (iz - r0) * s.nxl;
   return -1;
 }
-__device__ __forceinline__ int soff_vz(int row, const StripCols& c) { return (row >= 0 && c.tb >= 0) ? row + c.tb : -1; }
-__device__ __forceinline__ int soff_vx(int lr, const StripCols& c) { return (lr >= 0 && c.vx >= 0) ? lr + c.vx : -1; }
-__device__ __forceinline__ int soff_p(int lr, int tb, const StripCols& c)
-{
-  return (lr >= 0 && c.plr >= 0) ? lr + c.plr : ((tb >= 0 && c.tb >= 0) ? tb + c.tb : -1);
-}
-
-// A stored strip value is fetched with the first loads of a pass (raw: the
-// fp32 value, or the 16-bit code in the low bits) and decoded where it is
-// used, with the four block scales of its step from a small LDS table: the
-// compute phases then wait for no store reads.
+// A stored strip value is fetched with the other operands of its phase (raw:
+// the fp32 value, or the 16-bit code in the low bits) and decoded where it is
+// used, with the scale of its block (0 vx, 1 vz, 2 p-lr, 3 p-tb) and step.
 __device__ __forceinline__ float store_raw(const ShotDev& s, int it, int off)
 {
   const long long k = (long long)it * s.strip_len + off;
   if (s.store_fmt == ST_F32) return GCF(s.store)[k];
   return __uint_as_float((unsigned int)((const gushort*)s.store)[k]);
 }
-// blk: the strip block of the value (0 vx, 1 vz, 2 p-lr, 3 p-tb)
-__device__ __forceinline__ float store_decode(const ShotDev& s, int blk, float raw, const float* sc4)
+__device__ __forceinline__ float store_value(const ShotDev& s, float sc, float raw)
 {
   if (s.store_fmt == ST_F32) return raw;
-  const float sc = sc4[blk];
   const unsigned int h = __float_as_uint(raw);
   if (s.store_fmt == ST_F16) return __half2float(__ushort_as_half((unsigned short)h)) * sc;
   return __uint_as_float(h << 16) * sc;
@@ -166,22 +152,20 @@ struct Geo {
   static constexpr int G = G_, RPT = RPT_;
   static constexpr int TZ = G * RPT;                   // tile rows
   static constexpr int NT = 64 * G;                    // threads
-  static constexpr int PW = 128;                       // p row: columns x0-20 .. x0+83 (pitch a
-                                                       // multiple of 64 for stride-64 paired reads)
-  static constexpr int VXW = 84;                       // vx row: columns x0-10 .. x0+73
+  static constexpr int PW = 108;                       // p row: column x at float x - x0 + 21 (x0-20..x0+83 held):
+                                                       // a quad's window x-9..x+14 starts on 16 bytes
+  static constexpr int VXW = 88;                       // vx row: columns x0-12 .. x0+75
   static constexpr int ZR = TZ + 19;                   // vz rows z0-10 .. z0+TZ+8
-  static constexpr int KZ = (ZR + G - 1) / G;          // vz rows per thread (consecutive)
+  static constexpr int KZ = (ZR + G - 1) / G;          // vz rows per wave (consecutive)
   static constexpr int PZR = G * KZ + 19;              // p rows held (>= TZ + 38; the last
-                                                       // thread's window may run past TZ+38)
-  static constexpr int KP = (TZ + 38 + G - 1) / G;     // p rows staged per thread
-  static constexpr int KH = (20 * TZ + NT - 1) / NT;   // halo vx cells per thread
-  static_assert((20 * TZ) % 64 == 0, "halo cells fill whole waves");
-  static constexpr int LDS_A = PZR * PW;               // p rows z0-19.. (x halo on the tile rows)
-  static constexpr int LDS_B = TZ * VXW + ZR * 64 + TZ * 64;   // VXL | VZL | SXL
+                                                       // wave's window may run past TZ+38)
+  static constexpr int KQ = (RPT * 22 + 63) / 64;      // vx quads per lane (16 own and 6 halo quads a row)
+  static constexpr int KO = (RPT * 16 + 63) / 64;      // own quads per lane
+  static constexpr int LDS_A = PZR * PW;               // p rows z0-19..
+  static constexpr int LDS_B = 4 + TZ * VXW + ZR * 64; // new vx | new vz
   static constexpr int LDS = LDS_A > LDS_B ? LDS_A : LDS_B;
-  // damping factors of the tile (after LDS; written once per pass): a, b at
-  // the vz rows, at the vx columns x0-10..x0+73, and at the own rows
-  static constexpr int LDS_D = 2 * ZR + 2 * VXW + 2 * TZ;
+  static constexpr int LDS_D = 2 * VXW;                // vx damping of the tile's columns (after LDS)
+  static_assert(RPT == 2 || RPT % 4 == 0, "own quads fill whole waves, or half of one");
 };
 
 // ------------------------------------------------------- buffer access --
@@ -243,18 +227,14 @@ __device__ __forceinline__ void bst(rsrc_t r, float v, int voff, int soff)
 {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, voff, soff, 2);
 }
-// An LDS pointer the compiler must materialise as one register: the taps of
-// a stencil then use the small immediate offsets of that base instead of a
-// separate address add per access (large constant row offsets do not fit
-// the 8-bit offsets of the paired LDS reads)
-typedef __attribute__((address_space(3))) const float lds_cfloat_t;
-__device__ __forceinline__ const float* lds_base(const float* p)
+__device__ __forceinline__ f4 bld4(rsrc_t r, int voff, int soff)
 {
-  unsigned a = (unsigned)(uintptr_t)(lds_cfloat_t*)p;
-  asm volatile("" : "+v"(a));
-  return (const float*)(lds_cfloat_t*)(uintptr_t)a;
+  return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
-
+__device__ __forceinline__ void bst4(rsrc_t r, f4 v, int voff, int soff)
+{
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, 2);
+}
 // load one dword per lane into LDS: lane i writes lds_row[i] (lds_row is
 // wave-uniform)
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -268,567 +248,623 @@ __device__ __forceinline__ void bld_lds(rsrc_t r, float* lds_row, int voff, int 
 // cells) cost their instructions only in the waves that hold them
 __device__ __forceinline__ bool any_lane(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
 
-// radius-r staggered difference a[i] - b[i] with the coefficient row of
-// order 2r; the fma chain runs i = 1..r as the reference loops
-// (kernel.cu:459-460).  cf is the coefficient table in LDS with each row
-// zero beyond its order, so a reduced-radius lane runs the same ten steps
-// with its own row and no predicate: the extra steps add 0*(a-b) = +-0,
-// which leaves the sum unchanged (the operands past the radius are finite
-// cells of the staged halo or the zero margins).  Row r-1 = 9 is c10, so
-// lanes at full radius give the same sums in either branch.  The reduced
-// branch writes the difference as -(b - a), the same value: were it the
-// same expression as the full branch's, the compiler would hoist the ten
-// differences above the branch and hold them in registers across it.
-#define STENCIL_SUM(acc, r, c10, cf, A, B)                                                        \
-  do {                                                                                            \
-    if (!any_lane((r) != RTM_R)) {                                                                \
-      _Pragma("unroll") for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c10[i - 1], (A) - (B), acc); \
-    } else {                                                                                      \
-      const float* cr_ = lds_base((cf) + ((r) - 1) * RTM_R); /* read per use, not hoisted */      \
-      _Pragma("unroll") for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(cr_[i - 1], -((B) - (A)), acc); \
-    }                                                                                             \
-  } while (0)
+// keeps the instructions of one part of a step from being moved into another:
+// left free, the scheduler fetches the operands of every part first and needs
+// 256 registers for them
+__device__ __forceinline__ void part() { __builtin_amdgcn_sched_barrier(0); }
 
-// entry t of the coefficient table as the kernels hold it: row t/10 (order
-// 2(t/10+1)) zero beyond its t/10+1 coefficients
+// the value is computed here: a result that is first used in a later part
+// would otherwise be computed there, and its whole window held until then
+__device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
+
+// sum of the staggered differences w[h + i] - w[h + 1 - i], i = 1..10, as the
+// reference loops (kernel.cu:459-460), one fused multiply-add a tap
+template <class W, class Cf>
+__device__ __forceinline__ float taps(const W& w, int h, const Cf& c)
+{
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c[i - 1], w[h + i] - w[h + 1 - i], acc);
+  return acc;
+}
+// The same with the coefficient row of order 2 r from the LDS table (rows of
+// CTW floats, zero beyond their order): a reduced-radius cell runs the same
+// ten steps with its own row and no predicate, the extra steps add
+// 0*(a-b) = +-0, which leaves the sum unchanged (the operands past the radius
+// are finite cells of the staged halo or the zero margins), and row 9 gives
+// the radius-10 sum bit for bit.
+constexpr int CTW = 12;
+template <class W>
+__device__ __forceinline__ float taps_r(const W& w, int h, const float* ctab, int r)
+{
+  const f4* cr = (const f4*)(ctab + (r - 1) * CTW);
+  const f4 a = cr[0], b = cr[1], d = cr[2];
+  const float c[RTM_R] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, d.x, d.y};
+  // (the difference as -(b - a), the same value: the compiler would hoist the
+  // differences it shares with the full-radius branch and hold them)
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c[i - 1], -(w[h + 1 - i] - w[h + i]), acc);
+  return acc;
+}
+// entry t of that table
 __device__ __forceinline__ float ctab_entry(const ShotDev& s, int t)
 {
-  return (t % RTM_R) <= (t / RTM_R) ? GCF(s.coef)[t] : 0.0f;
+  const int r = t / CTW, i = t - r * CTW;
+  return i <= r && i < RTM_R ? GCF(s.coef)[r * RTM_R + i] : 0.0f;
 }
 
 // field kinds of one pass
 enum : int { FK_SRC = 0, FK_RCV = 1, FK_RCN = 2 };
-
-// New velocity of one cell from the p window Pr (Pr[i] = p at +i along the
-// derivative), old value vo and reciprocal density ib.  Forward-type fields
-// (source in the forward phase, receiver in the reverse phase):
-//   v = (c1*v - u)/c2, u = (sum c_i (p[+i] - p[-i+1]) * dt/h) / rho
-//   (kernel.cu:588-594), evaluated as u = (s*dt/h)*ib, v = fma(a, v, -(u*b))
-//   with a = c1/c2, b = 1/c2; off the absorbing layer (a = b = 1) that is
-//   v - u (kernel.cu:462); radius min(10, distance to the grid edge)
-//   (cuda_norderx/z, kernel.cu:299-317).  VALID false: the velocity does
-//   not exist there (its value is never read); the damping arrays carry 1
-//   outside the grid.
-// Reconstruction: strip cells restored from the store of step it+1
-// (kernel.cu:1294-1347; VO then holds the raw stored value), interior cells
-// v + u as fma(s*dt/h, ib, v) (kernel.cu:318-388).
-#define VEL_CELL(FK, gen, strips, SOFF, VALID, RAD, INTERIOR, P_AT, VO, IB, DTH, AV, BV, OUT)               \
-  do {                                                                                                     \
-    float v_ = 0.0f;                                                                                       \
-    if (FK == FK_RCN) {                                                                                    \
-      /* computed for every cell and then selected (no divergent branch): */                               \
-      /* cells off the interior stay 0, strip cells take the stored value */                               \
-      float acc = 0.0f;                                                                                    \
-      _Pragma("unroll") for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c10[i - 1], P_AT(i) - P_AT(1 - i), acc); \
-      v_ = __builtin_fmaf(acc * (DTH), (IB), (VO));                                                        \
-      if ((gen) && !(INTERIOR)) v_ = 0.0f;                                                                 \
-      if (strips) {                                                                                        \
-        const int sb_ = (SOFF);  /* strip block of a strip cell, -1 elsewhere */                            \
-        if (sb_ >= 0) v_ = store_decode(s, sb_, (VO), DMP);                                                \
-      }                                                                                                    \
-    } else if (!(gen)) {                                                                                   \
-      float acc = 0.0f;                                                                                    \
-      _Pragma("unroll") for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c10[i - 1], P_AT(i) - P_AT(1 - i), acc); \
-      v_ = (VO) - (acc * (DTH)) * (IB);                                                                    \
-    } else {                                                                                               \
-      const int rr_ = (VALID) ? (RAD) : RTM_R;                                                             \
-      float acc = 0.0f;                                                                                    \
-      STENCIL_SUM(acc, rr_, c10, ctab, P_AT(i), P_AT(1 - i));                                              \
-      const float u_ = (acc * (DTH)) * (IB);                                                               \
-      /* one form for every cell of the tile: a = b = 1 (undamped) gives */                                \
-      /* fma(1, v, -u) == v - u exactly, cheaper than a branch per cell */                                 \
-      v_ = __builtin_fmaf((AV), (VO), -(u_ * (BV)));                                                       \
-    }                                                                                                      \
-    OUT = v_;                                                                                              \
-  } while (0)
-
-// ------------------------------------------------------------ pressure --
-struct DivV { float sx, sz; };
-
-// Staggered difference of vz along z (kernel.cu:520-534) of thread-local row
-// r from the column window cz of vz rows; the x half (sx) comes from the row
-// segments of the pressure phase
-template <int NW>
-__device__ __forceinline__ float div_z(const float (&cz)[NW], int r, int rad, const float* c10,
-                                       const float* __restrict__ cf)
-{
-  float sz = 0.0f;
-  if (rad == RTM_R) {
-#pragma unroll
-    for (int i = 1; i <= RTM_R; i++) sz = __builtin_fmaf(c10[i - 1], cz[r + 9 + i] - cz[r + 10 - i], sz);
-  } else {
-    const float* c = lds_base(cf + (rad - 1) * RTM_R);
-#pragma unroll
-    for (int i = 1; i <= RTM_R; i++) sz = __builtin_fmaf(c[i - 1], cz[r + 9 + i] - cz[r + 10 - i], sz);
-  }
-  return sz;
-}
-
-// p - rho v^2 (sx dt/dx + sz dt/dz) (kernel.cu:536-539), kk = rho v^2
-__device__ __forceinline__ float pres_sum(const DivV& d, float dtx, float dtz)
-{
-  return __builtin_fmaf(d.sx, dtx, d.sz * dtz);
-}
+// tile classes: interior (no damping, no strips), general (absorbing layer or
+// strips), edge (general with cells of reduced radius)
+enum : int { TC_IN = 0, TC_GEN = 1, TC_EDGE = 2 };
 
 // One field through one time step on a tile: p of the current level pc (with
-// velocities vxc, vzc) to the next level (pn, vxn, vzn).  On return pnew
-// holds the new pressure of the thread's own cells (rows g*RPT+r); ps is the
-// reconstructed source pressure of the same cells (receiver pass imaging).
+// velocities vxc, vzc) to the next level (pn, vxn, vzn).  A reconstruction
+// pass with `img` also adds the imaging products of the PREVIOUS reverse step,
+// of the pressure levels both fields read (pr: the receiver field's), so that
+// the two fields of a reverse step need not wait for each other.
 //
-// Thread roles (lane lx, wave g):
-//   p staging  rows g+G*m of the tile columns (PZ) and their x wings (PC)
-//   vz         rows z0-10 + g*KZ + k of column x0+lx (z window from PZ)
-//   vx         own rows z0 + g*RPT + r of column x0+lx, and the halo
-//              columns x0-10..x0-1, x0+64..x0+73 dealt over all threads
-//   p          own rows z0 + g*RPT + r of column x0+lx
-template <class Q, int FK>
-__device__ __forceinline__ void field_step(float* __restrict__ lds, const ShotDev& s, const Tile& tl, int it,
-                                           const float* pc, const float* vxc, const float* vzc, float* pn, float* vxn,
-                                           float* vzn, const float* __restrict__ ctab, const float (&ps)[Q::RPT],
-                                           float (&pnew)[Q::RPT], unsigned char* actw = nullptr)
+// What bounds it: instruction issue and the chain of a workgroup's phases,
+// then HBM.  So the classes are compiled apart (straight-line code; one body
+// with per-cell tests issued three instructions for each stencil operation),
+// and everything but the z-differences is mapped to quads of four columns:
+//   p staging   rows g + G m of the tile (LDS-writing loads, no registers)
+//   z-derivatives (columns): lane = column, a wave takes consecutive rows and
+//               reads their window of rows once; row offsets, the damping of a
+//               row and its radius are wave-uniform (scalar registers)
+//   x-derivatives (quads): a wave's own RPT rows as 16 quads of a row and the
+//               6 quads of its halo columns x0-12.., x0+64..; a quad reads its
+//               window of 24 values as six 16-byte LDS loads instead of 20
+//               loads per cell, and its operands and results move as 16-byte
+//               accesses (a quarter of the memory instructions)
+// The rows of the new vx are written and read by the same wave, so only the
+// new vz crosses waves (one exchange), and the z-differences reach the quads
+// through the wave's own vx rows once those are consumed.
+template <class Q, int FK, int TC>
+__device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* __restrict__ ctab, const ShotDev& s,
+                                          const Tile& tl, int it, const float* pc, const float* vxc, const float* vzc,
+                                          float* pn, float* vxn, float* vzn, const float* pr, bool img,
+                                          unsigned char* actw)
 {
-  constexpr int G = Q::G, RPT = Q::RPT, TZ = Q::TZ, NT = Q::NT, KZ = Q::KZ, KP = Q::KP, KH = Q::KH;
+  constexpr int G = Q::G, RPT = Q::RPT, TZ = Q::TZ, KZ = Q::KZ, PW = Q::PW, VXW = Q::VXW, ZR = Q::ZR;
+  constexpr int KQ = Q::KQ, KO = Q::KO;
+  constexpr bool RCN = FK == FK_RCN, GEN = TC != TC_IN, EDGE = TC == TC_EDGE;
   // the OR of the bit patterns of the lane's stored field values (-0 counts
   // as non-zero): written to actw[wave] at the end for the zero-tile skip
   unsigned int nzb = 0u;
-  constexpr int PW = Q::PW, VXW = Q::VXW, ZR = Q::ZR;
-  float* PS = lds;                                     // p rows z0-19.., columns x0-20..x0+83
-  float* DMP = lds + Q::LDS;                           // damping table (damped passes of gen tiles)
-  constexpr int DZA = 0, DZB = ZR, DXA = 2 * ZR, DXB = 2 * ZR + VXW, DPA = 2 * ZR + 2 * VXW, DPB = DPA + TZ;
-  float* VXL = lds;                                    // after the second barrier
-  float* VZL = lds + TZ * VXW;
-  const int tid = threadIdx.x, lx = tid & 63;
-  const int g = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float* PS = lds;                                     // p rows z0-19.., columns x0-20..x0+83 from float 1 of a row
+  float* DMP = lds + Q::LDS;                           // a, b of vx at columns x0-12.. (88 each)
+  float* VXL = lds + 4;                                // (after the pressure is consumed) column x at x - x0 + 10
+  float* VZL = lds + 4 + TZ * VXW;                     // new vz rows z0-10.., 64 columns
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x0 = tl.x0, z0 = tl.z0, nxp = s.nxp, nzp = s.nzp, npml = s.npml;
-  // halo vx cell k*NT + tid exists for the whole wave or none of it (20*TZ
-  // is a multiple of 64): a wave-uniform test
-  auto halo_on = [&](int k) { return k * NT + g * 64 < 20 * TZ; };
-  const int ix = x0 + lx;
-  const bool gen = (tl.kind & TF_GEN) != 0;
-  // strip cells that the reconstruction restores (the tile's and its halo's);
-  // the forward pass saves its strips in k_save after the step
-  const bool strips = FK == FK_RCN && (tl.kind & TF_STRIP) != 0;
+  const int ix = x0 + lane;                            // the lane's column (column mapping)
+  const int zw = z0 + g * RPT;                         // the wave's first own row
+  const bool strips = RCN && GEN && (tl.kind & TF_STRIP) != 0;
   const int pr4 = s.pitch * 4;
-  const int srow0 = (z0 + RTM_MZT) * pr4;             // byte offset of tile row 0
-  const int vcol = (ix + RTM_MXL) * 4;                // byte offset of the lane's column
-  const int vld = col_load(vcol, ix, nxp);             // ... for loads
-  const int icol = (ix - npml) * 4;                    // ... in the imaging accumulators
+  const int srow0 = (z0 + RTM_MZT) * pr4;              // byte offset of tile row 0
+  const int vcol = (ix + RTM_MXL) * 4;                 // byte offset of the lane's column
+  const int vld = GEN ? col_load(vcol, ix, nxp) : vcol;
   const rsrc_t Rp = field_rsrc(pc, s), Rvx = field_rsrc(vxc, s), Rvz = field_rsrc(vzc, s);
-  const rsrc_t Rib = model_rsrc(s.mib, s);
-  const int mcol = model_col(s, ix);                   // the lane's model column
+  const rsrc_t Rib = model_rsrc(s.mib, s), Rkk = model_rsrc(s.mkk, s);
+  const float dtx = s.dtx, dtz = s.dtz;
+  auto inner_row = [&](int z) { return z >= npml && z < nzp - npml; };
+  auto inner_col = [&](int x) { return x >= npml && x < nxp - npml; };
   float c10[RTM_R];
 #pragma unroll
-  for (int i = 0; i < RTM_R; i++) c10[i] = GCF(s.coef)[90 + i];
-  const float dtx = s.dtx, dtz = s.dtz;
+  for (int i = 0; i < RTM_R; i++) c10[i] = CCF(s.coef)[90 + i];
 
-  // ---- 1. loads: p with its halo straight into LDS (buffer loads with the
-  //         lds modifier: lane i of a wave writes its dword to base + 4 i),
-  //         old velocities and density of every velocity cell into registers
+  // ---- 1. the pressure and its halo into LDS (buffer loads with the lds
+  //         modifier: lane i of a wave writes its dword to base + 4 i): tile
+  //         rows as two full-wave loads (x0-20..x0+43, x0+20..x0+83; the
+  //         middle 24 columns arrive twice with the same values), halo rows
+  //         the tile's columns; old vz and its 1/rho into registers
   {
-    // tile rows: columns x0-20..x0+83 as two full-wave loads (x0-20..x0+43
-    // and x0+20..x0+83; the middle 24 columns arrive twice with the same
-    // values), so that no load is issued by part of a wave; halo rows:
-    // columns x0..x0+63
-    const int ca = col_load((x0 - 20 + lx + RTM_MXL) * 4, x0 - 20 + lx, nxp);
-    const int cb = col_load((x0 + 20 + lx + RTM_MXL) * 4, x0 + 20 + lx, nxp);
+    int ca = (x0 - 20 + lane + RTM_MXL) * 4, cb = (x0 + 20 + lane + RTM_MXL) * 4;
+    if (GEN) {
+      ca = col_load(ca, x0 - 20 + lane, nxp);
+      cb = col_load(cb, x0 + 20 + lane, nxp);
+    }
+    const int sw = srow0 + g * RPT * pr4;
 #pragma unroll
-    for (int m = 0; m < KP; m++) {
-      const int k = g + G * m;
-      if (k < TZ + 38) {
-        const int so = srow0 + (k - 19) * pr4;
-        if (k >= 19 && k < 19 + TZ) {
-          bld_lds(Rp, PS + k * PW, ca, so);
-          bld_lds(Rp, PS + k * PW + 40, cb, so);
-        } else {
-          bld_lds(Rp, PS + k * PW + 20, vld, so);
-        }
+    for (int m = 0; m < RPT; m++) {
+      bld_lds(Rp, PS + (g * RPT + m + 19) * PW + 1, ca, sw + m * pr4);
+      bld_lds(Rp, PS + (g * RPT + m + 19) * PW + 41, cb, sw + m * pr4);
+    }
+#pragma unroll
+    for (int m = 0; m < (38 + G - 1) / G; m++) {       // 19 rows above the tile, 19 below
+      const int h = g + G * m;
+      if (G * (m + 1) <= 38 || h < 38) {
+        const int k = h < 19 ? h : h + TZ;
+        bld_lds(Rp, PS + k * PW + 21, vld, srow0 + (k - 19) * pr4);
       }
     }
   }
+  // rows of the z phase that exist for every wave need no test
+  auto zrow = [&](int k) { return k < ZR - (G - 1) * KZ || g * KZ + k < ZR; };
+  const int mcol = model_col(s, ix);
+  const bool zcol = ix >= npml && ix < nxp - npml;     // interior columns
   float vzo[KZ], ibz[KZ];
 #pragma unroll
   for (int k = 0; k < KZ; k++) {
-    const int kz = g * KZ + k;
+    const int kz = g * KZ + k, iz = z0 - 10 + kz;
     vzo[k] = 0.0f;
     ibz[k] = 1.0f;
-    if (kz < ZR) {
-      const int so = srow0 + (kz - 10) * pr4;
-      vzo[k] = bld(Rvz, vld, so);
-      ibz[k] = bld(Rib, mcol, model_row(s, z0 - 10 + kz));
+    if (zrow(k)) {
+      // a strip row of the reconstruction: the stored value of step it+1 (raw)
+      const int st = strips ? strip_row_vz(s, iz) : -1;
+      if (st >= 0) {
+        if (zcol) vzo[k] = store_raw(s, it + 1, st + ix - npml);
+      } else {
+        vzo[k] = bld(Rvz, vld, srow0 + (kz - 10) * pr4);
+      }
+      ibz[k] = bld(Rib, mcol, GEN ? model_row(s, iz) : (iz - s.mz0) * s.mpitch * 4);
     }
   }
-  // reconstruction of a strip tile: the stored value of a strip cell
-  // replaces its old velocity, fetched now with the rest (after the old
-  // value's load, which it overwrites) and decoded where it is used; which
-  // cells are strip cells is kept as bits of sm (vz rows, vx rows, halo vx,
-  // p rows, p rows in the top/bottom block), so the offsets are computed once
-  StripCols sc{-1, -1, -1};
-  if (strips) sc = strip_cols(s, ix);
-  const bool rstrips = FK == FK_RCN && strips;
-  constexpr int SMX = KZ, SMH = KZ + RPT, SMP = KZ + RPT + KH, SMT = KZ + RPT + KH + RPT;
-  static_assert(SMT + RPT <= 64, "strip bits");
-  unsigned long long sm = 0;
-  if (rstrips) {
-#pragma unroll
-    for (int k = 0; k < KZ; k++) {
-      const int kz = g * KZ + k;
-      const int st = kz < ZR ? soff_vz(strip_row_vz(s, z0 - 10 + kz), sc) : -1;
-      if (st >= 0) { vzo[k] = store_raw(s, it + 1, st); sm |= 1ull << k; }
+  // quads of the x phase.  Own quads: lane n of quad round k has row
+  // n / 16 + 4 k, columns 4 (n % 16), so that the rounds differ by a scalar
+  // row offset.  The last round holds the halo quads, 6 a row (two rows a
+  // wave: in the lanes past the 32 own quads)
+  const bool oq = RPT >= 4 || lane < 32;               // the lane has own quads
+  const int hn = RPT >= 4 ? lane : lane - 32;          // its halo quad
+  const bool hon = hn >= 0 && hn < RPT * 6;
+  const int hr = hn / 6, hq = hn - hr * 6;
+  const int hcol = hq < 3 ? -12 + 4 * hq : 52 + 4 * hq;
+  const int orow = RPT >= 4 ? lane >> 4 : (oq ? lane >> 4 : (hon ? hr : 0));
+  const int ocol = RPT >= 4 ? 4 * (lane & 15) : (oq ? 4 * (lane & 15) : (hon ? hcol : 0));
+  const int xrow = hon ? hr : 0, xcol = hon ? hcol : 0;   // the halo round's (RPT >= 4)
+  const int ooff = ((zw + orow + RTM_MZT) * s.pitch + x0 + ocol + RTM_MXL) * 4;
+  const int xoff = ((zw + xrow + RTM_MZT) * s.pitch + x0 + xcol + RTM_MXL) * 4;
+  auto qrow = [&](int k) { return k < KO ? orow + 4 * k : xrow; };
+  auto qcol = [&](int k) { return k < KO ? ocol : xcol; };
+  auto qx = [&](int k) { return x0 + qcol(k); };       // first column of a quad
+  auto qsoff = [&](int k) { return k < KO ? 4 * k * pr4 : 0; };
+  // load offset of a quad: quads off the grid's columns fetch nothing
+  const int old_ = GEN ? pred_off(ooff, x0 + ocol >= 0 && x0 + ocol < nxp) : ooff;
+  const int xld_ = GEN ? pred_off(xoff, x0 + xcol >= 0 && x0 + xcol < nxp) : xoff;
+  auto qld = [&](int k) { return k < KO ? old_ : xld_; };
+  if (!RCN && GEN) {                                   // vx damping of the columns x0-12..x0+75
+    for (int t = threadIdx.x; t < 22; t += 64 * G) {
+      ((f4*)DMP)[t] = *(const gf4*)(GCF(s.axv) + x0 - 12 + 4 * t);
+      ((f4*)DMP)[22 + t] = *(const gf4*)(GCF(s.bxv) + x0 - 12 + 4 * t);
     }
   }
-  auto sbit = [&](int b) { return ((sm >> b) & 1ull) != 0; };
-  // per-lane column data of the generic path: existence, radius, damping;
-  // the damping of the tile's rows and halo columns goes to an LDS table, so
-  // that the compute phases wait for no small loads
-  bool vxv = true;
-  int rrx = RTM_R;
-  float axv = 1.0f, bxv = 1.0f, ax = 1.0f, bx = 1.0f;
-  if (gen) {
-    vxv = ix <= nxp - 2;
-    rrx = vxv ? imin(RTM_R, imin(ix + 1, nxp - 1 - ix)) : RTM_R;
-  }
-  if (FK != FK_RCN && gen) {
-    axv = GCF(s.axv)[ix];
-    bxv = GCF(s.bxv)[ix];
-    if (ix < nxp) { ax = GCF(s.ax)[ix]; bx = GCF(s.bx)[ix]; }
-    // rows z0-10.. and columns x0-10.. lie within the arrays' margins
-    if (tid < ZR) { DMP[DZA + tid] = GCF(s.azv)[z0 - 10 + tid]; DMP[DZB + tid] = GCF(s.bzv)[z0 - 10 + tid]; }
-    if (tid < VXW) { DMP[DXA + tid] = GCF(s.axv)[x0 - 10 + tid]; DMP[DXB + tid] = GCF(s.bxv)[x0 - 10 + tid]; }
-    if (tid < TZ) { DMP[DPA + tid] = GCF(s.az)[z0 + tid]; DMP[DPB + tid] = GCF(s.bz)[z0 + tid]; }
-  }
-  // 16-bit store: block scales of the steps the reconstruction reads (it+1:
-  // velocities, it: pressure) in the damping table's place (unused there)
-  if (rstrips && s.store_fmt != ST_F32 && tid < 8)
-    DMP[tid] = GCF(s.sscale)[(long long)(tid < 4 ? it + 1 : it) * 4 + (tid & 3)];
   __builtin_amdgcn_s_waitcnt(0);                       // the LDS writes of the staging loads
   __syncthreads();                                     // p staged
-  float vxo[RPT], ibx[RPT];
-#pragma unroll
-  for (int r = 0; r < RPT; r++) {
-    const int so = srow0 + (g * RPT + r) * pr4;
-    vxo[r] = bld(Rvx, vld, so);
-    ibx[r] = bld(Rib, mcol, model_row(s, z0 + g * RPT + r));
-  }
-  float hvo[KH], hib[KH];
-  int hrow[KH], hcol[KH];
-#pragma unroll
-  for (int k = 0; k < KH; k++) {
-    const int h = k * NT + tid;
-    hvo[k] = 0.0f;
-    hib[k] = 1.0f;
-    hrow[k] = h / 20;
-    const int hc = h - hrow[k] * 20;
-    hcol[k] = hc < 10 ? hc : hc + 64;                  // VXL column: x = x0 - 10 + hcol
-    if (halo_on(k)) {
-      const int off = col_load(srow0 + hrow[k] * pr4 + (x0 - 10 + hcol[k] + RTM_MXL) * 4, x0 - 10 + hcol[k], nxp);
-      hvo[k] = bld(Rvx, off, 0);
-      hib[k] = bld(Rib, model_col(s, x0 - 10 + hcol[k]) +
-                            imin(imax(z0 + hrow[k] - s.mz0, 0), s.mzn - 1) * s.mpitch * 4, 0);
+
+  // operands of the x phase: they arrive while the z phase computes.  Four
+  // model values of a quad: one 16-byte load where no column is clamped
+  auto model4 = [&](rsrc_t r, int k) -> f4 {
+    if (!GEN) {
+      const int o = ((zw + (k < KO ? orow : xrow) - s.mz0) * s.mpitch + s.mx0 + qx(k) - s.mxs) * 4;
+      return bld4(r, o, k < KO ? 16 * k * s.mpitch : 0);
     }
+    const int ro = model_row(s, zw + qrow(k)), x = qx(k);
+    return f4{bld(r, ro + model_col(s, x), 0), bld(r, ro + model_col(s, x + 1), 0), bld(r, ro + model_col(s, x + 2), 0),
+              bld(r, ro + model_col(s, x + 3), 0)};
+  };
+  f4 vxo[KQ], ibx[KQ];
+#pragma unroll
+  for (int k = 0; k < KQ; k++) {
+    vxo[k] = bld4(Rvx, qld(k), qsoff(k));
+    ibx[k] = model4(Rib, k);
   }
-  if (rstrips) {
+  // reconstruction: block scales of the 16-bit store (1 for fp32: unused)
+  float scv[4] = {1.0f, 1.0f, 1.0f, 1.0f};             // vx, vz of step it+1, p-lr, p-tb of step it
+  if (strips && s.store_fmt != ST_F32) {
 #pragma unroll
-    for (int r = 0; r < RPT; r++) {
-      const int st = soff_vx(strip_row_lr(s, z0 + g * RPT + r), sc);
-      if (st >= 0) { vxo[r] = store_raw(s, it + 1, st); sm |= 1ull << (SMX + r); }
-    }
+    for (int b = 0; b < 4; b++) scv[b] = CCF(s.sscale)[(long long)(b < 2 ? it + 1 : it) * 4 + b];
+  }
+  // vx strip cells of a quad (reconstruction): raw stored values and a mask
+  f4 sxr[KQ];
+  int sxm[KQ];
+  if (strips) {
 #pragma unroll
-    for (int k = 0; k < KH; k++) {
-      const int st = halo_on(k) ? strip_vx(s, z0 + hrow[k], x0 - 10 + hcol[k]) : -1;
-      if (st >= 0) { hvo[k] = store_raw(s, it + 1, st); sm |= 1ull << (SMH + k); }
+    for (int k = 0; k < KQ; k++) {
+      sxm[k] = 0;
+      sxr[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int st = strip_vx(s, zw + qrow(k), qx(k) + c);
+        if (st >= 0) {
+          sxr[k][c] = store_raw(s, it + 1, st);
+          sxm[k] |= 1 << c;
+        }
+      }
     }
   }
 
-  // ---- 2. new velocities
-  float vzn_[KZ], vxn_[RPT], hvn[KH];
+  part();
+  // ---- 2. new vz (rows z0-10 + g KZ + k of the lane's column).  Forward
+  //         fields: v = (c1*v - u)/c2, u = (sum * dt/h) / rho
+  //         (kernel.cu:588-594) as u = (s*dt/h)*ib, v = fma(a, v, -(u*b)) with
+  //         a = c1/c2, b = 1/c2 (off the layer v - u, kernel.cu:462), radius
+  //         min(10, distance to the grid edge) (cuda_norderx/z,
+  //         kernel.cu:299-317); off the grid b = 0, so the value stays +0.
+  //         Reconstruction: v + u as fma(s*dt/h, ib, v) (kernel.cu:318-388),
+  //         stored strip values (kernel.cu:1294-1347), 0 elsewhere
+  float vzn_[KZ];
   {
-    const rsrc_t Rvzn = field_rsrc(vzn, s);
-    float cw[KZ + 19];                                 // p rows z0-19+g*KZ+m of the column
+    float cw[KZ + 19];                                 // p rows z0-19 + g KZ + m of the column
 #pragma unroll
-    for (int m = 0; m < KZ + 19; m++) cw[m] = PS[(g * KZ + m) * PW + 20 + lx];
+    for (int m = 0; m < KZ + 19; m++) cw[m] = PS[(g * KZ + m) * PW + 21 + lane];
 #pragma unroll
     for (int k = 0; k < KZ; k++) {
-      const int kz = g * KZ + k;
-      const int iz = z0 - 10 + kz;                     // wave-uniform
-#define PZA(i) cw[k + 9 + (i)]
-      VEL_CELL(FK, gen, strips, (sbit(k) ? 1 : -1), (iz >= 0 && iz <= nzp - 2), imin(RTM_R, imin(iz + 1, nzp - 1 - iz)),
-               (ix >= npml && ix < nxp - npml && iz >= npml && iz <= nzp - npml - 2), PZA, vzo[k], ibz[k], dtz,
-               DMP[DZA + kz], DMP[DZB + kz], vzn_[k]);
-#undef PZA
-      if (kz >= 10 && kz < 10 + TZ) {                  // own rows (wave-uniform)
-        if (!gen) bst(Rvzn, vzn_[k], vcol, srow0 + (kz - 10) * pr4);   // every lane's cell exists
-        else bst(Rvzn, vzn_[k], pred_off(vcol, ix < nxp && iz <= nzp - 2), srow0 + (kz - 10) * pr4);
-        nzb |= __float_as_uint(vzn_[k]);
+      if (k % 3 == 0) part();
+      vzn_[k] = 0.0f;
+      if (zrow(k)) {
+        const int kz = g * KZ + k, iz = z0 - 10 + kz;  // wave-uniform
+        if (RCN) {
+          if (!GEN) {
+            vzn_[k] = __builtin_fmaf(taps(cw, k + 9, c10) * dtz, ibz[k], vzo[k]);
+          } else if (strips && strip_row_vz(s, iz) >= 0) {
+            vzn_[k] = zcol ? store_value(s, scv[1], vzo[k]) : 0.0f;
+          } else if (iz >= npml && iz <= nzp - npml - 2) {
+            const float v = __builtin_fmaf(taps(cw, k + 9, c10) * dtz, ibz[k], vzo[k]);
+            vzn_[k] = zcol ? v : 0.0f;
+          }
+        } else {
+          float sum;
+          if (EDGE) {
+            const int rad = iz >= 0 && iz <= nzp - 2 ? imin(RTM_R, imin(iz + 1, nzp - 1 - iz)) : RTM_R;
+            sum = rad == RTM_R ? taps(cw, k + 9, c10) : taps_r(cw, k + 9, ctab, rad);
+          } else {
+            sum = taps(cw, k + 9, c10);
+          }
+          const float u = (sum * dtz) * ibz[k];
+          vzn_[k] = GEN ? __builtin_fmaf(CCF(s.azv)[iz], vzo[k], -(u * CCF(s.bzv)[iz])) : vzo[k] - u;
+        }
       }
+      pin(vzn_[k]);
     }
   }
 
-  // operands of the pressure phase, fetched now so that one memory round trip
-  // for all rows overlaps the vx computation (inside the row loop each row
-  // would wait for its own): rho v^2 of the own cells, and per cell either
-  // the PML split pair (forward-type passes, damped cells) or the imaging
-  // accumulators (receiver pass, interior cells) -- never both
-  const bool xin = ix >= npml && ix < nxp - npml;
-  const bool xring = ix == 0 || ix == nxp - 1;
-  float kk[RPT], qa[RPT], qb[RPT];
-  {
-    const rsrc_t Rkk = model_rsrc(s.mkk, s);
-    const rsrc_t R1 = field_rsrc(s.q1, s), R2 = field_rsrc(s.q2, s);
+  // ---- 3. new vx of the own and the halo quads; the quad's own pressure is
+  //         in its window
+  f4 hv[KQ], po[KO];
 #pragma unroll
-    for (int r = 0; r < RPT; r++) {
-      const int j = g * RPT + r, iz = z0 + j;
-      const int so = srow0 + j * pr4;
-      kk[r] = bld(Rkk, mcol, model_row(s, iz));
-      qa[r] = qb[r] = 0.0f;
-      const bool incell = ix < nxp && iz < nzp;
-      const bool inner = xin && iz >= npml && iz < nzp - npml;
-      const int io = imax(iz - npml, 0) * s.nxl * 4;   // wave-uniform row offset (rows >= npml used)
-      if (FK == FK_RCV && !gen) {                      // every lane's cell is interior
-        qa[r] = bld(image_rsrc(s.g1, s), icol, io);
-        qb[r] = bld(image_rsrc(s.illum, s), icol, io);
-      } else if (FK != FK_RCN && gen) {
-        // the split pair of damped cells, the accumulators of interior cells:
-        // loads with predicated offsets (0 where a lane takes no part), each
-        // pair issued only by waves that hold such a cell
-        const bool dm = incell && iz > 0 && iz < nzp - 1 && !xring && !inner;
-        if (any_lane(dm)) {
-          const int pq = pred_off(vcol, dm);
-          qa[r] = bld(R1, pq, so);
-          qb[r] = bld(R2, pq, so);
+  for (int k = 0; k < KQ; k++) {
+    part();
+    float w[24];                                       // p at columns x-9 .. x+14
+    const f4* row = (const f4*)(PS + (g * RPT + qrow(k) + 19) * PW + qcol(k) + 12);
+#pragma unroll
+    for (int m = 0; m < 6; m++) {
+      const f4 v = row[m];
+      w[4 * m] = v.x; w[4 * m + 1] = v.y; w[4 * m + 2] = v.z; w[4 * m + 3] = v.w;
+    }
+    if (k < KO) po[k < KO ? k : 0] = f4{w[9], w[10], w[11], w[12]};
+    f4 av, bv;
+    if (!RCN && GEN) {
+      av = *(const f4*)(DMP + qcol(k) + 12);
+      bv = *(const f4*)(DMP + VXW + qcol(k) + 12);
+    }
+    int rad[4] = {RTM_R, RTM_R, RTM_R, RTM_R};
+    bool red = false;
+    if (EDGE && !RCN) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int x = qx(k) + c;
+        if (x >= 0 && x <= nxp - 2) rad[c] = imin(RTM_R, imin(x + 1, nxp - 1 - x));
+        red = red || rad[c] != RTM_R;
+      }
+      red = any_lane(red);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      float sum;
+      if (EDGE && !RCN && red) sum = taps_r(w, 9 + c, ctab, rad[c]);
+      else sum = taps(w, 9 + c, c10);
+      if (RCN) {
+        float v = __builtin_fmaf(sum * dtx, ibx[k][c], vxo[k][c]);
+        if (GEN) {
+          const int x = qx(k) + c;
+          v = inner_row(zw + qrow(k)) && x >= npml && x <= nxp - npml - 2 ? v : 0.0f;
+          if (strips) v = (sxm[k] >> c) & 1 ? store_value(s, scv[0], sxr[k][c]) : v;
         }
-        if (FK == FK_RCV) {
-          const bool im = incell && inner;
-          if (any_lane(im)) {
-            const int pi = pred_off(icol, im);
-            const float a2 = bld(image_rsrc(s.g1, s), pi, io), b2 = bld(image_rsrc(s.illum, s), pi, io);
-            qa[r] = im ? a2 : qa[r];
-            qb[r] = im ? b2 : qb[r];
+        hv[k][c] = v;
+      } else {
+        const float u = (sum * dtx) * ibx[k][c];
+        hv[k][c] = GEN ? __builtin_fmaf(av[c], vxo[k][c], -(u * bv[c])) : vxo[k][c] - u;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      float v = hv[k][c];
+      pin(v);
+      hv[k][c] = v;
+    }
+    if (k < KO) {                                      // own quads to memory
+      const bool on = oq && (!GEN || (qx(k) < nxp && zw + qrow(k) < nzp));
+      bst4(field_rsrc(vxn, s), hv[k], pred_off(ooff, on), qsoff(k));
+      if (oq)
+#pragma unroll
+        for (int c = 0; c < 4; c++) nzb |= __float_as_uint(hv[k][c]);
+    }
+  }
+  part();
+  // operands of the pressure phase, fetched now so that the round trip
+  // overlaps the exchange and the differences below: rho v^2 of the own quads, and the PML split pair
+  // (forward-type passes, quads with a damped cell) or, in the
+  // reconstruction, the imaging accumulators and the receiver pressure
+  f4 kk[KO], qa[KO], qb[KO], qc[KO];
+  int qsp[KO];                                         // split cells of a quad / strip cells (bits 0-3 lr, 4-7 tb)
+#pragma unroll
+  for (int h = 0; h < KO; h++) {
+    const int z = zw + qrow(h), x = qx(h);
+    kk[h] = model4(Rkk, h);
+    qsp[h] = 0;
+    qa[h] = qb[h] = qc[h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (!RCN && GEN) {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const bool on = z > 0 && z < nzp - 1 && x + c > 0 && x + c < nxp - 1 && !(inner_row(z) && inner_col(x + c));
+        qsp[h] |= on ? 1 << c : 0;
+      }
+      if (any_lane(qsp[h] != 0 && oq)) {
+        const int o = pred_off(ooff, qsp[h] != 0 && oq);
+        qa[h] = bld4(field_rsrc(s.q1, s), o, qsoff(h));
+        qb[h] = bld4(field_rsrc(s.q2, s), o, qsoff(h));
+      }
+    }
+    if (RCN) {
+      if (img) {
+        qc[h] = bld4(field_rsrc(pr, s), old_, qsoff(h));
+        const int o = ((z - npml) * s.nxl + x - npml) * 4;
+        if (!GEN) {
+          qa[h] = bld4(image_rsrc(s.g1, s), o, 0);
+          qb[h] = bld4(image_rsrc(s.illum, s), o, 0);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const int oc = pred_off(o + 4 * c, inner_row(z) && inner_col(x + c) && oq);
+            qa[h][c] = bld(image_rsrc(s.g1, s), oc, 0);
+            qb[h][c] = bld(image_rsrc(s.illum, s), oc, 0);
           }
         }
       }
-      if (rstrips) {                                   // reconstruction: stored p of strip cells
-        const int lr = strip_row_lr(s, iz);
-        const int sp_ = soff_p(lr, strip_row_ptb(s, iz), sc);
-        if (sp_ >= 0) {
-          qa[r] = store_raw(s, it, sp_);
-          sm |= 1ull << (SMP + r);
-          if (lr < 0) sm |= 1ull << (SMT + r);         // top/bottom block (rows outside n..nzp-n-1)
+    }
+  }
+  // stored p of the strip cells of an own quad (reconstruction)
+  f4 spr[KO];
+  if (strips) {
+#pragma unroll
+    for (int h = 0; h < KO; h++) {
+      const int z = zw + qrow(h), x = qx(h);
+      const int lr = strip_row_lr(s, z), tb = strip_row_ptb(s, z);
+      spr[h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int pl = lr >= 0 ? strip_col_plr(s, x + c) : -1;
+        const int st = pl >= 0 ? lr + pl : (tb >= 0 && inner_col(x + c) ? tb + x + c - npml : -1);
+        if (st >= 0) {
+          spr[h][c] = store_raw(s, it, st);
+          qsp[h] |= pl >= 0 ? 1 << c : 16 << c;
         }
       }
     }
   }
-  {
-    const rsrc_t Rvxn = field_rsrc(vxn, s);
-#pragma unroll
-    for (int r = 0; r < RPT; r++) {
-      const int j = g * RPT + r, iz = z0 + j;
-      const float* __restrict__ Pr = lds_base(PS + (j + 19) * PW + lx + 11) + 9;   // p at column ix
-#define PCA(i) Pr[(i)]
-      VEL_CELL(FK, gen, strips, (sbit(SMX + r) ? 0 : -1), vxv, rrx,
-               (ix >= npml && ix <= nxp - npml - 2 && iz >= npml && iz < nzp - npml), PCA, vxo[r], ibx[r], dtx,
-               axv, bxv, vxn_[r]);
-#undef PCA
-      if (!gen) bst(Rvxn, vxn_[r], vcol, srow0 + j * pr4);
-      else bst(Rvxn, vxn_[r], pred_off(vcol, iz < nzp && ix <= nxp - 2), srow0 + j * pr4);
-      nzb |= __float_as_uint(vxn_[r]);
-    }
-#pragma unroll
-    for (int k = 0; k < KH; k++) {
-      const int iz = z0 + hrow[k], jx = x0 - 10 + hcol[k];
-      const float* __restrict__ Pr = lds_base(PS + (hrow[k] + 19) * PW + hcol[k] + 1) + 9;   // p at column jx
-      hvn[k] = 0.0f;
-      if (halo_on(k)) {
-        const bool hv = jx >= 0 && jx <= nxp - 2;
-#define PCA(i) Pr[(i)]
-        VEL_CELL(FK, gen, strips, (sbit(SMH + k) ? 0 : -1), hv, (hv ? imin(RTM_R, imin(jx + 1, nxp - 1 - jx)) : RTM_R),
-                 (jx >= npml && jx <= nxp - npml - 2 && iz >= npml && iz < nzp - npml), PCA, hvo[k], hib[k], dtx,
-                 DMP[DXA + hcol[k]], DMP[DXB + hcol[k]], hvn[k]);
-#undef PCA
-      }
-    }
-  }
 
-  // own old pressure out of LDS
-  float po[RPT];
-#pragma unroll
-  for (int r = 0; r < RPT; r++) po[r] = PS[(g * RPT + r + 19) * PW + 20 + lx];
   __syncthreads();                                     // PS consumed
 #pragma unroll
-  for (int k = 0; k < KZ; k++) {
-    const int kz = g * KZ + k;
-    if (kz < ZR) VZL[kz * 64 + lx] = vzn_[k];
-  }
+  for (int k = 0; k < KZ; k++)
+    if (zrow(k)) VZL[(g * KZ + k) * 64 + lane] = vzn_[k];
 #pragma unroll
-  for (int r = 0; r < RPT; r++) VXL[(g * RPT + r) * VXW + lx + 10] = vxn_[r];
-#pragma unroll
-  for (int k = 0; k < KH; k++)
-    if (halo_on(k)) VXL[hrow[k] * VXW + hcol[k]] = hvn[k];
+  for (int k = 0; k < KQ; k++)
+    if ((k < KO && oq) || ((k >= KO || RPT < 4) && hon)) {
+      f2* d = (f2*)(VXL + (g * RPT + qrow(k)) * VXW + qcol(k) + 10);
+      d[0] = f2{hv[k].x, hv[k].y};
+      d[1] = f2{hv[k].z, hv[k].w};
+    }
   __syncthreads();                                     // new velocities staged
 
-  // ---- 3. x-differences of the new vx by row segments: thread tid takes
-  //         RPT consecutive cells of one tile row and reads their vx window
-  //         once (RPT + 19 values instead of 20 per cell), and parks the sums
-  //         in SXL for the pressure update.  The radius is the cell's own
-  //         (the same rule as the pressure update's); a segment of a wave
-  //         with any reduced-radius cell takes the zero-padded coefficient
-  //         rows, which give the radius-10 sums bit for bit.
-  float* SXL = lds + TZ * VXW + ZR * 64;
-  {
-    constexpr int NSEG = 64 / RPT;                     // NSEG * TZ == NT
-    const int j = tid / NSEG, c0 = (tid - j * NSEG) * RPT;
-    const int iz = z0 + j;
-    float w[RPT + 19];                                 // vx at columns x0 + c0 - 10 ..
+  // ---- 4. differences of the new velocities (kernel.cu:520-534): in x by
+  //         own quads, in z by columns, the latter handed to the quads
+  //         through the wave's vx rows.  Radius of a cell: min(10, distance
+  //         to the nearest grid edge); cells off the grid or on its ring are
+  //         computed with radius 10 and dropped
+  f4 dx_[KO], dz_[KO];
 #pragma unroll
-    for (int m = 0; m < RPT + 19; m++) w[m] = VXL[j * VXW + c0 + m];
-    int radc[RPT];
-    bool red = false;
+  for (int h = 0; h < KO; h++) {
+    part();
+    float w[24];                                       // vx at columns x-10 .. x+13
+    const f4* row = (const f4*)(VXL + (g * RPT + qrow(h)) * VXW + (oq ? ocol : 0));
 #pragma unroll
-    for (int c = 0; c < RPT; c++) {
-      radc[c] = RTM_R;
-      if (FK != FK_RCN && gen) {
-        const int jx = x0 + c0 + c;
-        const bool upd = iz > 0 && iz < nzp - 1 && jx < nxp && jx != 0 && jx != nxp - 1;
-        if (upd) radc[c] = imin(imin(RTM_R, imin(jx, nxp - 1 - jx)), imin(iz, nzp - 1 - iz));
-        red = red || radc[c] != RTM_R;
-      }
+    for (int m = 0; m < 6; m++) {
+      const f4 v = row[m];
+      w[4 * m] = v.x; w[4 * m + 1] = v.y; w[4 * m + 2] = v.z; w[4 * m + 3] = v.w;
     }
-    if (FK == FK_RCN || !gen || !any_lane(red)) {
+    int rad[4] = {RTM_R, RTM_R, RTM_R, RTM_R};
+    bool red = false;
+    if (EDGE && !RCN) {
 #pragma unroll
-      for (int c = 0; c < RPT; c++) {
-        float sx = 0.0f;
-#pragma unroll
-        for (int i = 1; i <= RTM_R; i++) sx = __builtin_fmaf(c10[i - 1], w[c + 9 + i] - w[c + 10 - i], sx);
-        SXL[j * 64 + c0 + c] = sx;
+      for (int c = 0; c < 4; c++) {
+        const int x = qx(h) + c, z = zw + qrow(h);
+        if (z > 0 && z < nzp - 1 && x > 0 && x < nxp - 1)
+          rad[c] = imin(imin(RTM_R, imin(x, nxp - 1 - x)), imin(z, nzp - 1 - z));
+        red = red || rad[c] != RTM_R;
       }
-    } else {
+      red = any_lane(red);
+    }
 #pragma unroll
-      for (int c = 0; c < RPT; c++) {
-        const float* cr = lds_base(ctab + (radc[c] - 1) * RTM_R);
-        float sx = 0.0f;
-#pragma unroll
-        for (int i = 1; i <= RTM_R; i++) sx = __builtin_fmaf(cr[i - 1], w[c + 9 + i] - w[c + 10 - i], sx);
-        SXL[j * 64 + c0 + c] = sx;
-      }
+    for (int c = 0; c < 4; c++) {
+      float v;
+      if (EDGE && !RCN && red) v = taps_r(w, 9 + c, ctab, rad[c]);
+      else v = taps(w, 9 + c, c10);
+      pin(v);
+      dx_[h][c] = v;
     }
   }
-  __syncthreads();                                     // x-differences staged
-
-  // ---- 4. new pressure of the own cells
-  float cz[RPT + 19];
+  part();
+  {
+    float cz[RPT + 19];                                // new vz rows zw-10 + m of the column
 #pragma unroll
-  for (int m = 0; m < RPT + 19; m++) cz[m] = VZL[(g * RPT + m) * 64 + lx];
-  const int radx = imin(RTM_R, imin(ix, nxp - 1 - ix));
-  const bool xsrc = (tl.kind & TF_SRC) && ix >= s.sx0 && ix <= s.sx1;
-  const rsrc_t Rpn = field_rsrc(pn, s);
-
+    for (int m = 0; m < RPT + 19; m++) cz[m] = VZL[(g * RPT + m) * 64 + lane];
+    const rsrc_t Rvzn = field_rsrc(vzn, s);
+    float* T = VXL + g * RPT * VXW;                    // the wave's vx rows, consumed above
+    float szc[RPT];
 #pragma unroll
-  for (int r = 0; r < RPT; r++) {
-    const int j = g * RPT + r;
-    const int iz = z0 + j;                             // wave-uniform
-    const int so = srow0 + j * pr4;
-    float p = po[r];
-    const float sxl = SXL[j * 64 + lx];
-    const bool incell = ix < nxp && iz < nzp;
-    if (FK == FK_RCN) {
-      const bool inner = xin && iz >= npml && iz < nzp - npml;
-      // computed for every cell and then selected (no divergent branch):
-      // interior cells take the update, strip cells the stored value
-      DivV d;
-      d.sx = sxl;
-      d.sz = div_z(cz, r, RTM_R, c10, ctab);
-      const float pc = __builtin_fmaf(kk[r], pres_sum(d, dtx, dtz), p);   // kernel.cu:389-429
-      bool wr = !gen || inner;
-      if (wr) p = pc;
-      if (strips && sbit(SMP + r)) {
-        p = store_decode(s, sbit(SMT + r) ? 3 : 2, qa[r], DMP + 4);   // kernel.cu:1348-1400
-        wr = true;
-      }
-      if ((tl.kind & TF_SRC) && iz >= s.sz0 && iz <= s.sz1 && wr && xsrc)   // source removal (rtm_model.cu:437)
-        p = __builtin_fmaf(-GCF(s.sa)[(iz - s.sz0) * (s.sx1 - s.sx0 + 1) + ix - s.sx0], GCF(s.wav)[it], p);
-      if (!gen) bst(Rpn, p, vcol, so);                 // every lane's cell is interior
-      else bst(Rpn, p, pred_off(vcol, wr), so);
-    } else {
-      if (!gen) {
-        DivV d;
-        d.sx = sxl;
-        d.sz = div_z(cz, r, RTM_R, c10, ctab);
-        p = __builtin_fmaf(-kk[r], pres_sum(d, dtx, dtz), p);  // kernel.cu:539
+    for (int r = 0; r < RPT; r++) {
+      if (r % 2 == 0) part();
+      const int iz = zw + r;
+      bst(Rvzn, cz[r + 10], GEN ? pred_off(vcol, ix < nxp && iz < nzp) : vcol, srow0 + (g * RPT + r) * pr4);
+      nzb |= __float_as_uint(cz[r + 10]);
+      if (EDGE && !RCN) {
+        int rad = RTM_R;
+        if (iz > 0 && iz < nzp - 1 && ix > 0 && ix < nxp - 1)
+          rad = imin(imin(RTM_R, imin(ix, nxp - 1 - ix)), imin(iz, nzp - 1 - iz));
+        szc[r] = any_lane(rad != RTM_R) ? taps_r(cz, r + 9, ctab, rad) : taps(cz, r + 9, c10);
       } else {
-        // the outer ring keeps its value (only the source is added there);
-        // cells off the grid are computed with radius 10 and dropped
-        const bool zupd = iz > 0 && iz < nzp - 1;
-        const bool upd = zupd && incell && !xring;
-        const int rad = upd ? imin(radx, imin(iz, nzp - 1 - iz)) : RTM_R;
-        DivV d;
-        d.sx = sxl;
-        if (!any_lane(rad != RTM_R)) d.sz = div_z(cz, r, RTM_R, c10, ctab);
-        else d.sz = div_z(cz, r, rad, c10, ctab);
-        const bool split = upd && !(xin && iz >= npml && iz < nzp - npml);
-        float pu = __builtin_fmaf(-kk[r], pres_sum(d, dtx, dtz), p);
-        if (any_lane(split)) {                         // split pair, p = p1 + p2 (kernel.cu:780-783)
-          const rsrc_t R1 = field_rsrc(s.q1, s), R2 = field_rsrc(s.q2, s);
-          float q1 = qa[r], q2 = qb[r];
-          const float dxv = (d.sx * dtx) * kk[r], dzv = (d.sz * dtz) * kk[r];
-          q1 = __builtin_fmaf(ax, q1, -(dxv * bx));   // (c1 q - d)/c2 (kernel.cu:774-779)
-          q2 = __builtin_fmaf(DMP[DPA + j], q2, -(dzv * DMP[DPB + j]));
-          const int pq = pred_off(vcol, split);
-          bst(R1, q1, pq, so);
-          bst(R2, q2, pq, so);
-          if (split) nzb |= __float_as_uint(q1) | __float_as_uint(q2);
-          if (split) pu = q1 + q2;
-        }
-        if (upd) p = pu;
+        szc[r] = taps(cz, r + 9, c10);
       }
-      if (FK == FK_SRC) {
-        if ((tl.kind & TF_SRC) && iz >= s.sz0 && iz <= s.sz1 && xsrc)   // kernel.cu:36-47
-          p = __builtin_fmaf(GCF(s.sa)[(iz - s.sz0) * (s.sx1 - s.sx0 + 1) + ix - s.sx0], GCF(s.wav)[it], p);
-        auto record = [&](bool on) {
-          if ((tl.kind & TF_REC) && s.record && iz == npml) {   // kernel.cu:48-71
-            const int ir = ix - s.rcol0;
-            if (on && ir >= 0 && ir < s.nrec) GF(s.rec)[(size_t)it * s.nrec + ir] = p;
-          }
-        };
-        if (!gen) {
-          bst(Rpn, p, vcol, so);
-          record(true);
-        } else {
-          bst(Rpn, p, pred_off(vcol, incell), so);
-          record(incell);
-        }
-      } else {                                         // receiver wavefield
-        if ((tl.kind & TF_REC) && iz == npml) {        // Dirichlet insertion (kernel.cu:72-95)
-          const int ir = ix - s.rcol0;
-          if (ir >= 0 && ir < s.nrec) {
-            const float rv = (it <= ((const gint*)s.cut)[ir]) ? 0.0f : GCF(s.rec)[(size_t)it * s.nrec + ir];
-            p = s.dt * rv;
-          }
-        }
-        auto image = [&]() {                           // imaging (kernel.cu:1401-1416)
-          const int io = (iz - npml) * s.nxl * 4;
-          bst(image_rsrc(s.g1, s), __builtin_fmaf(ps[r], p, qa[r]), icol, io);
-          bst(image_rsrc(s.illum, s), __builtin_fmaf(ps[r], ps[r], qb[r]), icol, io);
-        };
-        if (!gen) {                                    // every lane's cell is interior
-          bst(Rpn, p, vcol, so);
-          image();
-        } else {
-          bst(Rpn, p, pred_off(vcol, incell), so);
-          const bool im = incell && xin && iz >= npml && iz < nzp - npml;
-          if (any_lane(im)) {
-            const int io = imax(iz - npml, 0) * s.nxl * 4;
-            const int pi = pred_off(icol, im);
-            bst(image_rsrc(s.g1, s), __builtin_fmaf(ps[r], p, qa[r]), pi, io);
-            bst(image_rsrc(s.illum, s), __builtin_fmaf(ps[r], ps[r], qb[r]), pi, io);
-          }
-        }
-      }
-      nzb |= __float_as_uint(p);
     }
-    pnew[r] = p;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < RPT; r++) T[r * 64 + lane] = szc[r];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int h = 0; h < KO; h++) dz_[h] = *(const f4*)(T + (oq ? qrow(h) * 64 + ocol : 0));
+  }
+
+  // ---- 5. new pressure of the own quads
+  const rsrc_t Rpn = field_rsrc(pn, s);
+#pragma unroll
+  for (int h = 0; h < KO; h++) {
+    part();
+    const int z = zw + qrow(h), x = qx(h);
+    const bool on = oq;
+    f4 p = po[h];
+    if (RCN) {
+      if (img) {                                       // imaging of the step before (kernel.cu:1401-1416)
+        const int o = ((z - npml) * s.nxl + x - npml) * 4;
+        f4 gi, ii;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          gi[c] = __builtin_fmaf(po[h][c], qc[h][c], qa[h][c]);
+          ii[c] = __builtin_fmaf(po[h][c], po[h][c], qb[h][c]);
+        }
+        if (!GEN) {
+          const int oo = pred_off(o, on);
+          bst4(image_rsrc(s.g1, s), gi, oo, 0);
+          bst4(image_rsrc(s.illum, s), ii, oo, 0);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const int oc = pred_off(o + 4 * c, inner_row(z) && inner_col(x + c) && on);
+            bst(image_rsrc(s.g1, s), gi[c], oc, 0);
+            bst(image_rsrc(s.illum, s), ii[c], oc, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const float sum = __builtin_fmaf(dx_[h][c], dtx, dz_[h][c] * dtz);
+        float v = __builtin_fmaf(kk[h][c], sum, po[h][c]);   // kernel.cu:389-429
+        bool wr = true;
+        if (GEN) {
+          wr = inner_row(z) && inner_col(x + c);
+          if (strips && (qsp[h] >> c) & 17) {
+            v = store_value(s, (qsp[h] >> c) & 1 ? scv[2] : scv[3], spr[h][c]);   // kernel.cu:1348-1400
+            wr = true;
+          }
+          v = wr ? v : 0.0f;                           // cells the reconstruction does not hold
+        }
+        p[c] = v;
+      }
+      if (tl.kind & TF_SRC) {                          // source removal (rtm_model.cu:437)
+        const float wv = CCF(s.wav)[it];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const bool wr = !GEN || (inner_row(z) && inner_col(x + c)) || (strips && ((qsp[h] >> c) & 17));
+          if (wr && on && z >= s.sz0 && z <= s.sz1 && x + c >= s.sx0 && x + c <= s.sx1)
+            p[c] = __builtin_fmaf(-GCF(s.sa)[(z - s.sz0) * (s.sx1 - s.sx0 + 1) + x + c - s.sx0], wv, p[c]);
+        }
+      }
+      bst4(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+      continue;
+    }
+    f4 pu;
+#pragma unroll
+    for (int c = 0; c < 4; c++)                        // p - rho v^2 (sx dt/dx + sz dt/dz) (kernel.cu:536-539)
+      pu[c] = __builtin_fmaf(-kk[h][c], __builtin_fmaf(dx_[h][c], dtx, dz_[h][c] * dtz), po[h][c]);
+    if (!GEN) {
+      p = pu;
+    } else {
+      // the outer ring and the cells off the grid keep their value
+#pragma unroll
+      for (int c = 0; c < 4; c++) p[c] = inner_row(z) && inner_col(x + c) ? pu[c] : po[h][c];
+      if (any_lane(qsp[h] != 0 && on)) {               // split pair, p = p1 + p2 (kernel.cu:774-783)
+        const f4 ax = *(const gf4*)(GCF(s.ax) + x);
+        const f4 bx = *(const gf4*)(GCF(s.bx) + x);
+        const float az = GCF(s.az)[z], bz = GCF(s.bz)[z];
+        f4 q1, q2;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float dxv = (dx_[h][c] * dtx) * kk[h][c], dzv = (dz_[h][c] * dtz) * kk[h][c];
+          const bool sp = (qsp[h] >> c) & 1;
+          q1[c] = sp ? __builtin_fmaf(ax[c], qa[h][c], -(dxv * bx[c])) : qa[h][c];   // (c1 q - d)/c2
+          q2[c] = sp ? __builtin_fmaf(az, qb[h][c], -(dzv * bz)) : qb[h][c];
+          if (sp) p[c] = q1[c] + q2[c];
+          if (on) nzb |= __float_as_uint(q1[c]) | __float_as_uint(q2[c]);
+        }
+        const int o = pred_off(ooff, qsp[h] != 0 && on);
+        bst4(field_rsrc(s.q1, s), q1, o, qsoff(h));
+        bst4(field_rsrc(s.q2, s), q2, o, qsoff(h));
+      }
+    }
+    if (FK == FK_SRC && (tl.kind & TF_SRC)) {          // kernel.cu:36-47
+      const float wv = CCF(s.wav)[it];
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        if (on && z >= s.sz0 && z <= s.sz1 && x + c >= s.sx0 && x + c <= s.sx1)
+          p[c] = __builtin_fmaf(GCF(s.sa)[(z - s.sz0) * (s.sx1 - s.sx0 + 1) + x + c - s.sx0], wv, p[c]);
+    }
+    if (tl.kind & TF_REC) {
+      if (on && z == npml && (FK == FK_RCV || s.record)) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const int ir = x + c - s.rcol0;
+          if (ir >= 0 && ir < s.nrec) {
+            if (FK == FK_SRC) {                        // kernel.cu:48-71
+              GF(s.rec)[(size_t)it * s.nrec + ir] = p[c];
+            } else {                                   // Dirichlet insertion (kernel.cu:72-95)
+              const float rv = (it <= ((const gint*)s.cut)[ir]) ? 0.0f : GCF(s.rec)[(size_t)it * s.nrec + ir];
+              p[c] = s.dt * rv;
+            }
+          }
+        }
+      }
+    }
+    if (on)
+#pragma unroll
+      for (int c = 0; c < 4; c++) nzb |= __float_as_uint(p[c]);
+    bst4(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
   }
   if (FK == FK_SRC && actw) {
     const bool any = any_lane(nzb != 0u);
-    if (lx == 0) actw[g] = any ? 1 : 0;
+    // (a word is 8 bytes whatever the wave count: its bytes start non-zero)
+    if (lane == 0) {
+      if (G == 4) ((unsigned short*)actw)[g] = any ? 1 : 0;
+      else actw[g] = any ? 1 : 0;
+    }
+  }
+}
+
+template <class Q, int FK>
+__device__ __forceinline__ void field_step(float* __restrict__ lds, float* __restrict__ ctab, const ShotDev& s,
+                                           const Tile& tl, int it, const float* pc, const float* vxc,
+                                           const float* vzc, float* pn, float* vxn, float* vzn,
+                                           const float* pr = nullptr, bool img = false, unsigned char* actw = nullptr)
+{
+  if (!(tl.kind & TF_GEN)) {
+    tile_step<Q, FK, TC_IN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
+  } else if (FK == FK_RCN || !(tl.kind & TF_EDGE)) {
+    tile_step<Q, FK, TC_GEN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
+  } else {
+    for (int t = threadIdx.x; t < RTM_R * CTW; t += Q::NT) ctab[t] = ctab_entry(s, t);   // read after the first barrier
+    tile_step<Q, FK, TC_EDGE>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
   }
 }
 
@@ -863,16 +899,24 @@ __device__ __forceinline__ bool skip_of(const SkipWords& w, int it)
   return (in | out) == 0ull;
 }
 
+// index of the snapshot of step k (below: decimated snapshots), -1 if none
+__device__ __forceinline__ int snap_index(const ShotDev& s, int k)
+{
+  if (!s.snap || k < 0 || k % s.snap_every != 0) return -1;
+  const int q = k / s.snap_every - s.snap_k0;
+  return (q >= 0 && q < s.nsnap) ? q : -1;
+}
+
 }  // namespace
 
 // ================================================================ kernels ==
 // forward time step of the source wavefield (modelling, recording, strips)
 template <int G, int RPT>
-__global__ __launch_bounds__(64 * G) void k_fwd(LaunchArgs a)
+__global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd(LaunchArgs a)
 {
   using Q = Geo<G, RPT>;
-  __shared__ float lds[Q::LDS + Q::LDS_D];
-  __shared__ float ctab[100];                          // coefficient table (reduced radii near the edges)
+  __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
+  __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];   // coefficient table (reduced radii near the edges)
   const int t = xcd_tile(a.ntiles);
   if (t < 0) return;
   const Tile tl = a.tiles[t];
@@ -883,45 +927,77 @@ __global__ __launch_bounds__(64 * G) void k_fwd(LaunchArgs a)
   const ShotDev& s = shot_of(a.shots, tl.slot);
   const int it = s.it_off + s.it_dir * a.step;
   if (track && skip_of(sw, it)) return;                // the forward field is +0 around the tile
-  if (threadIdx.x < 100) ctab[threadIdx.x] = ctab_entry(s, threadIdx.x);
   const bool odd = it & 1;                             // (a runtime index into s would spill it to scratch)
-  float none[Q::RPT], pnew[Q::RPT];
-#pragma unroll
-  for (int r = 0; r < Q::RPT; r++) none[r] = 0.0f;
   unsigned char* actw = a.act ? (unsigned char*)(a.act + (size_t)((it + 1) & 1) * a.ntiles + t) : nullptr;
-  field_step<Q, FK_SRC>(lds, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
+  field_step<Q, FK_SRC>(lds, ctab, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
                         odd ? s.svz[1] : s.svz[0], odd ? s.sp[0] : s.sp[1], odd ? s.svx[0] : s.svx[1],
-                        odd ? s.svz[0] : s.svz[1], ctab, none, pnew, actw);
+                        odd ? s.svz[0] : s.svz[1], nullptr, false, actw);
 }
 
-// reverse time step: source reconstruction, then the receiver wavefield and
-// the imaging products of the tile
+// tiles whose receiver halves, then reconstruction halves, follow each other
+// on an XCD: workgroups go to its shader engines in turn, so alternating the
+// two kinds one by one gave half of the engines the shorter kind only (10.3 of
+// 16 waves resident per CU, 634 us a reverse step of 128 survey shots; in
+// groups of 8, 16 or 32: 13.5 waves, 519 us)
+constexpr int RGRP = 16;
+
+// reverse time step: two workgroups per tile, close together on one XCD, one
+// for the receiver wavefield and one for the source reconstruction with the
+// imaging products.  The reconstruction images the step before (both fields'
+// old levels: its own pressure is staged anyway, the receiver pressure is in
+// L2 from the other workgroup), so the two run at the same time; the last
+// step's products are added by k_image after the pass, those of a step whose
+// snapshot is restored by k_snap_load before it overwrites the field.
 template <int G, int RPT>
-__global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(G == 4 && RPT == 4 ? 5 : 1))) void k_rev(LaunchArgs a)
+__global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_rev(LaunchArgs a)
 {
   using Q = Geo<G, RPT>;
-  __shared__ float lds[Q::LDS + Q::LDS_D];
-  __shared__ float ctab[100];
-  const int t = xcd_tile(a.ntiles);
-  if (t < 0) return;
+  __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
+  __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];
+  // XCD c's workgroups take its run of the table RGRP tiles at a time, their
+  // receiver halves and then their reconstruction halves
+  const int per = (a.ntiles + 7) >> 3, b = blockIdx.x >> 3, r = b % (2 * RGRP);
+  const int i = b / (2 * RGRP) * RGRP + r % RGRP;
+  if (i >= per) return;
+  const int t = (blockIdx.x & 7) * per + i;
+  if (t >= a.ntiles) return;
   const Tile tl = a.tiles[t];
   if (tl.slot < 0) return;                             // padding of a shorter XCD run
   const ShotDev& s = shot_of(a.shots, tl.slot);
-  if (threadIdx.x < 100) ctab[threadIdx.x] = ctab_entry(s, threadIdx.x);
   const int it = s.it_off + s.it_dir * a.step;
   const bool odd = it & 1;
-  float ps[Q::RPT], pr[Q::RPT], none[Q::RPT];
-#pragma unroll
-  for (int r = 0; r < Q::RPT; r++) ps[r] = none[r] = 0.0f;
-  if (tl.kind & TF_INT) {
-    field_step<Q, FK_RCN>(lds, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
+  if (r >= RGRP) {
+    if (!(tl.kind & TF_INT)) return;
+    const bool img = it < s.nt - 2 && snap_index(s, it + 1) < 0;
+    field_step<Q, FK_RCN>(lds, ctab, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
                           odd ? s.svz[1] : s.svz[0], odd ? s.sp[0] : s.sp[1], odd ? s.svx[0] : s.svx[1],
-                          odd ? s.svz[0] : s.svz[1], ctab, none, ps);
-    __syncthreads();                                   // LDS reused by the receiver pass
+                          odd ? s.svz[0] : s.svz[1], odd ? s.rp[1] : s.rp[0], img);
+  } else {
+    field_step<Q, FK_RCV>(lds, ctab, s, tl, it, odd ? s.rp[1] : s.rp[0], odd ? s.rvx[1] : s.rvx[0],
+                          odd ? s.rvz[1] : s.rvz[0], odd ? s.rp[0] : s.rp[1], odd ? s.rvx[0] : s.rvx[1],
+                          odd ? s.rvz[0] : s.rvz[1]);
   }
-  field_step<Q, FK_RCV>(lds, s, tl, it, odd ? s.rp[1] : s.rp[0], odd ? s.rvx[1] : s.rvx[0],
-                        odd ? s.rvz[1] : s.rvz[0], odd ? s.rp[0] : s.rp[1], odd ? s.rvx[0] : s.rvx[1],
-                        odd ? s.rvz[0] : s.rvz[1], ctab, ps, pr);
+}
+
+// imaging products of reverse step `it` of the listed slots from the levels
+// it wrote (kernel.cu:1401-1416): the last step of a pass, which no later
+// step images.  Grid (slots, GY), one wave per row.
+__global__ __launch_bounds__(NTHR) void k_image(const ShotDev* __restrict__ shots, const int* __restrict__ slots, int it)
+{
+  const ShotDev& s = shot_of(shots, slots[blockIdx.x]);
+  const bool lev = (it + 1) & 1;
+  const float* fs = lev ? s.sp[1] : s.sp[0];
+  const float* fr = lev ? s.rp[1] : s.rp[0];
+  const int nxl = s.nxl, lane = threadIdx.x & 63;
+  for (int r = blockIdx.y * (NTHR / 64) + (threadIdx.x >> 6); r < s.nzi; r += gridDim.y * (NTHR / 64)) {
+    const long long o = (long long)(s.npml + r) * s.pitch + s.npml;
+    for (int c = lane; c < nxl; c += 64) {
+      const float ps = GCF(fs)[o + c], p = GCF(fr)[o + c];
+      const long long e = (long long)r * nxl + c;
+      GF(s.g1)[e] = __builtin_fmaf(ps, p, GCF(s.g1)[e]);
+      GF(s.illum)[e] = __builtin_fmaf(ps, ps, GCF(s.illum)[e]);
+    }
+  }
 }
 
 // Boundary strips of forward step `it` -- the new fields of that step -- into
@@ -1084,12 +1160,6 @@ __global__ __launch_bounds__(NTHR) void k_model_prep(const float* __restrict__ r
 // start from the stored field.  Block (q, f), f = 0 p, 1 vx, 2 vz: nzi x nxl
 // codes; 16-bit forms with one max-abs scale per block (the strips' rule:
 // max(maxabs / 32768, FLT_MIN), 1 for an all-zero block).
-__device__ __forceinline__ int snap_index(const ShotDev& s, int k)
-{
-  if (!s.snap || k < 0 || k % s.snap_every != 0) return -1;
-  const int q = k / s.snap_every - s.snap_k0;
-  return (q >= 0 && q < s.nsnap) ? q : -1;
-}
 // the snapshot a forward step `it` contributes field f to: p of step k = it,
 // velocities of step it = k + 1
 __device__ __forceinline__ int snap_of_fwd(const ShotDev& s, int it, int f)
@@ -1189,7 +1259,8 @@ __global__ __launch_bounds__(NTHR) void k_snap_q(const ShotDev* __restrict__ sho
 // k replaces the reconstructed interior cells: p on the
 // interior, vx on its columns npml..nxp-npml-2, vz on its rows
 // npml..nzp-npml-2 (the cells the reconstruction computes; the strips come
-// from the boundary store as on every step)
+// from the boundary store as on every step).  The step's imaging products are
+// added first: they take the reconstructed pressure
 __global__ __launch_bounds__(NTHR) void k_snap_load(const ShotDev* __restrict__ shots, const int* __restrict__ slots,
                                                      int step)
 {
@@ -1203,9 +1274,19 @@ __global__ __launch_bounds__(NTHR) void k_snap_load(const ShotDev* __restrict__ 
   const int ncol = f == 1 ? nxl - 1 : nxl, nrow = f == 2 ? s.nzi - 1 : s.nzi;
   const long long base = (long long)(q * 3 + f) * n;
   const float sc = s.snap_scale[q * 3 + f];
+  const float* fr = (it + 1) & 1 ? s.rp[1] : s.rp[0];
   for (int r = blockIdx.y * SWB + (threadIdx.x >> 6); r < nrow; r += gridDim.y * SWB) {
     gfloat* row = GF(fld) + (long long)(s.npml + r) * s.pitch + s.npml;
     const long long ib = base + (long long)r * nxl;
+    if (f == 0) {                                      // the step's imaging products, before its field is replaced
+      const gfloat* rr = GCF(fr) + (long long)(s.npml + r) * s.pitch + s.npml;
+      for (int c = lane; c < nxl; c += 64) {
+        const float ps = row[c], p = rr[c];
+        const long long e = (long long)r * nxl + c;
+        GF(s.g1)[e] = __builtin_fmaf(ps, p, GCF(s.g1)[e]);
+        GF(s.illum)[e] = __builtin_fmaf(ps, ps, GCF(s.illum)[e]);
+      }
+    }
     for (int c0 = lane; c0 < ncol; c0 += SU * 64) {
       float v[SU];
 #pragma unroll
@@ -1704,9 +1785,9 @@ static inline int grid8(int ntiles) { return ((ntiles + 7) / 8) * 8; }
 template <int G, int RPT>
 static hipError_t launch_step_t(const LaunchArgs& a, int phase, hipStream_t st)
 {
-  const dim3 g(grid8(a.ntiles)), b(64 * G);
-  if (phase == PH_FWD) hipLaunchKernelGGL((k_fwd<G, RPT>), g, b, 0, st, a);
-  else hipLaunchKernelGGL((k_rev<G, RPT>), g, b, 0, st, a);
+  const dim3 b(64 * G);
+  if (phase == PH_FWD) hipLaunchKernelGGL((k_fwd<G, RPT>), dim3(grid8(a.ntiles)), b, 0, st, a);
+  else hipLaunchKernelGGL((k_rev<G, RPT>), dim3(16 * (((a.ntiles + 7) / 8 + RGRP - 1) / RGRP * RGRP)), b, 0, st, a);
   return hipGetLastError();
 }
 
@@ -1714,14 +1795,26 @@ hipError_t rtm_launch_step(const LaunchArgs& a, int phase, int tz, hipStream_t s
 {
   if (a.ntiles <= 0) return hipSuccess;
   switch (tz) {
-    case 16: return launch_step_t<4, 4>(a, phase, st);
-    // 32 rows: the forward step as 8 waves x 4 rows (76 registers, 6 waves
-    // per SIMD), the reverse step as 4 waves x 8 rows (its 8 x 4 form needs
-    // 91 registers and loses 15 %)
-    case 32: return phase == PH_FWD ? launch_step_t<8, 4>(a, phase, st) : launch_step_t<4, 8>(a, phase, st);
+    // 16 rows are the height of the smallest launches.  Up to one and a half
+    // tiles per CU the time is a workgroup's own chain of phases, which 8
+    // waves of 2 rows shorten; past that the 4 x 4 form does less halo work a
+    // wave.  us per forward (with its strip save) / reverse step, 8 x 2
+    // against 4 x 4: one 184 x 124 window (24 tiles) 10.3 / 9.5 against 11.4 /
+    // 11.6, 480 x 280 (144) 11.5 / 12.5 against 12.6 / 13.0, 401 x 612 (273)
+    // 14.3 / 10.9 against 15.4 / 12.3, two of them (546) 15.9 / 18.2 against
+    // 16.0 / 15.1, four 24.4 / 29.9 against 22.2 / 24.9
+    case 16: return a.ntiles <= 384 ? launch_step_t<8, 2>(a, phase, st) : launch_step_t<4, 4>(a, phase, st);
+    case 32: return launch_step_t<4, 8>(a, phase, st);
     case 64: return launch_step_t<8, 8>(a, phase, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, int it, hipStream_t st)
+{
+  if (nslots <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_image, dim3(nslots, std::min(64, std::max(8, 2048 / nslots))), dim3(NTHR), 0, st, shots, slots, it);
+  return hipGetLastError();
 }
 
 hipError_t rtm_launch_save(const ShotDev* shots, const int* slots, int nslots, int step, int store_fmt,

@@ -7,6 +7,9 @@
 // modelling) or PH_REV (reconstruction, receiver wavefield, imaging); tz the
 // tile height (16, 32 or 64)
 hipError_t rtm_launch_step(const LaunchArgs& a, int phase, int tz, hipStream_t st);
+// after the last reverse step `it` of the listed slots: its imaging products
+// (every other reverse step's are added by the step after it)
+hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, int it, hipStream_t st);
 // after a forward step: its boundary strips into the store of the listed
 // slots (fp32 copy, or 16-bit with per-step block scales; one workgroup per
 // slot and strip block)

@@ -598,6 +598,7 @@ void Server::finish_shot(int sid)
   SrvRequest& r = *reqs_[sl.req];
   const int k = sl.k;
   const size_t n = (size_t)r.P.nz * r.setup[k].g.nxl * 4;
+  (void)rtm_launch_image(d_ds_, d_id_ + sid, 1, 0, st_);   // the last reverse step's imaging products
   // the guard after the shot's last step (tick_ - 1), then its word to the host
   (void)rtm_launch_guard(d_ds_, d_id_ + sid, 1, (int)(tick_ - 1), nullptr, st_);
   (void)hipMemcpyAsync(&r.guard[k], rtm_guard_word(hds_[sid]), 4, hipMemcpyDeviceToHost, st_);
