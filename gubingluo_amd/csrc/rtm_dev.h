@@ -127,4 +127,7 @@ struct LaunchArgs {
   // level one word whose byte g says that wave g stored a non-zero value of
   // the forward field at that level; two levels of ntiles words
   unsigned long long* act = nullptr;
+  // 1: the launches in flight keep their fields in the Infinity Cache
+  // (ordinary field stores; 0: stores with the non-temporal hint)
+  int cached = 0;
 };

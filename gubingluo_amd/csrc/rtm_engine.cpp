@@ -589,6 +589,7 @@ bool GraphKey::operator<(const GraphKey& o) const
   if (guard != o.guard) return guard < o.guard;
   if (snap != o.snap) return snap < o.snap;
   if (skip != o.skip) return skip < o.skip;
+  if (cached != o.cached) return cached < o.cached;
   if (shots != o.shots) return shots < o.shots;
   if (tiles != o.tiles) return tiles < o.tiles;
   return slots < o.slots;
@@ -597,7 +598,8 @@ bool GraphKey::operator<(const GraphKey& o) const
 Engine::Engine(int device) : device_(device)
 {
   (void)hipSetDevice(device_);
-  (void)hipStreamCreateWithFlags(&st_, hipStreamNonBlocking);
+  for (auto& l : lane_) (void)hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking);
+  st_ = lane_[0].st;
 }
 
 Engine::~Engine()
@@ -610,7 +612,8 @@ Engine::~Engine()
   models_.clear();
   if (cb_) (void)hipFree(cb_);
   pool_.trim();
-  if (st_) (void)hipStreamDestroy(st_);
+  for (auto& l : lane_)
+    if (l.st) (void)hipStreamDestroy(l.st);
 }
 
 void Engine::drop_graphs()
@@ -761,95 +764,212 @@ void Engine::layout_slot(const rtmh_params& P, const ShotSetup& s, int store_fmt
   }
 }
 
-hipGraphExec_t Engine::graph_for(const GraphKey& k, const ShotDev* dshots, const Tile* dtiles, const int* dslots,
-                                 int nslots, int store_fmt)
+int Engine::step_launches(const LaunchArgs& a, int phase, int tz, int store_fmt, const Lane& L, int nslots)
+{
+  HIPCHK(rtm_launch_step(a, phase, tz, L.st));
+  if (phase == PH_FWD) HIPCHK(rtm_launch_save(a.shots, L.slots, nslots, a.step, store_fmt, L.st));
+  else if (ic_cells_) HIPCHK(rtm_launch_ic(a.shots, L.slots, nslots, a.step, ic_cells_, L.st));
+  if (snap_.on()) HIPCHK(rtm_launch_snap(a.shots, L.slots, nslots, phase, a.step, snap_.fmt, L.st));
+  return 0;
+}
+
+hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
 {
   auto it = graphs_.find(k);
   if (it != graphs_.end()) return it->second;
   hipGraph_t g = nullptr;
-  if (hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
-  LaunchArgs a{dshots, dtiles, k.ntiles, 0};
-  if (k.skip) a.act = d_act_;
+  if (hipStreamBeginCapture(L.st, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
+  LaunchArgs a{d_ds_, L.tiles, k.ntiles, 0};
+  if (k.skip) a.act = L.act;
+  a.cached = k.cached;
   for (int s = 0; s < k.k; s++) {
     a.step = s;
-    (void)rtm_launch_step(a, k.phase, k.tz, st_);
-    if (k.save) (void)rtm_launch_save(dshots, dslots, nslots, s, store_fmt, st_);
-    if (k.ic) (void)rtm_launch_ic(dshots, dslots, nslots, s, k.ic, st_);
-    if (k.snap) (void)rtm_launch_snap(dshots, dslots, nslots, k.phase, s, k.snap - 1, st_);
+    (void)step_launches(a, k.phase, k.tz, k.fmt, L, k.nslots);
   }
-  (void)rtm_launch_bump((ShotDev*)dshots, dslots, nslots, k.k, st_);
+  (void)rtm_launch_bump(d_ds_, L.slots, k.nslots, k.k, L.st);
   // the chunk's last step, relative to the advanced time origin
-  if (k.guard) (void)rtm_launch_guard(dshots, dslots, nslots, -1, d_flag_, st_);
-  if (hipStreamEndCapture(st_, &g) != hipSuccess || !g) return nullptr;
+  if (k.guard) (void)rtm_launch_guard(d_ds_, L.slots, k.nslots, -1, d_flag_, L.st);
+  if (hipStreamEndCapture(L.st, &g) != hipSuccess || !g) return nullptr;
   hipGraphExec_t ex = nullptr;
   if (hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) != hipSuccess) ex = nullptr;
   (void)hipGraphDestroy(g);
   if (ex) graphs_[k] = ex;
-  (void)store_fmt;
   return ex;
 }
 
-int Engine::run_pass(int phase, int nsteps, const ShotDev* dshots, const Tile* dtiles, int ntiles,
-                     const std::vector<int>& slots, const int* dslots, int tz, int store_fmt, int chunk,
-                     rtmh_stats* prof, int guard_every, bool skip)
+double live_bytes(const ShotDev& d, int phase)
 {
-  // zero-tile skip words: every tile active until its first step has stepped
-  // (the words then follow the fields), whatever the fields hold now
-  unsigned long long* act = skip ? d_act_ : nullptr;
-  if (act) HIPCHK(hipMemsetAsync(act, 0xFF, 2 * (size_t)ntiles * sizeof(unsigned long long), st_));
-  const int save = phase == PH_FWD ? 1 : 0;
-  const int ic = phase == PH_REV ? ic_cells_ : 0;          // the other imaging conditions after each reverse step
-  const int nslots = (int)slots.size();
-  int done = 0;
-  if (prof) {
-    // every step kernel (and the strip save after it) bracketed by its own
-    // event pair on the launch stream
-    hipEvent_t ev[3];
-    for (auto& e : ev) HIPCHK(hipEventCreate(&e));
-    LaunchArgs a{dshots, dtiles, ntiles, 0};
-    a.act = act;
-    const int kb = phase == PH_FWD ? 0 : 2;
-    for (int s = 0; s < nsteps; s++) {
-      a.step = s;
-      HIPCHK(hipEventRecord(ev[0], st_));
-      HIPCHK(rtm_launch_step(a, phase, tz, st_));
-      HIPCHK(hipEventRecord(ev[1], st_));
-      if (save) HIPCHK(rtm_launch_save(dshots, dslots, nslots, s, store_fmt, st_));
-      if (ic) HIPCHK(rtm_launch_ic(dshots, dslots, nslots, s, ic, st_));
-      if (snap_.on()) HIPCHK(rtm_launch_snap(dshots, dslots, nslots, phase, s, snap_.fmt, st_));
-      HIPCHK(hipEventRecord(ev[2], st_));
-      HIPCHK(hipEventSynchronize(ev[2]));
-      float m0 = 0, m1 = 0;
-      HIPCHK(hipEventElapsedTime(&m0, ev[0], ev[1]));
-      HIPCHK(hipEventElapsedTime(&m1, ev[1], ev[2]));
-      prof->kern_ms[kb] += m0; prof->kern_calls[kb]++;
-      if (save) { prof->kern_ms[kb + 1] += m1; prof->kern_calls[kb + 1]++; }
-    }
-    for (auto& e : ev) (void)hipEventDestroy(e);
-    return 0;
+  const double cells = (double)d.nxp * d.nzp, in = (double)d.nxl * d.nzi;
+  // two levels of p, vx, vz of one field (forward) or two (reverse), the
+  // split pair in the layer, the imaging accumulators
+  return phase == PH_FWD ? 4 * (6 * cells + 2 * (cells - in)) : 4 * (12 * cells + 2 * (cells - in) + 2 * in);
+}
+
+std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int phase, bool& cached)
+{
+  const int nb = (int)ds.size();
+  double total = 0, most = 0;
+  for (const ShotDev& d : ds) {
+    const double b = live_bytes(d, phase);
+    total += b;
+    most = std::max(most, b);
   }
-  if (chunk > 0 && nsteps >= chunk) {
-    GraphKey key{ntiles, tz, phase, save, store_fmt, chunk, ic, nslots, guard_every > 0 ? 1 : 0,
-                 snap_.on() ? 1 + snap_.fmt : 0, act ? 1 : 0, dshots, dtiles, dslots};
-    hipGraphExec_t ex = graph_for(key, dshots, dtiles, dslots, nslots, store_fmt);
-    if (!ex) { set_error("hipGraph capture/instantiate failed"); return -11; }
-    const int nch = nsteps / chunk;
-    for (int c = 0; c < nch; c++) HIPCHK(hipGraphLaunch(ex, st_));
-    done = nch * chunk;
+  const double half = kCacheBytes / 2;
+  int n = 1;
+  if (nb > 1) {
+    n = 2;
+    if (most <= half && phase == PH_REV) n = 2 * std::max(1, (int)std::ceil(total / kCacheBytes));
+    n = std::min(n, nb);
   }
-  LaunchArgs a{dshots, dtiles, ntiles, 0};
-  a.act = act;
-  const int rest = nsteps - done;
-  for (int s = 0; s < rest; s++) {
+  std::vector<std::vector<int>> g(n);
+  double acc = 0;
+  for (int j = 0, k = 0; j < nb; j++) {
+    const double b = live_bytes(ds[j], phase);
+    // the next group from where its share starts; every group gets a shot
+    if (!g[k].empty() && k + 1 < n && (acc + 0.5 * b >= total * (k + 1) / n || nb - j <= n - 1 - k)) k++;
+    g[k].push_back(j);
+    acc += b;
+  }
+  // the two largest neighbours may run together
+  double worst = 0, prev = 0;
+  for (auto& v : g) {
+    double b = 0;
+    for (int j : v) b += live_bytes(ds[j], phase);
+    worst = std::max(worst, prev + b);
+    prev = b;
+  }
+  cached = worst <= 1.15 * kCacheBytes;
+  return g;
+}
+
+int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt, rtmh_stats* prof, bool skip)
+{
+  // every step kernel (and the strip save after it) bracketed by its own
+  // event pair on the launch stream
+  const Lane& L = lane_[0];
+  const int ntiles = (int)g.tiles.size(), nslots = (int)g.slots.size();
+  HIPCHK(hipMemcpyAsync(L.tiles, g.tiles.data(), ntiles * sizeof(Tile), hipMemcpyHostToDevice, st_));
+  HIPCHK(hipMemcpyAsync(L.slots, g.slots.data(), nslots * sizeof(int), hipMemcpyHostToDevice, st_));
+  LaunchArgs a{d_ds_, L.tiles, ntiles, 0};
+  if (skip) {
+    a.act = L.act;
+    HIPCHK(hipMemsetAsync(a.act, 0xFF, 2 * (size_t)ntiles * sizeof(unsigned long long), st_));
+  }
+  hipEvent_t ev[3];
+  for (auto& e : ev) HIPCHK(hipEventCreate(&e));
+  const int kb = phase == PH_FWD ? 0 : 2;
+  for (int s = 0; s < nsteps; s++) {
     a.step = s;
+    HIPCHK(hipEventRecord(ev[0], st_));
     HIPCHK(rtm_launch_step(a, phase, tz, st_));
-    if (save) HIPCHK(rtm_launch_save(dshots, dslots, nslots, s, store_fmt, st_));
-    if (ic) HIPCHK(rtm_launch_ic(dshots, dslots, nslots, s, ic, st_));
-    if (snap_.on()) HIPCHK(rtm_launch_snap(dshots, dslots, nslots, phase, s, snap_.fmt, st_));
-    if (guard_every > 0 && ((s + 1) % guard_every == 0 || s == rest - 1))
-      HIPCHK(rtm_launch_guard(dshots, dslots, nslots, s, d_flag_, st_));
+    HIPCHK(hipEventRecord(ev[1], st_));
+    if (phase == PH_FWD) HIPCHK(rtm_launch_save(d_ds_, L.slots, nslots, s, store_fmt, st_));
+    else if (ic_cells_) HIPCHK(rtm_launch_ic(d_ds_, L.slots, nslots, s, ic_cells_, st_));
+    if (snap_.on()) HIPCHK(rtm_launch_snap(d_ds_, L.slots, nslots, phase, s, snap_.fmt, st_));
+    HIPCHK(hipEventRecord(ev[2], st_));
+    HIPCHK(hipEventSynchronize(ev[2]));
+    float m0 = 0, m1 = 0;
+    HIPCHK(hipEventElapsedTime(&m0, ev[0], ev[1]));
+    HIPCHK(hipEventElapsedTime(&m1, ev[1], ev[2]));
+    prof->kern_ms[kb] += m0; prof->kern_calls[kb]++;
+    if (phase == PH_FWD) { prof->kern_ms[kb + 1] += m1; prof->kern_calls[kb + 1]++; }
   }
+  for (auto& e : ev) (void)hipEventDestroy(e);
   return 0;
+}
+
+int Engine::run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, int store_fmt, int chunk, bool cached,
+                     int guard_every, bool skip)
+{
+  // every group's table and slot list to the device; a lane copies the one it
+  // starts into its own place
+  std::vector<Tile>& tiles = stage_tiles_;
+  std::vector<int>& slots = stage_slots_;
+  tiles.clear();
+  slots.clear();
+  for (Group& g : groups) {
+    g.tile0 = tiles.size();
+    g.slot0 = slots.size();
+    tiles.insert(tiles.end(), g.tiles.begin(), g.tiles.end());
+    slots.insert(slots.end(), g.slots.begin(), g.slots.end());
+  }
+  HIPCHK(hipMemcpyAsync(d_tiles_, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
+  HIPCHK(hipMemcpyAsync(d_slots_, slots.data(), slots.size() * sizeof(int), hipMemcpyHostToDevice, st_));
+  struct Run {
+    size_t next;                                       // its next group
+    Group* g = nullptr;
+    int left = 0, step = 0;                            // steps left of the group; plain steps taken since its last chunk
+    hipGraphExec_t ex = nullptr;
+  } run[kLanes];
+  const int nl = std::min<int>(kLanes, (int)groups.size());
+  hipEvent_t ev;
+  HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+  int rc = 0;
+  auto body = [&]() -> int {
+    HIPCHK(hipEventRecord(ev, st_));                   // slots, tables and phase start are set up
+    for (int l = 1; l < nl; l++) HIPCHK(hipStreamWaitEvent(lane_[l].st, ev, 0));
+    for (int l = 0; l < nl; l++) run[l].next = l;
+    // one unit (a replayed chunk, or some plain steps) of each lane in turn,
+    // so that neither queue runs dry while the host fills the other
+    for (bool busy = true; busy;) {
+      busy = false;
+      for (int l = 0; l < nl; l++) {
+        Run& r = run[l];
+        const Lane& L = lane_[l];
+        if (!r.g) {
+          if (r.next >= groups.size()) continue;
+          Group& g = groups[r.next];
+          r.next += nl;
+          r.g = &g;
+          r.left = nsteps - g.done;
+          r.step = 0;
+          const int nt = (int)g.tiles.size(), ns = (int)g.slots.size();
+          HIPCHK(hipMemcpyAsync(L.tiles, d_tiles_ + g.tile0, nt * sizeof(Tile), hipMemcpyDeviceToDevice, L.st));
+          HIPCHK(hipMemcpyAsync(L.slots, d_slots_ + g.slot0, ns * sizeof(int), hipMemcpyDeviceToDevice, L.st));
+          // zero-tile skip words: every tile active until its first step has
+          // stepped (the words then follow the fields)
+          if (skip) HIPCHK(hipMemsetAsync(L.act, 0xFF, 2 * (size_t)nt * sizeof(unsigned long long), L.st));
+          r.ex = nullptr;
+          if (chunk > 0 && r.left >= chunk) {
+            GraphKey key{nt, tz, phase, phase == PH_FWD ? 1 : 0, store_fmt, chunk, phase == PH_REV ? ic_cells_ : 0, ns,
+                         guard_every > 0 ? 1 : 0, snap_.on() ? 1 + snap_.fmt : 0, skip ? 1 : 0, cached ? 1 : 0,
+                         d_ds_, L.tiles, L.slots};
+            r.ex = graph_for(key, L);
+            if (!r.ex) { set_error("hipGraph capture/instantiate failed"); return -11; }
+          }
+        }
+        busy = true;
+        if (r.ex && r.left >= chunk) {
+          HIPCHK(hipGraphLaunch(r.ex, L.st));
+          r.left -= chunk;
+        } else {
+          LaunchArgs a{d_ds_, L.tiles, (int)r.g->tiles.size(), 0};
+          a.act = skip ? L.act : nullptr;
+          a.cached = cached ? 1 : 0;
+          const int ns = (int)r.g->slots.size();
+          for (int k = 0; k < 8 && r.left > 0; k++, r.left--, r.step++) {
+            a.step = r.step;
+            const int e = step_launches(a, phase, tz, store_fmt, L, ns);
+            if (e) return e;
+            if (guard_every > 0 && ((r.step + 1) % guard_every == 0 || r.left == 1))
+              HIPCHK(rtm_launch_guard(d_ds_, L.slots, ns, r.step, d_flag_, L.st));
+          }
+        }
+        if (r.left == 0) r.g = nullptr;
+      }
+    }
+    return 0;
+  };
+  rc = body();
+  // the engine's stream goes on when every lane has ended (also after an
+  // error: nothing may still run when the slots are given back)
+  for (int l = 1; l < nl; l++) {
+    const hipError_t e1 = hipEventRecord(ev, lane_[l].st), e2 = hipStreamWaitEvent(st_, ev, 0);
+    if (rc == 0 && (e1 != hipSuccess || e2 != hipSuccess)) { set_error("lane join failed"); rc = -10; }
+  }
+  if (rc) for (auto& l : lane_) (void)hipStreamSynchronize(l.st);
+  (void)hipEventDestroy(ev);
+  return rc;
 }
 
 int Engine::guard_clear()
@@ -971,20 +1091,34 @@ void layout_runs(std::vector<Tile>& tiles, int phase)
 // neighbours of (z0, x0) are at z0 +- tz and x0 +- 64 in the same slot
 void link_neighbours(std::vector<Tile>& tiles, int tz)
 {
-  std::map<std::tuple<int, int, int>, int> at;
+  // table position of the tile at (z0, x0) of a slot: one grid per slot with
+  // a border of -1 (a map keyed by slot and origin took 20 ms for 200 shots)
+  struct Grid { int nz = 0, nx = 0; size_t at = 0; };
+  std::map<int, Grid> grids;
+  for (const Tile& t : tiles)
+    if (t.slot >= 0) {
+      Grid& g = grids[t.slot];
+      g.nz = std::max(g.nz, t.z0 / tz + 1);
+      g.nx = std::max(g.nx, t.x0 / RTM_TX + 1);
+    }
+  size_t n = 0;
+  int top = -1;
+  for (auto& kv : grids) { kv.second.at = n; n += (size_t)(kv.second.nz + 2) * (kv.second.nx + 2); top = kv.first; }
+  std::vector<const Grid*> by(top + 1, nullptr);
+  for (auto& kv : grids) by[kv.first] = &kv.second;
+  std::vector<int> pos(n, -1);
+  auto cell = [&](const Tile& t) {
+    const Grid& g = *by[t.slot];
+    return g.at + (size_t)(t.z0 / tz + 1) * (g.nx + 2) + t.x0 / RTM_TX + 1;
+  };
   for (int i = 0; i < (int)tiles.size(); i++)
-    if (tiles[i].slot >= 0) at[std::make_tuple(tiles[i].slot, tiles[i].z0, tiles[i].x0)] = i;
+    if (tiles[i].slot >= 0) pos[cell(tiles[i])] = i;
   for (Tile& t : tiles) {
-    int n = 0;
+    int k = 0;
     for (int dz = -1; dz <= 1; dz++)
       for (int dx = -1; dx <= 1; dx++) {
         if (dz == 0 && dx == 0) continue;
-        int k = -1;
-        if (t.slot >= 0) {
-          auto it = at.find(std::make_tuple(t.slot, t.z0 + dz * tz, t.x0 + dx * RTM_TX));
-          if (it != at.end()) k = it->second;
-        }
-        t.nbr[n++] = k;
+        t.nbr[k++] = t.slot < 0 ? -1 : pos[(long long)cell(t) + dz * (by[t.slot]->nx + 2) + dx];
       }
   }
 }
@@ -1113,16 +1247,25 @@ int Engine::ensure_cb(int nslots, size_t ntiles)
   cb_slots_ = nslots > cb_slots_ ? nslots : cb_slots_;
   if (cb_slots_ < 64) cb_slots_ = 64;
   cb_tiles_ = ntiles > cb_tiles_ ? ntiles * 2 : cb_tiles_;
-  const size_t bytes = align256(cb_slots_ * sizeof(ShotDev)) + align256(cb_tiles_ * sizeof(Tile)) +
-                       align256(cb_slots_ * 4) + align256(cb_slots_ * sizeof(StackShotHost)) + 256 +
-                       align256(2 * cb_tiles_ * sizeof(unsigned long long));
+  // descriptors | the batch's tile tables, slot lists, stack entries | guard
+  // flag | per lane: table, slot list, skip words
+  const size_t bt = align256(cb_tiles_ * sizeof(Tile)), bs = align256(cb_slots_ * 4),
+               ba = align256(2 * cb_tiles_ * sizeof(unsigned long long));
+  const size_t bytes = align256(cb_slots_ * sizeof(ShotDev)) + bt + bs + align256(cb_slots_ * sizeof(StackShotHost)) + 256 +
+                       kLanes * (bt + bs + ba);
   HIPCHK(hipMalloc(&cb_, bytes));
-  d_ds_ = (ShotDev*)cb_;
-  d_tiles_ = (Tile*)((char*)cb_ + align256(cb_slots_ * sizeof(ShotDev)));
-  d_slots_ = (int*)((char*)d_tiles_ + align256(cb_tiles_ * sizeof(Tile)));
-  d_stk_ = (StackShotHost*)((char*)d_slots_ + align256(cb_slots_ * 4));
-  d_flag_ = (unsigned int*)((char*)d_stk_ + align256(cb_slots_ * sizeof(StackShotHost)));
-  d_act_ = (unsigned long long*)((char*)d_flag_ + 256);
+  char* p = (char*)cb_;
+  auto take = [&](size_t n) { char* q = p; p += n; return q; };
+  d_ds_ = (ShotDev*)take(align256(cb_slots_ * sizeof(ShotDev)));
+  d_tiles_ = (Tile*)take(bt);
+  d_slots_ = (int*)take(bs);
+  d_stk_ = (StackShotHost*)take(align256(cb_slots_ * sizeof(StackShotHost)));
+  d_flag_ = (unsigned int*)take(256);
+  for (auto& l : lane_) {
+    l.tiles = (Tile*)take(bt);
+    l.slots = (int*)take(bs);
+    l.act = (unsigned long long*)take(ba);
+  }
   return 0;
 }
 
@@ -1305,60 +1448,91 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
       if (cr != tuned_.end()) tz_r = cr->second;
       else tune_r = can;
     }
-    std::vector<Tile> tiles, tcand[3];
-    size_t tcap = 0;
-    for (int c = 0; c < 3; c++) {
-      build_tiles(ds, cands[c], tcand[c]);
-      tcap = std::max(tcap, tcand[c].size());
-    }
-    build_tiles(ds, tz, tiles);
-    layout_runs(tiles, PH_FWD);
-    link_neighbours(tiles, tz);
-    // room for any height's padded table (runs at most 1.25 x the even share)
-    tcap = std::max(tcap, tiles.size()) * 5 / 4 + 16;
-    // the first 3 x kTuneSteps steps of a pass, kTuneSteps with each candidate
-    // height, timed with events; every candidate computes the same cells, so
-    // these are steps of the pass.  Returns the fastest height.
-    auto tune_pass = [&](int phase) -> int {
-      hipEvent_t te[4];
-      for (auto& e : te) HIPCHK(hipEventCreate(&e));
-      HIPCHK(hipEventRecord(te[0], st_));
-      for (int c = 0; c < 3; c++) {
-        HIPCHK(hipMemcpyAsync(d_tiles_, tcand[c].data(), tcand[c].size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
-        LaunchArgs a{d_ds_, d_tiles_, (int)tcand[c].size(), 0};
-        for (int s2 = 0; s2 < kTuneSteps; s2++) {
-          a.step = c * kTuneSteps + s2;
-          HIPCHK(rtm_launch_step(a, phase, cands[c], st_));
-          if (phase == PH_FWD) HIPCHK(rtm_launch_save(d_ds_, d_slots_, nb, a.step, opt.store_fmt, st_));
-          else if (ic_cells_) HIPCHK(rtm_launch_ic(d_ds_, d_slots_, nb, a.step, ic_cells_, st_));
-          if (snap_.on()) HIPCHK(rtm_launch_snap(d_ds_, d_slots_, nb, phase, a.step, snap_.fmt, st_));
-        }
-        HIPCHK(hipEventRecord(te[c + 1], st_));
+    // groups of shots for each pass (one group when every launch is timed by
+    // itself), and tables of any height for them (per-XCD runs are padded to
+    // at most 1.25 x the even share)
+    const bool prof = opt.profile && stats;
+    bool cached_f = false, cached_r = false;
+    auto plan = [&](int phase, bool& cached) {
+      std::vector<std::vector<int>> v;
+      if (prof) {
+        v.resize(1);
+        for (int j = 0; j < nb; j++) v[0].push_back(j);
+        cached = false;
+      } else {
+        v = plan_groups(ds, phase, cached);
       }
-      HIPCHK(rtm_launch_bump(d_ds_, d_slots_, nb, 3 * kTuneSteps, st_));
-      HIPCHK(hipEventSynchronize(te[3]));
+      std::vector<Group> g(v.size());
+      for (size_t i = 0; i < v.size(); i++) g[i].slots = v[i];
+      return g;
+    };
+    std::vector<Group> gf = plan(PH_FWD, cached_f), gr = plan(PH_REV, cached_r);
+    size_t tcap = 0;
+    {
+      std::vector<Tile> t;
+      build_tiles(ds, 16, t);
+      tcap = t.size() * 5 / 4 + 16 * std::max(gf.size(), gr.size());
+    }
+    // a group's table at height tz: its slots' tiles in per-XCD runs
+    auto tables = [&](std::vector<Group>& gs, int phase, int h) {
+      for (Group& g : gs) {
+        std::vector<ShotDev> sub;
+        for (int j : g.slots) sub.push_back(ds[j]);
+        build_tiles(sub, h, g.tiles, &g.slots);
+        layout_runs(g.tiles, phase);
+        if (phase == PH_FWD) link_neighbours(g.tiles, h);
+      }
+    };
+    // the first 3 x kTuneSteps steps of the groups that start a pass (as one
+    // launch, the load of the lanes together), kTuneSteps with each candidate
+    // height, timed with events after the height's first kWarmSteps; every
+    // candidate computes the same cells, so these are steps of the pass.
+    // Returns the fastest height.
+    auto tune_pass = [&](int phase, std::vector<Group>& gs, bool cached) -> int {
+      std::vector<int> sl;
+      for (size_t i = 0; i < gs.size() && i < (size_t)kLanes; i++) {
+        sl.insert(sl.end(), gs[i].slots.begin(), gs[i].slots.end());
+        gs[i].done = 3 * kTuneSteps;
+      }
+      std::vector<ShotDev> sub;
+      for (int j : sl) sub.push_back(ds[j]);
+      hipEvent_t te[6];
+      for (auto& e : te) HIPCHK(hipEventCreate(&e));
+      const Lane& L = lane_[0];
+      HIPCHK(hipMemcpyAsync(L.slots, sl.data(), sl.size() * 4, hipMemcpyHostToDevice, st_));
+      std::vector<Tile> tc[3];
+      for (int c = 0; c < 3; c++) {
+        build_tiles(sub, cands[c], tc[c], &sl);
+        layout_runs(tc[c], phase);
+        HIPCHK(hipMemcpyAsync(L.tiles, tc[c].data(), tc[c].size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
+        LaunchArgs a{d_ds_, L.tiles, (int)tc[c].size(), 0};
+        a.cached = cached ? 1 : 0;
+        for (int s2 = 0; s2 < kTuneSteps; s2++) {
+          if (s2 == kWarmSteps) HIPCHK(hipEventRecord(te[2 * c], st_));
+          a.step = c * kTuneSteps + s2;
+          const int e = step_launches(a, phase, cands[c], opt.store_fmt, L, (int)sl.size());
+          if (e) return e;
+        }
+        HIPCHK(hipEventRecord(te[2 * c + 1], st_));
+      }
+      HIPCHK(rtm_launch_bump(d_ds_, L.slots, (int)sl.size(), 3 * kTuneSteps, st_));
+      HIPCHK(hipEventSynchronize(te[5]));
       float best = 1e30f;
       int pick = cands[0];
       for (int c = 0; c < 3; c++) {
         float m = 0;
-        HIPCHK(hipEventElapsedTime(&m, te[c], te[c + 1]));
+        HIPCHK(hipEventElapsedTime(&m, te[2 * c], te[2 * c + 1]));
         if (m < best) { best = m; pick = cands[c]; }
       }
       for (auto& e : te) (void)hipEventDestroy(e);
       return pick;
     };
-    std::vector<int> slots(nb);
-    for (int j = 0; j < nb; j++) slots[j] = j;
     if (ensure_cb(nb, tcap) != 0) { for (void* p : mem) pool_.put(p); rc = -3; break; }
     ShotDev* d_ds = d_ds_;
-    Tile* d_tiles = d_tiles_;
-    int* d_slots = d_slots_;
     StackShotHost* d_stk = d_stk_;
     for (auto& u : uploads) HIPCHK(hipMemcpyAsync(u.first, u.second.data(), u.second.size(), hipMemcpyHostToDevice, st_));
     for (int j = 0; j < nb; j++) { ds[j].phase = PH_FWD; ds[j].it_off = 0; ds[j].it_dir = 1; }
     HIPCHK(hipMemcpyAsync(d_ds, ds.data(), nb * sizeof(ShotDev), hipMemcpyHostToDevice, st_));
-    HIPCHK(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
-    HIPCHK(hipMemcpyAsync(d_slots, slots.data(), nb * 4, hipMemcpyHostToDevice, st_));
     for (int j = 0; j < nb; j++) {
       HIPCHK(rtm_launch_phase_init(d_ds, j, PH_FWD, 512, st_));
       if (smooth)                                    // the factors of the shot's smoothed windows
@@ -1371,18 +1545,14 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     // ---- forward pass: propagation + record + boundary strips
     if (guard_clear() != 0) { for (void* p : mem) pool_.put(p); rc = -10; break; }
     HIPCHK(hipEventRecord(e0, st_));
-    int fwd_done = 0;
     if (tune) {
-      tz = tune_pass(PH_FWD);
+      tz = tune_pass(PH_FWD, gf, cached_f);
+      if (tz < 0) { for (void* p : mem) pool_.put(p); rc = tz; break; }
       tuned_[tkey] = tz;
-      fwd_done = 3 * kTuneSteps;
-      build_tiles(ds, tz, tiles);
-      layout_runs(tiles, PH_FWD);
-      link_neighbours(tiles, tz);
-      HIPCHK(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
     }
-    rc = run_pass(PH_FWD, nt - fwd_done, d_ds, d_tiles, (int)tiles.size(), slots, d_slots, tz, opt.store_fmt,
-                  opt.graph_chunk, (opt.profile && stats) ? stats : nullptr, guard_every, fwd_skip_ok(tz));
+    tables(gf, PH_FWD, tz);
+    rc = prof ? profile_pass(PH_FWD, nt, gf[0], tz, opt.store_fmt, stats, fwd_skip_ok(tz))
+              : run_pass(PH_FWD, nt, gf, tz, opt.store_fmt, opt.graph_chunk, cached_f, guard_every, fwd_skip_ok(tz));
     if (rc) { for (void* p : mem) pool_.put(p); break; }
     HIPCHK(hipEventRecord(e1, st_));
     HIPCHK(hipStreamSynchronize(st_));
@@ -1488,21 +1658,19 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     if (opt.verbose) printf("source wavefiled prepared over...\nBegin backward......\n");
     if (guard_clear() != 0) { for (void* p : mem) pool_.put(p); rc = -10; break; }
     HIPCHK(hipEventRecord(e1, st_));
-    int rev_done = 0;
     if (tune_r) {
-      tz_r = tune_pass(PH_REV);
+      tz_r = tune_pass(PH_REV, gr, cached_r);
+      if (tz_r < 0) { for (void* p : mem) pool_.put(p); rc = tz_r; break; }
       tuned_[rkey] = tz_r;
-      rev_done = 3 * kTuneSteps;
     }
-    build_tiles(ds, tz_r, tiles);
-    layout_runs(tiles, PH_REV);
-    HIPCHK(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
-    rc = run_pass(PH_REV, nt - 1 - rev_done, d_ds, d_tiles, (int)tiles.size(), slots, d_slots, tz_r, opt.store_fmt,
-                  opt.graph_chunk, (opt.profile && stats) ? stats : nullptr, guard_every);
+    tables(gr, PH_REV, tz_r);
+    rc = prof ? profile_pass(PH_REV, nt - 1, gr[0], tz_r, opt.store_fmt, stats, false)
+              : run_pass(PH_REV, nt - 1, gr, tz_r, opt.store_fmt, opt.graph_chunk, cached_r, guard_every, false);
     last_tz = tz;
     last_tz_r = tz_r;
     if (rc) { for (void* p : mem) pool_.put(p); break; }
-    HIPCHK(rtm_launch_image(d_ds, d_slots, nb, 0, st_));
+    // (the groups are consecutive shots, so d_slots_ lists the batch in order)
+    HIPCHK(rtm_launch_image(d_ds, prof ? lane_[0].slots : d_slots_, nb, 0, st_));
     HIPCHK(hipEventRecord(e2, st_));
     HIPCHK(hipStreamSynchronize(st_));
     if ((rc = guard_check(ds, shots, k0, "reverse")) != 0) { for (void* p : mem) pool_.put(p); break; }

@@ -173,6 +173,7 @@ struct GraphKey {
   int guard;                               // wavefield guard after the chunk
   int snap;                                // snapshot launches after every step: 0 off, else 1 + format
   int skip;                                // zero-tile skip of the step kernels
+  int cached;                              // field stores of the step kernels (LaunchArgs::cached)
   const void* shots;
   const void* tiles;
   const void* slots;
@@ -254,11 +255,33 @@ class Engine {
  private:
   int device_;
   hipStream_t st_ = nullptr;
+  // A pass runs its batch in groups of shots, two groups at a time on two
+  // streams (plan_groups).  Lane 0 is the engine's stream; each lane has its
+  // own tile table, slot list and skip words, which its groups use in turn,
+  // so that groups of one shape share a captured graph.
+  struct Lane {
+    hipStream_t st = nullptr;
+    Tile* tiles = nullptr;
+    int* slots = nullptr;
+    unsigned long long* act = nullptr;   // zero-tile skip words (2 x tiles)
+  };
+  static constexpr int kLanes = 2;
+  Lane lane_[kLanes];
+  std::vector<Tile> stage_tiles_;       // host copies of a pass's uploads (kept until the next pass)
+  std::vector<int> stage_slots_;
+  // the shots of one group: indices into the batch, its tile table, the steps
+  // it has taken (the autotuner's), its place in the uploaded tables
+  struct Group {
+    std::vector<int> slots;
+    std::vector<Tile> tiles;
+    int done = 0;
+    size_t tile0 = 0, slot0 = 0;
+  };
   DevPool pool_;
   std::map<GraphKey, hipGraphExec_t> graphs_;
   std::map<int, Model> models_;
   std::map<long long, int> tuned_;      // geometry class -> tile height
-  static constexpr int kTuneSteps = 12;
+  static constexpr int kTuneSteps = 12, kWarmSteps = 4;
   mutable std::mutex models_mu_;
   int next_model_ = 1;
   // persistent control block: captured graphs reference these addresses
@@ -270,24 +293,44 @@ class Engine {
   int* d_slots_ = nullptr;
   struct StackShotHost* d_stk_ = nullptr;
   unsigned int* d_flag_ = nullptr;      // wavefield guard of the running pass (largest |p| bits)
-  unsigned long long* d_act_ = nullptr; // zero-tile skip words of the running pass (2 x tiles)
   int ic_cells_ = 0;                    // the other imaging conditions of the running batch: interior cells (0: off)
   SnapPlan snap_;                       // snapshots of the running job
   int ensure_cb(int nslots, size_t ntiles);
 
-  // guard_every > 0: the wavefield guard after every guard_every steps (plain
-  // launches) or after every replayed chunk, and after the last step
-  int run_pass(int phase, int nsteps, const ShotDev* dshots, const Tile* dtiles, int ntiles,
-               const std::vector<int>& slots, const int* dslots, int tz, int store_fmt, int chunk,
-               rtmh_stats* prof, int guard_every = 0, bool skip = false);
+  // All steps of a pass on every group, the groups dealt to the lanes in
+  // turn.  guard_every > 0: the wavefield guard after every guard_every steps
+  // (plain launches) or after every replayed chunk, and after the last step.
+  int run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, int store_fmt, int chunk, bool cached,
+               int guard_every, bool skip);
+  // the same with every launch timed by its own events (one group, no graph)
+  int profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt, rtmh_stats* prof, bool skip);
+  // one step's launches of a lane's group
+  int step_launches(const LaunchArgs& a, int phase, int tz, int store_fmt, const Lane& L, int nslots);
   // clears the guard flag before a pass; after it, checks the flag and names
   // the shots whose wavefield is not finite (-7)
   int guard_clear();
   int guard_check(const std::vector<ShotDev>& ds, const std::vector<int>& shots, int k0, const char* pass);
-  hipGraphExec_t graph_for(const GraphKey& k, const ShotDev* dshots, const Tile* dtiles, const int* dslots,
-                           int nslots, int store_fmt);
+  hipGraphExec_t graph_for(const GraphKey& k, const Lane& L);
   void drop_graphs();
 };
+
+// Groups of consecutive slots that a pass steps together, and whether the
+// groups in flight (two at a time) fit the 256 MB Infinity Cache.  Two lanes
+// in turn fill each other's launch tails, and in the reverse pass a group's
+// fields stay in the cache from step to step: a reverse step works on
+// `live_bytes` of a slot, a group takes at most half of kCacheBytes of them,
+// groups are of about equal size and even in number, so that both lanes are
+// busy to the end.  A forward pass, and shots too large for that, run as two
+// halves: a forward launch of few shots is short while the wavefield is still
+// small and its fixed costs then weigh more than the cache gives.  Measured,
+// ms of the forward and the reverse pass as one group / two halves / cached
+// groups: 48 survey shots (nt 3000) 260, 555 / 222, - / 245, 437; 160 (nt
+// 1000) 174, 638 / 160, - / 201, 531; 16 ragged windows of 400-1600 columns
+// 38, 176 / 34, - / 50, 155; 4 shots of 2148 x 1124 (nt 1200) 52, 194 / 51,
+// 187 / 95, -.
+constexpr double kCacheBytes = 200e6;
+double live_bytes(const ShotDev& d, int phase);
+std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int phase, bool& cached);
 
 // tile table of a list of slot descriptors with the per-tile flags
 // (tiles carry the index of the descriptor in `ds` plus `slot_base`)

@@ -147,9 +147,10 @@ __device__ __forceinline__ float store_value(const ShotDev& s, float sc, float r
 
 // ------------------------------------------------------------ tile shape --
 // G waves of 64 lanes; each thread owns RPT consecutive rows of one column.
-template <int G_, int RPT_>
+template <int G_, int RPT_, bool CACHED>
 struct Geo {
   static constexpr int G = G_, RPT = RPT_;
+  static constexpr int ST = CACHED ? 0 : 2;            // cache policy of the field stores (bst)
   static constexpr int TZ = G * RPT;                   // tile rows
   static constexpr int NT = 64 * G;                    // threads
   static constexpr int PW = 108;                       // p row: column x at float x - x0 + 21 (x0-20..x0+83 held):
@@ -218,22 +219,28 @@ __device__ __forceinline__ float bld(rsrc_t r, int voff, int soff)
 {
   return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
 }
-// Field stores carry the non-temporal hint (cache-policy bit 1, "nt" on
-// gfx950): a value written in one step is next read in the following step,
-// after the whole batch (far more than the L2 and the Infinity Cache hold)
-// has streamed through the caches.  Measured +0.4-0.8 % on the 200-shot
-// survey (three alternations with the cached form on one device).
+// Cache policy ST of the field stores: 2 is the non-temporal hint ("nt" on
+// gfx950), 0 an ordinary store.  A value written in one step is next read in
+// the following step.  Where the launches in flight work on more than the
+// 256 MB Infinity Cache holds, it is gone by then, and the hint keeps the
+// stores from pushing out lines that neighbouring tiles still read; where
+// they work on less, an ordinary store leaves the value there for the next
+// step.  Survey shots, us per reverse step, nt against ordinary: 64 shots
+// (0.9 GB) 268 / 277, 32 shots 139 / 143, 16 shots (220 MB) 75 / 68, 8 shots
+// 44 / 36, 4 shots 26 / 23.  rtm_launch.h's `cached` says which.
+template <int ST>
 __device__ __forceinline__ void bst(rsrc_t r, float v, int voff, int soff)
 {
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, voff, soff, 2);
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, voff, soff, ST);
 }
 __device__ __forceinline__ f4 bld4(rsrc_t r, int voff, int soff)
 {
   return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
+template <int ST>
 __device__ __forceinline__ void bst4(rsrc_t r, f4 v, int voff, int soff)
 {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, 2);
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, ST);
 }
 // load one dword per lane into LDS: lane i writes lds_row[i] (lds_row is
 // wave-uniform)
@@ -578,7 +585,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     }
     if (k < KO) {                                      // own quads to memory
       const bool on = oq && (!GEN || (qx(k) < nxp && zw + qrow(k) < nzp));
-      bst4(field_rsrc(vxn, s), hv[k], pred_off(ooff, on), qsoff(k));
+      bst4<Q::ST>(field_rsrc(vxn, s), hv[k], pred_off(ooff, on), qsoff(k));
       if (oq)
 #pragma unroll
         for (int c = 0; c < 4; c++) nzb |= __float_as_uint(hv[k][c]);
@@ -709,7 +716,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     for (int r = 0; r < RPT; r++) {
       if (r % 2 == 0) part();
       const int iz = zw + r;
-      bst(Rvzn, cz[r + 10], GEN ? pred_off(vcol, ix < nxp && iz < nzp) : vcol, srow0 + (g * RPT + r) * pr4);
+      bst<Q::ST>(Rvzn, cz[r + 10], GEN ? pred_off(vcol, ix < nxp && iz < nzp) : vcol, srow0 + (g * RPT + r) * pr4);
       nzb |= __float_as_uint(cz[r + 10]);
       if (EDGE && !RCN) {
         int rad = RTM_R;
@@ -747,14 +754,14 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
         }
         if (!GEN) {
           const int oo = pred_off(o, on);
-          bst4(image_rsrc(s.g1, s), gi, oo, 0);
-          bst4(image_rsrc(s.illum, s), ii, oo, 0);
+          bst4<Q::ST>(image_rsrc(s.g1, s), gi, oo, 0);
+          bst4<Q::ST>(image_rsrc(s.illum, s), ii, oo, 0);
         } else {
 #pragma unroll
           for (int c = 0; c < 4; c++) {
             const int oc = pred_off(o + 4 * c, inner_row(z) && inner_col(x + c) && on);
-            bst(image_rsrc(s.g1, s), gi[c], oc, 0);
-            bst(image_rsrc(s.illum, s), ii[c], oc, 0);
+            bst<Q::ST>(image_rsrc(s.g1, s), gi[c], oc, 0);
+            bst<Q::ST>(image_rsrc(s.illum, s), ii[c], oc, 0);
           }
         }
       }
@@ -782,7 +789,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
             p[c] = __builtin_fmaf(-GCF(s.sa)[(z - s.sz0) * (s.sx1 - s.sx0 + 1) + x + c - s.sx0], wv, p[c]);
         }
       }
-      bst4(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+      bst4<Q::ST>(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
       continue;
     }
     f4 pu;
@@ -810,8 +817,8 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
           if (on) nzb |= __float_as_uint(q1[c]) | __float_as_uint(q2[c]);
         }
         const int o = pred_off(ooff, qsp[h] != 0 && on);
-        bst4(field_rsrc(s.q1, s), q1, o, qsoff(h));
-        bst4(field_rsrc(s.q2, s), q2, o, qsoff(h));
+        bst4<Q::ST>(field_rsrc(s.q1, s), q1, o, qsoff(h));
+        bst4<Q::ST>(field_rsrc(s.q2, s), q2, o, qsoff(h));
       }
     }
     if (FK == FK_SRC && (tl.kind & TF_SRC)) {          // kernel.cu:36-47
@@ -840,7 +847,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     if (on)
 #pragma unroll
       for (int c = 0; c < 4; c++) nzb |= __float_as_uint(p[c]);
-    bst4(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+    bst4<Q::ST>(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
   }
   if (FK == FK_SRC && actw) {
     const bool any = any_lane(nzb != 0u);
@@ -911,10 +918,10 @@ __device__ __forceinline__ int snap_index(const ShotDev& s, int k)
 
 // ================================================================ kernels ==
 // forward time step of the source wavefield (modelling, recording, strips)
-template <int G, int RPT>
+template <int G, int RPT, bool C>
 __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd(LaunchArgs a)
 {
-  using Q = Geo<G, RPT>;
+  using Q = Geo<G, RPT, C>;
   __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];   // coefficient table (reduced radii near the edges)
   const int t = xcd_tile(a.ntiles);
@@ -948,10 +955,10 @@ constexpr int RGRP = 16;
 // L2 from the other workgroup), so the two run at the same time; the last
 // step's products are added by k_image after the pass, those of a step whose
 // snapshot is restored by k_snap_load before it overwrites the field.
-template <int G, int RPT>
+template <int G, int RPT, bool C>
 __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_rev(LaunchArgs a)
 {
-  using Q = Geo<G, RPT>;
+  using Q = Geo<G, RPT, C>;
   __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];
   // XCD c's workgroups take its run of the table RGRP tiles at a time, their
@@ -1066,7 +1073,7 @@ __global__ __launch_bounds__(NTHR) void k_save(const ShotDev* __restrict__ shots
     for (int u = 0; u < SV; u++) v[u] = e0 + u * NTHR < blk.n ? strip_elem(s, blk, e0 + u * NTHR) : 0.0f;
 #pragma unroll
     for (int u = 0; u < SV; u++)
-      if (e0 + u * NTHR < blk.n) GF(s.store)[base + e0 + u * NTHR] = v[u];
+      if (e0 + u * NTHR < blk.n) __builtin_nontemporal_store(v[u], GF(s.store) + base + e0 + u * NTHR);
   }
 }
 
@@ -1785,9 +1792,14 @@ static inline int grid8(int ntiles) { return ((ntiles + 7) / 8) * 8; }
 template <int G, int RPT>
 static hipError_t launch_step_t(const LaunchArgs& a, int phase, hipStream_t st)
 {
-  const dim3 b(64 * G);
-  if (phase == PH_FWD) hipLaunchKernelGGL((k_fwd<G, RPT>), dim3(grid8(a.ntiles)), b, 0, st, a);
-  else hipLaunchKernelGGL((k_rev<G, RPT>), dim3(16 * (((a.ntiles + 7) / 8 + RGRP - 1) / RGRP * RGRP)), b, 0, st, a);
+  const dim3 b(64 * G), gf(grid8(a.ntiles)), gr(16 * (((a.ntiles + 7) / 8 + RGRP - 1) / RGRP * RGRP));
+  if (phase == PH_FWD) {
+    if (a.cached) hipLaunchKernelGGL((k_fwd<G, RPT, true>), gf, b, 0, st, a);
+    else hipLaunchKernelGGL((k_fwd<G, RPT, false>), gf, b, 0, st, a);
+  } else {
+    if (a.cached) hipLaunchKernelGGL((k_rev<G, RPT, true>), gr, b, 0, st, a);
+    else hipLaunchKernelGGL((k_rev<G, RPT, false>), gr, b, 0, st, a);
+  }
   return hipGetLastError();
 }
 
