@@ -54,6 +54,7 @@ enum RtmTileFlag : int {
   TF_REC = 4,     // the tile holds receiver cells
   TF_GEN = 8,     // the tile or its halo leaves the undamped interior (per-cell rules)
   TF_INT = 16,    // reverse phase: the tile holds reconstructed cells (interior or strips)
+  TF_SAVE = 64,   // the tile holds boundary-strip cells (kept by the forward step)
   TF_EDGE = 32,   // the tile or its halo holds cells of reduced radius (near the grid's edge)
 };
 
@@ -93,7 +94,7 @@ struct ShotDev {
   const int* cut;              // mute: samples it <= cut[ir] are zero
   // boundary store
   void* store;
-  float* sscale;               // nt x 4 scales (16-bit formats), then the wavefield guard word
+  float* sscale;               // nt x 4 scales (16-bit formats), then the wavefield guard word and the strips' max-abs
   long long strip_len;         // values per step
   int store_fmt, _pad4;
   // the other imaging conditions (null when off): ud du lr rl g4 (nzi x nxl
@@ -130,4 +131,7 @@ struct LaunchArgs {
   // 1: the launches in flight keep their fields in the Infinity Cache
   // (ordinary field stores; 0: stores with the non-temporal hint)
   int cached = 0;
+  // boundary strips of a forward step: 0 not kept, 1 fp32 (written by the
+  // step), 2 16-bit (the step takes the blocks' max-abs for k_quant16)
+  int save = 0;
 };

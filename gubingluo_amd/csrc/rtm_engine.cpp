@@ -767,11 +767,14 @@ void Engine::layout_slot(const rtmh_params& P, const ShotSetup& s, int store_fmt
 int Engine::step_launches(const LaunchArgs& a, int phase, int tz, int store_fmt, const Lane& L, int nslots)
 {
   HIPCHK(rtm_launch_step(a, phase, tz, L.st));
-  if (phase == PH_FWD) HIPCHK(rtm_launch_save(a.shots, L.slots, nslots, a.step, store_fmt, L.st));
-  else if (ic_cells_) HIPCHK(rtm_launch_ic(a.shots, L.slots, nslots, a.step, ic_cells_, L.st));
+  if (phase == PH_FWD && store_fmt != ST_F32) HIPCHK(rtm_launch_quant16(a.shots, L.slots, nslots, a.step, L.st));
+  if (phase == PH_REV && ic_cells_) HIPCHK(rtm_launch_ic(a.shots, L.slots, nslots, a.step, ic_cells_, L.st));
   if (snap_.on()) HIPCHK(rtm_launch_snap(a.shots, L.slots, nslots, phase, a.step, snap_.fmt, L.st));
   return 0;
 }
+
+// LaunchArgs::save of a store format
+static int strip_save(int fmt) { return fmt == ST_F32 ? 1 : 2; }
 
 hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
 {
@@ -782,6 +785,7 @@ hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
   LaunchArgs a{d_ds_, L.tiles, k.ntiles, 0};
   if (k.skip) a.act = L.act;
   a.cached = k.cached;
+  a.save = strip_save(k.fmt);
   for (int s = 0; s < k.k; s++) {
     a.step = s;
     (void)step_launches(a, k.phase, k.tz, k.fmt, L, k.nslots);
@@ -851,6 +855,7 @@ int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt,
   HIPCHK(hipMemcpyAsync(L.tiles, g.tiles.data(), ntiles * sizeof(Tile), hipMemcpyHostToDevice, st_));
   HIPCHK(hipMemcpyAsync(L.slots, g.slots.data(), nslots * sizeof(int), hipMemcpyHostToDevice, st_));
   LaunchArgs a{d_ds_, L.tiles, ntiles, 0};
+  a.save = strip_save(store_fmt);
   if (skip) {
     a.act = L.act;
     HIPCHK(hipMemsetAsync(a.act, 0xFF, 2 * (size_t)ntiles * sizeof(unsigned long long), st_));
@@ -863,8 +868,8 @@ int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt,
     HIPCHK(hipEventRecord(ev[0], st_));
     HIPCHK(rtm_launch_step(a, phase, tz, st_));
     HIPCHK(hipEventRecord(ev[1], st_));
-    if (phase == PH_FWD) HIPCHK(rtm_launch_save(d_ds_, L.slots, nslots, s, store_fmt, st_));
-    else if (ic_cells_) HIPCHK(rtm_launch_ic(d_ds_, L.slots, nslots, s, ic_cells_, st_));
+    if (phase == PH_FWD && store_fmt != ST_F32) HIPCHK(rtm_launch_quant16(d_ds_, L.slots, nslots, s, st_));
+    if (phase == PH_REV && ic_cells_) HIPCHK(rtm_launch_ic(d_ds_, L.slots, nslots, s, ic_cells_, st_));
     if (snap_.on()) HIPCHK(rtm_launch_snap(d_ds_, L.slots, nslots, phase, s, snap_.fmt, st_));
     HIPCHK(hipEventRecord(ev[2], st_));
     HIPCHK(hipEventSynchronize(ev[2]));
@@ -946,6 +951,7 @@ int Engine::run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, 
           LaunchArgs a{d_ds_, L.tiles, (int)r.g->tiles.size(), 0};
           a.act = skip ? L.act : nullptr;
           a.cached = cached ? 1 : 0;
+          a.save = strip_save(store_fmt);
           const int ns = (int)r.g->slots.size();
           for (int k = 0; k < 8 && r.left > 0; k++, r.left--, r.step++) {
             a.step = r.step;
@@ -1027,6 +1033,9 @@ void build_tiles(const std::vector<ShotDev>& ds, int tz, std::vector<Tile>& tile
           f |= TF_STRIP;
         if (d.sx1 >= d.sx0 && hit(0, 0, d.sz0, d.sz1, d.sx0, d.sx1)) f |= TF_SRC;
         if (d.nrec > 0 && hit(0, 0, n, n, d.rcol0, d.rcol0 + d.nrec - 1)) f |= TF_REC;
+        if (hit(0, 0, n, nzp - n - 1, n - R, n - 1) || hit(0, 0, n, nzp - n - 1, nxp - n - 1, nxp - n + R - 1) ||
+            hit(0, 0, n - R, n - 1, n, nxp - n - 1) || hit(0, 0, nzp - n - 1, nzp - n + R - 1, n, nxp - n - 1))
+          f |= TF_SAVE;
         // undamped full-radius interior for every velocity the step computes
         // (vx columns x0-10..x0+73, vz rows z0-10..z0+tz+8)
         const bool inside = x0 - 10 >= n && x1 + 10 <= nxp - n - 2 && z0 - 10 >= n && z1 + 9 <= nzp - n - 2;
@@ -1507,6 +1516,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
         HIPCHK(hipMemcpyAsync(L.tiles, tc[c].data(), tc[c].size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
         LaunchArgs a{d_ds_, L.tiles, (int)tc[c].size(), 0};
         a.cached = cached ? 1 : 0;
+        a.save = strip_save(opt.store_fmt);
         for (int s2 = 0; s2 < kTuneSteps; s2++) {
           if (s2 == kWarmSteps) HIPCHK(hipEventRecord(te[2 * c], st_));
           a.step = c * kTuneSteps + s2;

@@ -128,6 +128,12 @@ __device__ __forceinline__ int strip_row_ptb(const ShotDev& s, int iz)
   if (iz >= r0 && iz < r0 + RTM_R) return b + RTM_R * s.nxl + (iz - r0) * s.nxl;
   return -1;
 }
+// after the nt x 4 scales: the wavefield guard word (k_guard), then the
+// largest |value| of the four strip blocks (16-bit store) of even and of odd
+// steps, as float bits
+__device__ __forceinline__ unsigned int* guard_word(const ShotDev& s) { return (unsigned int*)(s.sscale + (size_t)s.nt * 4); }
+__device__ __forceinline__ unsigned int* strip_max(const ShotDev& s, int it) { return guard_word(s) + 4 + 4 * (it & 1); }
+
 // A stored strip value is fetched with the other operands of its phase (raw:
 // the fp32 value, or the 16-bit code in the low bits) and decoded where it is
 // used, with the scale of its block (0 vx, 1 vz, 2 p-lr, 3 p-tb) and step.
@@ -329,10 +335,17 @@ enum : int { TC_IN = 0, TC_GEN = 1, TC_EDGE = 2 };
 // The rows of the new vx are written and read by the same wave, so only the
 // new vz crosses waves (one exchange), and the z-differences reach the quads
 // through the wave's own vx rows once those are consumed.
+// A forward step keeps its own boundary strips (`save`): 1 writes them to the
+// fp32 store from the registers that hold them, 2 takes the largest |value| of
+// each 16-bit block for k_quant16, which scales and stores them.  Only tiles
+// that hold strip cells (TF_SAVE) have the code run.  A launch of its own that
+// read the strips back from the new fields cost 2.4 us a step on a 480 x 280
+// shot (11.6 -> 9.1 us), 15.7 us on three survey shots in turn (43.9 ->
+// 28.1), 3.7 of 79 us on 48 of them.
 template <class Q, int FK, int TC>
 __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* __restrict__ ctab, const ShotDev& s,
                                           const Tile& tl, int it, const float* pc, const float* vxc, const float* vzc,
-                                          float* pn, float* vxn, float* vzn, const float* pr, bool img,
+                                          float* pn, float* vxn, float* vzn, const float* pr, bool img, int save_,
                                           unsigned char* actw)
 {
   constexpr int G = Q::G, RPT = Q::RPT, TZ = Q::TZ, KZ = Q::KZ, PW = Q::PW, VXW = Q::VXW, ZR = Q::ZR;
@@ -351,6 +364,12 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   const int ix = x0 + lane;                            // the lane's column (column mapping)
   const int zw = z0 + g * RPT;                         // the wave's first own row
   const bool strips = RCN && GEN && (tl.kind & TF_STRIP) != 0;
+  const int save = FK == FK_SRC && GEN && (tl.kind & TF_SAVE) ? save_ : 0;
+  float smax[4] = {0.0f, 0.0f, 0.0f, 0.0f};            // (save 2) largest |value| of the strip blocks
+  auto put = [&](int b, int off, float v) {
+    if (save == 1) __builtin_nontemporal_store(v, GF(s.store) + (long long)it * s.strip_len + off);
+    else smax[b] = fmaxf(smax[b], fabsf(v));
+  };
   const int pr4 = s.pitch * 4;
   const int srow0 = (z0 + RTM_MZT) * pr4;              // byte offset of tile row 0
   const int vcol = (ix + RTM_MXL) * 4;                 // byte offset of the lane's column
@@ -589,6 +608,16 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       if (oq)
 #pragma unroll
         for (int c = 0; c < 4; c++) nzb |= __float_as_uint(hv[k][c]);
+      if (save) {
+        const int x = qx(k);
+        const bool near = (x + 3 >= npml - RTM_R && x < npml) || (x + 3 >= nxp - npml - 1 && x < nxp - npml + RTM_R - 1);
+        if (oq && near)
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const int st = strip_vx(s, zw + qrow(k), x + c);
+            if (st >= 0) put(0, st, hv[k][c]);
+          }
+      }
     }
   }
   part();
@@ -718,6 +747,10 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       const int iz = zw + r;
       bst<Q::ST>(Rvzn, cz[r + 10], GEN ? pred_off(vcol, ix < nxp && iz < nzp) : vcol, srow0 + (g * RPT + r) * pr4);
       nzb |= __float_as_uint(cz[r + 10]);
+      if (save) {
+        const int st = strip_row_vz(s, iz);            // wave-uniform
+        if (st >= 0 && zcol) put(1, st + ix - npml, cz[r + 10]);
+      }
       if (EDGE && !RCN) {
         int rad = RTM_R;
         if (iz > 0 && iz < nzp - 1 && ix > 0 && ix < nxp - 1)
@@ -847,7 +880,28 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     if (on)
 #pragma unroll
       for (int c = 0; c < 4; c++) nzb |= __float_as_uint(p[c]);
+    if (save && on) {
+      const int lr = strip_row_lr(s, z), tb = strip_row_ptb(s, z);
+      const bool near = (x + 3 >= npml - RTM_R && x < npml) || (x + 3 >= nxp - npml && x < nxp - npml + RTM_R);
+      if ((lr >= 0 && near) || tb >= 0)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const int pl = lr >= 0 ? strip_col_plr(s, x + c) : -1;
+          if (pl >= 0) put(2, lr + pl, p[c]);
+          else if (tb >= 0 && inner_col(x + c)) put(3, tb + x + c - npml, p[c]);
+        }
+    }
     bst4<Q::ST>(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+  }
+  if (save == 2) {
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+      if (!any_lane(smax[b] > 0.0f)) continue;
+      float m = smax[b];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+      if (lane == 0) atomicMax(strip_max(s, it) + b, __float_as_uint(m));
+    }
   }
   if (FK == FK_SRC && actw) {
     const bool any = any_lane(nzb != 0u);
@@ -863,15 +917,16 @@ template <class Q, int FK>
 __device__ __forceinline__ void field_step(float* __restrict__ lds, float* __restrict__ ctab, const ShotDev& s,
                                            const Tile& tl, int it, const float* pc, const float* vxc,
                                            const float* vzc, float* pn, float* vxn, float* vzn,
-                                           const float* pr = nullptr, bool img = false, unsigned char* actw = nullptr)
+                                           const float* pr = nullptr, bool img = false, int save = 0,
+                                           unsigned char* actw = nullptr)
 {
   if (!(tl.kind & TF_GEN)) {
-    tile_step<Q, FK, TC_IN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
+    tile_step<Q, FK, TC_IN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, save, actw);
   } else if (FK == FK_RCN || !(tl.kind & TF_EDGE)) {
-    tile_step<Q, FK, TC_GEN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
+    tile_step<Q, FK, TC_GEN>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, save, actw);
   } else {
     for (int t = threadIdx.x; t < RTM_R * CTW; t += Q::NT) ctab[t] = ctab_entry(s, t);   // read after the first barrier
-    tile_step<Q, FK, TC_EDGE>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, actw);
+    tile_step<Q, FK, TC_EDGE>(lds, ctab, s, tl, it, pc, vxc, vzc, pn, vxn, vzn, pr, img, save, actw);
   }
 }
 
@@ -906,6 +961,23 @@ __device__ __forceinline__ bool skip_of(const SkipWords& w, int it)
   return (in | out) == 0ull;
 }
 
+// the strip values of a tile that skips its step: all +0
+template <class Q>
+__device__ __forceinline__ void save_zeros(const ShotDev& s, const Tile& tl, int it)
+{
+  gfloat* rec = GF(s.store) + (long long)it * s.strip_len;
+  for (int e = threadIdx.x; e < 64 * Q::TZ; e += Q::NT) {
+    const int z = tl.z0 + (e >> 6), x = tl.x0 + (e & 63);
+    const bool in = x >= s.npml && x < s.nxp - s.npml;
+    const int vx = strip_vx(s, z, x), vz = strip_row_vz(s, z), lr = strip_row_lr(s, z), tb = strip_row_ptb(s, z);
+    const int pl = lr >= 0 ? strip_col_plr(s, x) : -1;
+    if (vx >= 0) rec[vx] = 0.0f;
+    if (vz >= 0 && in) rec[vz + x - s.npml] = 0.0f;
+    if (pl >= 0) rec[lr + pl] = 0.0f;
+    else if (tb >= 0 && in) rec[tb + x - s.npml] = 0.0f;
+  }
+}
+
 // index of the snapshot of step k (below: decimated snapshots), -1 if none
 __device__ __forceinline__ int snap_index(const ShotDev& s, int k)
 {
@@ -933,12 +1005,15 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) 
   if (track) sw = skip_words(a.act, a.ntiles, t, tl);
   const ShotDev& s = shot_of(a.shots, tl.slot);
   const int it = s.it_off + s.it_dir * a.step;
-  if (track && skip_of(sw, it)) return;                // the forward field is +0 around the tile
+  if (track && skip_of(sw, it)) {                      // the forward field is +0 around the tile
+    if (a.save == 1 && (tl.kind & TF_SAVE)) save_zeros<Q>(s, tl, it);
+    return;
+  }
   const bool odd = it & 1;                             // (a runtime index into s would spill it to scratch)
   unsigned char* actw = a.act ? (unsigned char*)(a.act + (size_t)((it + 1) & 1) * a.ntiles + t) : nullptr;
   field_step<Q, FK_SRC>(lds, ctab, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
                         odd ? s.svz[1] : s.svz[0], odd ? s.sp[0] : s.sp[1], odd ? s.svx[0] : s.svx[1],
-                        odd ? s.svz[0] : s.svz[1], nullptr, false, actw);
+                        odd ? s.svz[0] : s.svz[1], nullptr, false, a.save, actw);
 }
 
 // tiles whose receiver halves, then reconstruction halves, follow each other
@@ -1007,11 +1082,12 @@ __global__ __launch_bounds__(NTHR) void k_image(const ShotDev* __restrict__ shot
   }
 }
 
-// Boundary strips of forward step `it` -- the new fields of that step -- into
+// Boundary strips of forward step `it` -- the new fields of that step -- in
 // the store, packed as kernel.cu:1186-1293 per step:
 //   vx lr [2][nzi][10] | vz tb [2][10][nxl] | p lr [2][nzi][10] | p tb [2][10][nxl]
-// fp32 is a copy (k_save); the 16-bit forms store each block with a scale of
-// its own (k_save16).
+// The step kernel writes the fp32 ones itself; the 16-bit forms store each
+// block with a scale of its own, known only once every tile has stepped
+// (k_quant16).
 struct StripBlock {
   const float* f;    // field (cell (0,0)), new level
   int lr;            // 1: [2][nzi][10] column strips, 0: [2][10][nxl] row strips
@@ -1038,108 +1114,58 @@ __device__ __forceinline__ float strip_elem(const ShotDev& s, const StripBlock& 
   if (k.lr) {                                          // e = (side*nzi + r)*10 + c
     const int q = e / RTM_R, c = e - q * RTM_R;
     const int side = q >= s.nzi, r = q - side * s.nzi;
-    return k.f[(size_t)(s.npml + r) * s.pitch + (side ? k.a1 : k.a0) + c];
+    return GCF(k.f)[(size_t)(s.npml + r) * s.pitch + (side ? k.a1 : k.a0) + c];
   }
   const int q = e / s.nxl, c = e - q * s.nxl;          // e = (side*10 + r)*nxl + c
   const int side = q >= RTM_R, r = q - side * RTM_R;
-  return k.f[(size_t)((side ? k.a1 : k.a0) + r) * s.pitch + s.npml + c];
+  return GCF(k.f)[(size_t)((side ? k.a1 : k.a0) + r) * s.pitch + s.npml + c];
 }
-// A step's strip record is small (2*40(nz+nxl) values per shot), so a save
-// is latency-bound: every thread keeps SV loads in flight, and each block is
-// split over gridDim.y workgroups with lane-contiguous elements (every load
-// and store of a wave covers 64 consecutive values of the record).
-constexpr int SV = 8;
-__device__ __forceinline__ int save_it(const ShotDev& s, int step)
-{
-  return step < 0 ? -step - 1 : s.it_off + s.it_dir * step;   // step < 0: absolute -step-1
-}
-// the wavefield guard word (k_guard) after the nt x 4 scales
-__device__ __forceinline__ unsigned int* guard_word(const ShotDev& s) { return (unsigned int*)(s.sscale + (size_t)s.nt * 4); }
 
-// fp32: copy block b of the slot's step into the store
-__global__ __launch_bounds__(NTHR) void k_save(const ShotDev* __restrict__ shots, const int* __restrict__ slots,
-                                                int nslots, int step)
+// 16-bit store of step `step`'s strips: block b of a slot with the scale
+// max(maxabs / 32768, FLT_MIN) (1 for an all-zero block; a denormal max-abs,
+// e.g. source tails before the wave arrives, must not underflow the scale to
+// zero: |x| <= 32768 * FLT_MIN then anyway), x / scale rounded to nearest
+// even.  The step's tiles have left the block's max-abs (strip_max), so a
+// block is spread over gridDim.y workgroups, SV loads in flight a thread, and
+// the words of the next step are cleared here.  Latency-bound: one workgroup
+// of 1024 threads per block, which also took the max-abs, needed 18.7 us a
+// step on 4 slots of 2148 x 1124 (16 workgroups on 256 CUs).
+constexpr int SV = 4;
+__global__ __launch_bounds__(NTHR) void k_quant16(const ShotDev* __restrict__ shots, const int* __restrict__ slots,
+                                                   int nslots, int step)
 {
   const int k = blockIdx.x >> 2, b = blockIdx.x & 3;
   if (k >= nslots) return;
-  const ShotDev s = shots[slots[k]];
-  const int it = save_it(s, step);
+  const ShotDev& s = shot_of(shots, slots[k]);
+  const int it = s.it_off + s.it_dir * step;
   const StripBlock blk = strip_block_of(s, b, (it + 1) & 1);
   const long long base = (long long)it * s.strip_len + blk.lo;
+  const float m = __uint_as_float(strip_max(s, it)[b]);
+  const float sc = m > 0.0f ? fmaxf(m * (1.0f / 32768.0f), 1.17549435e-38f) : 1.0f;
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
+    s.sscale[(long long)it * 4 + b] = sc;
+    strip_max(s, it + 1)[b] = 0u;
+  }
   const int stride = gridDim.y * NTHR * SV;
   for (int e0 = blockIdx.y * NTHR * SV + threadIdx.x; e0 < blk.n; e0 += stride) {
     float v[SV];
 #pragma unroll
     for (int u = 0; u < SV; u++) v[u] = e0 + u * NTHR < blk.n ? strip_elem(s, blk, e0 + u * NTHR) : 0.0f;
 #pragma unroll
-    for (int u = 0; u < SV; u++)
-      if (e0 + u * NTHR < blk.n) __builtin_nontemporal_store(v[u], GF(s.store) + base + e0 + u * NTHR);
-  }
-}
-
-// 16-bit forms: one workgroup of SQT threads per (slot, block) takes the
-// block's max-abs, keeps the scale max(maxabs / 32768, FLT_MIN) (1 for an
-// all-zero block; a denormal max-abs, e.g. source tails before the wave
-// arrives, must not underflow the scale to zero: |x| <= 32768 * FLT_MIN then
-// anyway) and stores x / scale rounded to nearest even.  Blocks of up to
-// SQV x SQT values stay in registers between the two steps (a block holds
-// 20 x nxl or 20 x nz values: windows up to 2457 cells wide and deep); a
-// larger one is read twice.  (Against a max-abs launch with an
-// atomic per workgroup followed by a quantising launch: 20.2 against 22.5 us
-// per step on 16 precision slots, one launch fewer.)
-constexpr int SQT = 1024, SQV = 48;
-__global__ __launch_bounds__(SQT) void k_save16(const ShotDev* __restrict__ shots, const int* __restrict__ slots,
-                                                 int nslots, int step)
-{
-  __shared__ float red[SQT / 64];
-  const int k = blockIdx.x >> 2, b = blockIdx.x & 3;
-  if (k >= nslots) return;
-  const ShotDev s = shots[slots[k]];
-  const int it = save_it(s, step);
-  const StripBlock blk = strip_block_of(s, b, (it + 1) & 1);
-  const long long base = (long long)it * s.strip_len + blk.lo;
-  const int tid = threadIdx.x;
-  const bool held = blk.n <= SQV * SQT;               // block-uniform
-  float v[SQV];
-  float m = 0.0f;
-  if (held) {
-#pragma unroll
-    for (int u = 0; u < SQV; u++) {
-      const int e = tid + u * SQT;
-      v[u] = e < blk.n ? strip_elem(s, blk, e) : 0.0f;
+    for (int u = 0; u < SV; u++) {
+      const int e = e0 + u * NTHR;
+      if (e >= blk.n) continue;
+      const float q = v[u] / sc;
+      unsigned short h;
+      if (s.store_fmt == ST_F16) {
+        h = __half_as_ushort(__float2half_rn(q));
+      } else {
+        unsigned int w = __float_as_uint(q);           // bf16, round to nearest even
+        w += 0x7FFFu + ((w >> 16) & 1u);
+        h = (unsigned short)(w >> 16);
+      }
+      __builtin_nontemporal_store(h, (gushort*)s.store + base + e);
     }
-#pragma unroll
-    for (int u = 0; u < SQV; u++) m = fmaxf(m, fabsf(v[u]));
-  } else {
-    for (int e = tid; e < blk.n; e += SQT) m = fmaxf(m, fabsf(strip_elem(s, blk, e)));
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((tid & 63) == 0) red[tid >> 6] = m;
-  __syncthreads();
-  m = red[0];
-#pragma unroll
-  for (int w = 1; w < SQT / 64; w++) m = fmaxf(m, red[w]);
-  const float sc = m > 0.0f ? fmaxf(m * (1.0f / 32768.0f), 1.17549435e-38f) : 1.0f;
-  if (tid == 0) s.sscale[(long long)it * 4 + b] = sc;
-  auto put = [&](int e, float x) {
-    const float q = x / sc;
-    if (s.store_fmt == ST_F16) {
-      ((__half*)s.store)[base + e] = __float2half_rn(q);
-    } else {
-      unsigned int w = __float_as_uint(q);             // bf16, round to nearest even
-      w += 0x7FFFu + ((w >> 16) & 1u);
-      ((unsigned short*)s.store)[base + e] = (unsigned short)(w >> 16);
-    }
-  };
-  if (held) {
-#pragma unroll
-    for (int u = 0; u < SQV; u++) {
-      const int e = tid + u * SQT;
-      if (e < blk.n) put(e, v[u]);
-    }
-  } else {
-    for (int e = tid; e < blk.n; e += SQT) put(e, strip_elem(s, blk, e));
   }
 }
 
@@ -1515,7 +1541,7 @@ __global__ __launch_bounds__(NTHR) void k_phase_init(const ShotDev* __restrict__
     for (int k = 0; k < 14; k++)
       if (k >= first) (f[k] - s.forg)[e] = 0.0f;
   if (phase == PH_FWD) {
-    if (g0 == 0) guard_word(s)[0] = 0u;
+    if (g0 < 12) guard_word(s)[g0] = 0u;               // ... and the strips' max-abs words
     if (s.snap)
       for (long long e = g0; e < 3LL * s.nsnap; e += gs) snap_acc(s)[e] = 0u;   // snapshot max-abs words
   } else {
@@ -1829,17 +1855,13 @@ hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, 
   return hipGetLastError();
 }
 
-hipError_t rtm_launch_save(const ShotDev* shots, const int* slots, int nslots, int step, int store_fmt,
-                           hipStream_t st)
+hipError_t rtm_launch_quant16(const ShotDev* shots, const int* slots, int nslots, int step, hipStream_t st)
 {
   if (nslots <= 0) return hipSuccess;
-  // blocks of up to 2*10*nz values: 4 workgroups each (fp32); the 16-bit
-  // passes use 8 (they run on the few-shot launches of the served form too)
-  if (store_fmt == ST_F32) {
-    hipLaunchKernelGGL(k_save, dim3(4 * nslots, 4), dim3(NTHR), 0, st, shots, slots, nslots, step);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(k_save16, dim3(4 * nslots), dim3(SQT), 0, st, shots, slots, nslots, step);
+  // about 1024 workgroups in all, at most 32 per block (a block of the widest
+  // windows holds 41 K values)
+  hipLaunchKernelGGL(k_quant16, dim3(4 * nslots, std::min(32, std::max(4, 256 / nslots))), dim3(NTHR), 0, st, shots,
+                     slots, nslots, step);
   return hipGetLastError();
 }
 
