@@ -131,7 +131,8 @@ struct LaunchArgs {
   // 1: the launches in flight keep their fields in the Infinity Cache
   // (ordinary field stores; 0: stores with the non-temporal hint)
   int cached = 0;
-  // boundary strips of a forward step: 0 not kept, 1 fp32 (written by the
-  // step), 2 16-bit (the step takes the blocks' max-abs for k_quant16)
+  // 1: a forward step keeps its boundary strips (fp32: writes them; 16-bit:
+  // takes the blocks' max-abs for k_quant16)
   int save = 0;
+  int s16 = 0;   // the slots' boundary store is 16-bit
 };

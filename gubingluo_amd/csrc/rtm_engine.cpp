@@ -773,8 +773,8 @@ int Engine::step_launches(const LaunchArgs& a, int phase, int tz, int store_fmt,
   return 0;
 }
 
-// LaunchArgs::save of a store format
-static int strip_save(int fmt) { return fmt == ST_F32 ? 1 : 2; }
+// a step that keeps its boundary strips in store format fmt
+static void keep_strips(LaunchArgs& a, int fmt) { a.save = 1; a.s16 = fmt != ST_F32; }
 
 hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
 {
@@ -785,7 +785,7 @@ hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
   LaunchArgs a{d_ds_, L.tiles, k.ntiles, 0};
   if (k.skip) a.act = L.act;
   a.cached = k.cached;
-  a.save = strip_save(k.fmt);
+  keep_strips(a, k.fmt);
   for (int s = 0; s < k.k; s++) {
     a.step = s;
     (void)step_launches(a, k.phase, k.tz, k.fmt, L, k.nslots);
@@ -855,7 +855,7 @@ int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt,
   HIPCHK(hipMemcpyAsync(L.tiles, g.tiles.data(), ntiles * sizeof(Tile), hipMemcpyHostToDevice, st_));
   HIPCHK(hipMemcpyAsync(L.slots, g.slots.data(), nslots * sizeof(int), hipMemcpyHostToDevice, st_));
   LaunchArgs a{d_ds_, L.tiles, ntiles, 0};
-  a.save = strip_save(store_fmt);
+  keep_strips(a, store_fmt);
   if (skip) {
     a.act = L.act;
     HIPCHK(hipMemsetAsync(a.act, 0xFF, 2 * (size_t)ntiles * sizeof(unsigned long long), st_));
@@ -951,7 +951,7 @@ int Engine::run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, 
           LaunchArgs a{d_ds_, L.tiles, (int)r.g->tiles.size(), 0};
           a.act = skip ? L.act : nullptr;
           a.cached = cached ? 1 : 0;
-          a.save = strip_save(store_fmt);
+          keep_strips(a, store_fmt);
           const int ns = (int)r.g->slots.size();
           for (int k = 0; k < 8 && r.left > 0; k++, r.left--, r.step++) {
             a.step = r.step;
@@ -1516,7 +1516,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
         HIPCHK(hipMemcpyAsync(L.tiles, tc[c].data(), tc[c].size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
         LaunchArgs a{d_ds_, L.tiles, (int)tc[c].size(), 0};
         a.cached = cached ? 1 : 0;
-        a.save = strip_save(opt.store_fmt);
+        keep_strips(a, opt.store_fmt);
         for (int s2 = 0; s2 < kTuneSteps; s2++) {
           if (s2 == kWarmSteps) HIPCHK(hipEventRecord(te[2 * c], st_));
           a.step = c * kTuneSteps + s2;

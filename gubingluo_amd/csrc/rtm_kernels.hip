@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "rtm_dev.h"
 
@@ -134,28 +135,12 @@ __device__ __forceinline__ int strip_row_ptb(const ShotDev& s, int iz)
 __device__ __forceinline__ unsigned int* guard_word(const ShotDev& s) { return (unsigned int*)(s.sscale + (size_t)s.nt * 4); }
 __device__ __forceinline__ unsigned int* strip_max(const ShotDev& s, int it) { return guard_word(s) + 4 + 4 * (it & 1); }
 
-// A stored strip value is fetched with the other operands of its phase (raw:
-// the fp32 value, or the 16-bit code in the low bits) and decoded where it is
-// used, with the scale of its block (0 vx, 1 vz, 2 p-lr, 3 p-tb) and step.
-__device__ __forceinline__ float store_raw(const ShotDev& s, int it, int off)
-{
-  const long long k = (long long)it * s.strip_len + off;
-  if (s.store_fmt == ST_F32) return GCF(s.store)[k];
-  return __uint_as_float((unsigned int)((const gushort*)s.store)[k]);
-}
-__device__ __forceinline__ float store_value(const ShotDev& s, float sc, float raw)
-{
-  if (s.store_fmt == ST_F32) return raw;
-  const unsigned int h = __float_as_uint(raw);
-  if (s.store_fmt == ST_F16) return __half2float(__ushort_as_half((unsigned short)h)) * sc;
-  return __uint_as_float(h << 16) * sc;
-}
-
 // ------------------------------------------------------------ tile shape --
 // G waves of 64 lanes; each thread owns RPT consecutive rows of one column.
-template <int G_, int RPT_, bool CACHED>
+template <int G_, int RPT_, bool CACHED, bool S16_>
 struct Geo {
   static constexpr int G = G_, RPT = RPT_;
+  static constexpr bool S16 = S16_;                    // the boundary store is 16-bit
   static constexpr int ST = CACHED ? 0 : 2;            // cache policy of the field stores (bst)
   static constexpr int TZ = G * RPT;                   // tile rows
   static constexpr int NT = 64 * G;                    // threads
@@ -216,7 +201,7 @@ __device__ __forceinline__ int model_col(const ShotDev& s, int ix)
 #define RTM_OOB ((int)0x80000000)
 __device__ __forceinline__ int col_load(int voff, int col, int nxp)
 {
-  return (col >= 0 && col < nxp) ? voff : (voff | RTM_OOB);
+  return (unsigned)col < (unsigned)nxp ? voff : (voff | RTM_OOB);
 }
 // a lane's offset, or the out-of-range one where the lane takes no part:
 // its load returns 0 and its store is dropped, with no exec-mask branch
@@ -248,6 +233,42 @@ __device__ __forceinline__ void bst4(rsrc_t r, f4 v, int voff, int soff)
 {
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, voff, soff, ST);
 }
+// The boundary strips of step `it` as a buffer.  It starts 16 bytes before the
+// record and ends 16 after it (both inside the slot): a quad that holds the
+// first or last columns of a strip loads four values at the strip's own
+// offsets, of which the ones past the strip are not used.
+template <bool S16>
+__device__ __forceinline__ rsrc_t strip_rsrc(const ShotDev& s, int it)
+{
+  constexpr int es = S16 ? 2 : 4;
+  return __builtin_amdgcn_make_buffer_rsrc((char*)s.store + (long long)it * s.strip_len * es - 16, (short)0,
+                                           (int)s.strip_len * es + 32, 0x00020000);
+}
+// raw stored values (the fp32 value, or the 16-bit code in the low bits) at
+// offset off (a row offset row and a lane's col), and the value of one with
+// the scale of its block and step
+template <bool S16>
+__device__ __forceinline__ float strip1(rsrc_t r, int col, int row, bool on)
+{
+  if (!S16) return bld(r, pred_off(col * 4 + 16, on), row * 4);
+  return __uint_as_float((unsigned int)__builtin_amdgcn_raw_buffer_load_b16(r, pred_off(col * 2 + 16, on), row * 2, 0));
+}
+template <bool S16>
+__device__ __forceinline__ f4 strip4(rsrc_t r, int off, bool on)
+{
+  if (!S16) return bld4(r, pred_off(off * 4 + 16, on), 0);
+  return f4{strip1<S16>(r, off, 0, on), strip1<S16>(r, off + 1, 0, on), strip1<S16>(r, off + 2, 0, on),
+            strip1<S16>(r, off + 3, 0, on)};
+}
+template <bool S16>
+__device__ __forceinline__ float strip_value(const ShotDev& s, float sc, float raw)
+{
+  if (!S16) return raw;
+  const unsigned int h = __float_as_uint(raw);
+  const float f = __half2float(__ushort_as_half((unsigned short)h)), b = __uint_as_float(h << 16);
+  return (s.store_fmt == ST_F16 ? f : b) * sc;
+}
+
 // load one dword per lane into LDS: lane i writes lds_row[i] (lds_row is
 // wave-uniform)
 typedef __attribute__((address_space(3))) void lds_void_t;
@@ -335,9 +356,9 @@ enum : int { TC_IN = 0, TC_GEN = 1, TC_EDGE = 2 };
 // The rows of the new vx are written and read by the same wave, so only the
 // new vz crosses waves (one exchange), and the z-differences reach the quads
 // through the wave's own vx rows once those are consumed.
-// A forward step keeps its own boundary strips (`save`): 1 writes them to the
-// fp32 store from the registers that hold them, 2 takes the largest |value| of
-// each 16-bit block for k_quant16, which scales and stores them.  Only tiles
+// A forward step keeps its own boundary strips (`save`): it writes them to the
+// fp32 store from the registers that hold them, or takes the largest |value|
+// of each 16-bit block for k_quant16, which scales and stores them.  Only tiles
 // that hold strip cells (TF_SAVE) have the code run.  A launch of its own that
 // read the strips back from the new fields cost 2.4 us a step on a 480 x 280
 // shot (11.6 -> 9.1 us), 15.7 us on three survey shots in turn (43.9 ->
@@ -345,11 +366,12 @@ enum : int { TC_IN = 0, TC_GEN = 1, TC_EDGE = 2 };
 template <class Q, int FK, int TC>
 __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* __restrict__ ctab, const ShotDev& s,
                                           const Tile& tl, int it, const float* pc, const float* vxc, const float* vzc,
-                                          float* pn, float* vxn, float* vzn, const float* pr, bool img, int save_,
+                                          float* pn, float* vxn, float* vzn, const float* pr, bool img, bool save_,
                                           unsigned char* actw)
 {
   constexpr int G = Q::G, RPT = Q::RPT, TZ = Q::TZ, KZ = Q::KZ, PW = Q::PW, VXW = Q::VXW, ZR = Q::ZR;
   constexpr int KQ = Q::KQ, KO = Q::KO;
+  constexpr bool S16 = Q::S16;
   constexpr bool RCN = FK == FK_RCN, GEN = TC != TC_IN, EDGE = TC == TC_EDGE;
   // the OR of the bit patterns of the lane's stored field values (-0 counts
   // as non-zero): written to actw[wave] at the end for the zero-tile skip
@@ -364,11 +386,12 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   const int ix = x0 + lane;                            // the lane's column (column mapping)
   const int zw = z0 + g * RPT;                         // the wave's first own row
   const bool strips = RCN && GEN && (tl.kind & TF_STRIP) != 0;
-  const int save = FK == FK_SRC && GEN && (tl.kind & TF_SAVE) ? save_ : 0;
-  float smax[4] = {0.0f, 0.0f, 0.0f, 0.0f};            // (save 2) largest |value| of the strip blocks
-  auto put = [&](int b, int off, float v) {
-    if (save == 1) __builtin_nontemporal_store(v, GF(s.store) + (long long)it * s.strip_len + off);
-    else smax[b] = fmaxf(smax[b], fabsf(v));
+  const bool save = FK == FK_SRC && GEN && save_ && (tl.kind & TF_SAVE);
+  float smax[4] = {0.0f, 0.0f, 0.0f, 0.0f};            // (16-bit store) largest |value| of the strip blocks
+  // a strip value of block b at offset off, where `on`: no branch per lane
+  auto put = [&](rsrc_t r, int b, int off, float v, bool on) {
+    if (!S16) bst<2>(r, v, pred_off(off * 4 + 16, on), 0);
+    else smax[b] = fmaxf(smax[b], on ? fabsf(v) : 0.0f);
   };
   const int pr4 = s.pitch * 4;
   const int srow0 = (z0 + RTM_MZT) * pr4;              // byte offset of tile row 0
@@ -377,8 +400,25 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   const rsrc_t Rp = field_rsrc(pc, s), Rvx = field_rsrc(vxc, s), Rvz = field_rsrc(vzc, s);
   const rsrc_t Rib = model_rsrc(s.mib, s), Rkk = model_rsrc(s.mkk, s);
   const float dtx = s.dtx, dtz = s.dtz;
-  auto inner_row = [&](int z) { return z >= npml && z < nzp - npml; };
-  auto inner_col = [&](int x) { return x >= npml && x < nxp - npml; };
+  // (per-lane conditions are combined with & and |: a short-circuit operator
+  // would branch on the lanes)
+  auto inner_row = [&](int z) { return (unsigned)(z - npml) < (unsigned)(nzp - 2 * npml); };
+  auto inner_col = [&](int x) { return (unsigned)(x - npml) < (unsigned)(nxp - 2 * npml); };
+  // the strips' columns beside the interior: vx and p left, vx right, p right
+  // (kernel.cu:1186-1293), and whether the tile's own and halo quads reach them
+  auto left = [&](int x) { return (unsigned)(x - npml + RTM_R) < (unsigned)RTM_R; };
+  auto rightv = [&](int x) { return (unsigned)(x - nxp + npml + 1) < (unsigned)RTM_R; };
+  auto rightp = [&](int x) { return (unsigned)(x - nxp + npml) < (unsigned)RTM_R; };
+  const bool hasL = x0 - 12 < npml && x0 + 75 >= npml - RTM_R;
+  const bool hasR = x0 - 12 < nxp - npml + RTM_R && x0 + 75 >= nxp - npml - 1;
+  const int blr = 2 * RTM_R * (s.nzi + s.nxl);         // the p lr block
+  // rows of the wave that hold cells of this pass (a partial last tile row,
+  // the absorbing rows beyond the reconstruction's strips)
+  const bool live = !GEN || (RCN ? zw + RPT > npml - RTM_R && zw < nzp - npml + RTM_R : zw < nzp);
+  // columns near the left or right edge; columns that no window edge clamps
+  const bool edge_x = EDGE && (x0 - 12 <= 9 || x0 + 75 >= nxp - 10);
+  const bool mfree = !GEN || (x0 - 12 >= s.mxs && x0 + 76 <= s.mxs + s.mxn);
+  const bool inner_cols = !GEN || (x0 >= npml && x0 + 64 <= nxp - npml);
   float c10[RTM_R];
 #pragma unroll
   for (int i = 0; i < RTM_R; i++) c10[i] = CCF(s.coef)[90 + i];
@@ -412,7 +452,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   // rows of the z phase that exist for every wave need no test
   auto zrow = [&](int k) { return k < ZR - (G - 1) * KZ || g * KZ + k < ZR; };
   const int mcol = model_col(s, ix);
-  const bool zcol = ix >= npml && ix < nxp - npml;     // interior columns
+  const bool zcol = inner_col(ix);                     // interior columns
   float vzo[KZ], ibz[KZ];
 #pragma unroll
   for (int k = 0; k < KZ; k++) {
@@ -420,12 +460,10 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     vzo[k] = 0.0f;
     ibz[k] = 1.0f;
     if (zrow(k)) {
-      // a strip row of the reconstruction: the stored value of step it+1 (raw)
-      const int st = strips ? strip_row_vz(s, iz) : -1;
-      if (st >= 0) {
-        if (zcol) vzo[k] = store_raw(s, it + 1, st + ix - npml);
-      } else {
-        vzo[k] = bld(Rvz, vld, srow0 + (kz - 10) * pr4);
+      vzo[k] = bld(Rvz, vld, srow0 + (kz - 10) * pr4);
+      if (strips) {                                    // a strip row: the stored value of step it+1 (raw)
+        const int st = strip_row_vz(s, iz);
+        if (st >= 0) vzo[k] = strip1<S16>(strip_rsrc<S16>(s, it + 1), ix - npml, st, zcol);
       }
       ibz[k] = bld(Rib, mcol, GEN ? model_row(s, iz) : (iz - s.mz0) * s.mpitch * 4);
     }
@@ -449,8 +487,8 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   auto qx = [&](int k) { return x0 + qcol(k); };       // first column of a quad
   auto qsoff = [&](int k) { return k < KO ? 4 * k * pr4 : 0; };
   // load offset of a quad: quads off the grid's columns fetch nothing
-  const int old_ = GEN ? pred_off(ooff, x0 + ocol >= 0 && x0 + ocol < nxp) : ooff;
-  const int xld_ = GEN ? pred_off(xoff, x0 + xcol >= 0 && x0 + xcol < nxp) : xoff;
+  const int old_ = GEN ? pred_off(ooff, (unsigned)(x0 + ocol) < (unsigned)nxp) : ooff;
+  const int xld_ = GEN ? pred_off(xoff, (unsigned)(x0 + xcol) < (unsigned)nxp) : xoff;
   auto qld = [&](int k) { return k < KO ? old_ : xld_; };
   if (!RCN && GEN) {                                   // vx damping of the columns x0-12..x0+75
     for (int t = threadIdx.x; t < 22; t += 64 * G) {
@@ -469,35 +507,36 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       return bld4(r, o, k < KO ? 16 * k * s.mpitch : 0);
     }
     const int ro = model_row(s, zw + qrow(k)), x = qx(k);
+    if (mfree) return bld4(r, ro + (s.mx0 + x - s.mxs) * 4, 0);
     return f4{bld(r, ro + model_col(s, x), 0), bld(r, ro + model_col(s, x + 1), 0), bld(r, ro + model_col(s, x + 2), 0),
               bld(r, ro + model_col(s, x + 3), 0)};
   };
-  f4 vxo[KQ], ibx[KQ];
-#pragma unroll
-  for (int k = 0; k < KQ; k++) {
-    vxo[k] = bld4(Rvx, qld(k), qsoff(k));
-    ibx[k] = model4(Rib, k);
-  }
-  // reconstruction: block scales of the 16-bit store (1 for fp32: unused)
-  float scv[4] = {1.0f, 1.0f, 1.0f, 1.0f};             // vx, vz of step it+1, p-lr, p-tb of step it
-  if (strips && s.store_fmt != ST_F32) {
-#pragma unroll
-    for (int b = 0; b < 4; b++) scv[b] = CCF(s.sscale)[(long long)(b < 2 ? it + 1 : it) * 4 + b];
-  }
-  // vx strip cells of a quad (reconstruction): raw stored values and a mask
-  f4 sxr[KQ];
-  int sxm[KQ];
-  if (strips) {
+  f4 vxo[KQ], ibx[KQ], sxr[KQ];                        // (sxr: stored vx of a quad's strip cells, raw)
+  float scv[4] = {1.0f, 1.0f, 1.0f, 1.0f};             // 16-bit block scales: vx, vz of step it+1, p-lr, p-tb of step it
+  if (live) {
 #pragma unroll
     for (int k = 0; k < KQ; k++) {
-      sxm[k] = 0;
-      sxr[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      vxo[k] = bld4(Rvx, qld(k), qsoff(k));
+      ibx[k] = model4(Rib, k);
+    }
+    if (strips) {
+      if (S16)
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int st = strip_vx(s, zw + qrow(k), qx(k) + c);
-        if (st >= 0) {
-          sxr[k][c] = store_raw(s, it + 1, st);
-          sxm[k] |= 1 << c;
+        for (int b = 0; b < 4; b++) scv[b] = CCF(s.sscale)[(long long)(b < 2 ? it + 1 : it) * 4 + b];
+      const rsrc_t R = strip_rsrc<S16>(s, it + 1);
+#pragma unroll
+      for (int k = 0; k < KQ; k++) {
+        const int x = qx(k), r = zw + qrow(k) - npml;
+        const bool in = inner_row(zw + qrow(k));
+        sxr[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (hasL) sxr[k] = strip4<S16>(R, r * RTM_R + x - npml + RTM_R, in & (x + 3 >= npml - RTM_R) & (x < npml));
+        if (hasR) {
+          const f4 u = strip4<S16>(R, RTM_R * s.nzi + r * RTM_R + x - nxp + npml + 1,
+                              in & (x + 3 >= nxp - npml - 1) & (x < nxp - npml - 1 + RTM_R));
+          if (!hasL) sxr[k] = u;
+          else                                         // a window narrower than the tile
+#pragma unroll
+            for (int c = 0; c < 4; c++) sxr[k][c] = rightv(x + c) ? u[c] : sxr[k][c];
         }
       }
     }
@@ -513,6 +552,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   //         Reconstruction: v + u as fma(s*dt/h, ib, v) (kernel.cu:318-388),
   //         stored strip values (kernel.cu:1294-1347), 0 elsewhere
   float vzn_[KZ];
+  const float scz = S16 && strips ? CCF(s.sscale)[(long long)(it + 1) * 4 + 1] : 1.0f;
   {
     float cw[KZ + 19];                                 // p rows z0-19 + g KZ + m of the column
 #pragma unroll
@@ -526,16 +566,16 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
         if (RCN) {
           if (!GEN) {
             vzn_[k] = __builtin_fmaf(taps(cw, k + 9, c10) * dtz, ibz[k], vzo[k]);
-          } else if (strips && strip_row_vz(s, iz) >= 0) {
-            vzn_[k] = zcol ? store_value(s, scv[1], vzo[k]) : 0.0f;
-          } else if (iz >= npml && iz <= nzp - npml - 2) {
+          } else {
+            // every row is computed and then selected, with no branch
             const float v = __builtin_fmaf(taps(cw, k + 9, c10) * dtz, ibz[k], vzo[k]);
-            vzn_[k] = zcol ? v : 0.0f;
+            vzn_[k] = zcol & (iz >= npml) & (iz <= nzp - npml - 2) ? v : 0.0f;
+            if (strips) vzn_[k] = zcol & (strip_row_vz(s, iz) >= 0) ? strip_value<S16>(s, scz, vzo[k]) : vzn_[k];
           }
-        } else {
+        } else if (!EDGE || (iz >= 0 && iz <= nzp - 2)) {   // (rows off the grid stay +0)
           float sum;
           if (EDGE) {
-            const int rad = iz >= 0 && iz <= nzp - 2 ? imin(RTM_R, imin(iz + 1, nzp - 1 - iz)) : RTM_R;
+            const int rad = imin(RTM_R, imin(iz + 1, nzp - 1 - iz));
             sum = rad == RTM_R ? taps(cw, k + 9, c10) : taps_r(cw, k + 9, ctab, rad);
           } else {
             sum = taps(cw, k + 9, c10);
@@ -551,6 +591,12 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   // ---- 3. new vx of the own and the halo quads; the quad's own pressure is
   //         in its window
   f4 hv[KQ], po[KO];
+  if (live) {
+  if (S16 && strips)
+#pragma unroll
+    for (int k = 0; k < KQ; k++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) sxr[k][c] = strip_value<S16>(s, scv[0], sxr[k][c]);
 #pragma unroll
   for (int k = 0; k < KQ; k++) {
     part();
@@ -569,12 +615,12 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     }
     int rad[4] = {RTM_R, RTM_R, RTM_R, RTM_R};
     bool red = false;
-    if (EDGE && !RCN) {
+    if (edge_x && !RCN) {
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const int x = qx(k) + c;
-        if (x >= 0 && x <= nxp - 2) rad[c] = imin(RTM_R, imin(x + 1, nxp - 1 - x));
-        red = red || rad[c] != RTM_R;
+        if ((unsigned)x <= (unsigned)(nxp - 2)) rad[c] = imin(RTM_R, imin(x + 1, nxp - 1 - x));
+        red = red | (rad[c] != RTM_R);
       }
       red = any_lane(red);
     }
@@ -587,8 +633,9 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
         float v = __builtin_fmaf(sum * dtx, ibx[k][c], vxo[k][c]);
         if (GEN) {
           const int x = qx(k) + c;
-          v = inner_row(zw + qrow(k)) && x >= npml && x <= nxp - npml - 2 ? v : 0.0f;
-          if (strips) v = (sxm[k] >> c) & 1 ? store_value(s, scv[0], sxr[k][c]) : v;
+          const bool in = inner_row(zw + qrow(k));
+          v = in & (x >= npml) & (x <= nxp - npml - 2) ? v : 0.0f;
+          if (strips) v = in & (left(x) | rightv(x)) ? sxr[k][c] : v;
         }
         hv[k][c] = v;
       } else {
@@ -603,81 +650,82 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       hv[k][c] = v;
     }
     if (k < KO) {                                      // own quads to memory
-      const bool on = oq && (!GEN || (qx(k) < nxp && zw + qrow(k) < nzp));
+      const bool on = oq & (!GEN | ((qx(k) < nxp) & (zw + qrow(k) < nzp)));
       bst4<Q::ST>(field_rsrc(vxn, s), hv[k], pred_off(ooff, on), qsoff(k));
       if (oq)
 #pragma unroll
         for (int c = 0; c < 4; c++) nzb |= __float_as_uint(hv[k][c]);
       if (save) {
-        const int x = qx(k);
-        const bool near = (x + 3 >= npml - RTM_R && x < npml) || (x + 3 >= nxp - npml - 1 && x < nxp - npml + RTM_R - 1);
-        if (oq && near)
+        const rsrc_t R = strip_rsrc<S16>(s, it);
+        const int x = qx(k), r = zw + qrow(k) - npml;
+        const bool in = oq & inner_row(zw + qrow(k));
+        if (hasL)
 #pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const int st = strip_vx(s, zw + qrow(k), x + c);
-            if (st >= 0) put(0, st, hv[k][c]);
-          }
+          for (int c = 0; c < 4; c++) put(R, 0, r * RTM_R + x + c - npml + RTM_R, hv[k][c], in & left(x + c));
+        if (hasR)
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            put(R, 0, RTM_R * s.nzi + r * RTM_R + x + c - nxp + npml + 1, hv[k][c], in & rightv(x + c));
       }
     }
+  }
   }
   part();
   // operands of the pressure phase, fetched now so that the round trip
   // overlaps the exchange and the differences below: rho v^2 of the own quads, and the PML split pair
   // (forward-type passes, quads with a damped cell) or, in the
   // reconstruction, the imaging accumulators and the receiver pressure
-  f4 kk[KO], qa[KO], qb[KO], qc[KO];
-  int qsp[KO];                                         // split cells of a quad / strip cells (bits 0-3 lr, 4-7 tb)
+  f4 kk[KO], qa[KO], qb[KO], qc[KO], spr[KO];          // (spr: stored p of a quad's strip cells, raw)
+  // split cells: the absorbing layer within the ring
+  auto split = [&](int z, int x) {
+    return ((unsigned)(z - 1) < (unsigned)(nzp - 2)) & ((unsigned)(x - 1) < (unsigned)(nxp - 2)) &
+           !(inner_row(z) & inner_col(x));
+  };
+  auto split_q = [&](int z, int x) { return oq & (split(z, x) | split(z, x + 1) | split(z, x + 2) | split(z, x + 3)); };
+  if (live) {
 #pragma unroll
-  for (int h = 0; h < KO; h++) {
-    const int z = zw + qrow(h), x = qx(h);
-    kk[h] = model4(Rkk, h);
-    qsp[h] = 0;
-    qa[h] = qb[h] = qc[h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (!RCN && GEN) {
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const bool on = z > 0 && z < nzp - 1 && x + c > 0 && x + c < nxp - 1 && !(inner_row(z) && inner_col(x + c));
-        qsp[h] |= on ? 1 << c : 0;
-      }
-      if (any_lane(qsp[h] != 0 && oq)) {
-        const int o = pred_off(ooff, qsp[h] != 0 && oq);
+    for (int h = 0; h < KO; h++) {
+      const int z = zw + qrow(h), x = qx(h);
+      kk[h] = model4(Rkk, h);
+      qa[h] = qb[h] = qc[h] = spr[h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (!RCN && GEN && any_lane(split_q(z, x))) {
+        const int o = pred_off(ooff, split_q(z, x));
         qa[h] = bld4(field_rsrc(s.q1, s), o, qsoff(h));
         qb[h] = bld4(field_rsrc(s.q2, s), o, qsoff(h));
       }
-    }
-    if (RCN) {
-      if (img) {
+      if (RCN && img) {
         qc[h] = bld4(field_rsrc(pr, s), old_, qsoff(h));
         const int o = ((z - npml) * s.nxl + x - npml) * 4;
-        if (!GEN) {
-          qa[h] = bld4(image_rsrc(s.g1, s), o, 0);
-          qb[h] = bld4(image_rsrc(s.illum, s), o, 0);
+        if (inner_cols) {
+          const int oo = GEN ? pred_off(o, inner_row(z)) : o;
+          qa[h] = bld4(image_rsrc(s.g1, s), oo, 0);
+          qb[h] = bld4(image_rsrc(s.illum, s), oo, 0);
         } else {
 #pragma unroll
           for (int c = 0; c < 4; c++) {
-            const int oc = pred_off(o + 4 * c, inner_row(z) && inner_col(x + c) && oq);
+            const int oc = pred_off(o + 4 * c, inner_row(z) & inner_col(x + c) & oq);
             qa[h][c] = bld(image_rsrc(s.g1, s), oc, 0);
             qb[h][c] = bld(image_rsrc(s.illum, s), oc, 0);
           }
         }
       }
-    }
-  }
-  // stored p of the strip cells of an own quad (reconstruction)
-  f4 spr[KO];
-  if (strips) {
+      if (strips) {
+        const rsrc_t R = strip_rsrc<S16>(s, it);
+        const int r = (z - npml) * RTM_R, tb = strip_row_ptb(s, z);
+        const bool in = inner_row(z);
+        if (hasL) spr[h] = strip4<S16>(R, blr + r + x - npml + RTM_R, in & (x + 3 >= npml - RTM_R) & (x < npml));
+        if (hasR) {
+          const f4 u = strip4<S16>(R, blr + RTM_R * s.nzi + r + x - nxp + npml,
+                              in & (x + 3 >= nxp - npml) & (x < nxp - npml + RTM_R));
+          if (!hasL) spr[h] = u;
+          else
 #pragma unroll
-    for (int h = 0; h < KO; h++) {
-      const int z = zw + qrow(h), x = qx(h);
-      const int lr = strip_row_lr(s, z), tb = strip_row_ptb(s, z);
-      spr[h] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int c = 0; c < 4; c++) spr[h][c] = rightp(x + c) ? u[c] : spr[h][c];
+        }
+        if (any_lane(tb >= 0)) {
+          const f4 u = strip4<S16>(R, tb + x - npml, (tb >= 0) & (x + 3 >= npml) & (x < nxp - npml));
 #pragma unroll
-      for (int c = 0; c < 4; c++) {
-        const int pl = lr >= 0 ? strip_col_plr(s, x + c) : -1;
-        const int st = pl >= 0 ? lr + pl : (tb >= 0 && inner_col(x + c) ? tb + x + c - npml : -1);
-        if (st >= 0) {
-          spr[h][c] = store_raw(s, it, st);
-          qsp[h] |= pl >= 0 ? 1 << c : 16 << c;
+          for (int c = 0; c < 4; c++) spr[h][c] = tb >= 0 ? u[c] : spr[h][c];
         }
       }
     }
@@ -687,6 +735,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
 #pragma unroll
   for (int k = 0; k < KZ; k++)
     if (zrow(k)) VZL[(g * KZ + k) * 64 + lane] = vzn_[k];
+  if (live)
 #pragma unroll
   for (int k = 0; k < KQ; k++)
     if ((k < KO && oq) || ((k >= KO || RPT < 4) && hon)) {
@@ -701,6 +750,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   //         through the wave's vx rows.  Radius of a cell: min(10, distance
   //         to the nearest grid edge); cells off the grid or on its ring are
   //         computed with radius 10 and dropped
+  if (live) {
   f4 dx_[KO], dz_[KO];
 #pragma unroll
   for (int h = 0; h < KO; h++) {
@@ -718,9 +768,9 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const int x = qx(h) + c, z = zw + qrow(h);
-        if (z > 0 && z < nzp - 1 && x > 0 && x < nxp - 1)
+        if (((unsigned)(z - 1) < (unsigned)(nzp - 2)) & ((unsigned)(x - 1) < (unsigned)(nxp - 2)))
           rad[c] = imin(imin(RTM_R, imin(x, nxp - 1 - x)), imin(z, nzp - 1 - z));
-        red = red || rad[c] != RTM_R;
+        red = red | (rad[c] != RTM_R);
       }
       red = any_lane(red);
     }
@@ -745,11 +795,11 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     for (int r = 0; r < RPT; r++) {
       if (r % 2 == 0) part();
       const int iz = zw + r;
-      bst<Q::ST>(Rvzn, cz[r + 10], GEN ? pred_off(vcol, ix < nxp && iz < nzp) : vcol, srow0 + (g * RPT + r) * pr4);
+      bst<Q::ST>(Rvzn, cz[r + 10], GEN ? pred_off(vcol, (ix < nxp) & (iz < nzp)) : vcol, srow0 + (g * RPT + r) * pr4);
       nzb |= __float_as_uint(cz[r + 10]);
       if (save) {
         const int st = strip_row_vz(s, iz);            // wave-uniform
-        if (st >= 0 && zcol) put(1, st + ix - npml, cz[r + 10]);
+        if (st >= 0) put(strip_rsrc<S16>(s, it), 1, st + ix - npml, cz[r + 10], zcol);
       }
       if (EDGE && !RCN) {
         int rad = RTM_R;
@@ -770,6 +820,10 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
 
   // ---- 5. new pressure of the own quads
   const rsrc_t Rpn = field_rsrc(pn, s);
+  auto strip_p = [&](int z, int x) {
+    const bool in = inner_row(z);
+    return strips && ((in & (left(x) | rightp(x))) | (!in & (strip_row_ptb(s, z) >= 0) & inner_col(x)));
+  };
 #pragma unroll
   for (int h = 0; h < KO; h++) {
     part();
@@ -785,31 +839,31 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
           gi[c] = __builtin_fmaf(po[h][c], qc[h][c], qa[h][c]);
           ii[c] = __builtin_fmaf(po[h][c], po[h][c], qb[h][c]);
         }
-        if (!GEN) {
-          const int oo = pred_off(o, on);
+        if (inner_cols) {
+          const int oo = pred_off(o, on & (!GEN | inner_row(z)));
           bst4<Q::ST>(image_rsrc(s.g1, s), gi, oo, 0);
           bst4<Q::ST>(image_rsrc(s.illum, s), ii, oo, 0);
         } else {
 #pragma unroll
           for (int c = 0; c < 4; c++) {
-            const int oc = pred_off(o + 4 * c, inner_row(z) && inner_col(x + c) && on);
+            const int oc = pred_off(o + 4 * c, inner_row(z) & inner_col(x + c) & on);
             bst<Q::ST>(image_rsrc(s.g1, s), gi[c], oc, 0);
             bst<Q::ST>(image_rsrc(s.illum, s), ii[c], oc, 0);
           }
         }
       }
+      if (S16 && strips)
+#pragma unroll
+        for (int c = 0; c < 4; c++) spr[h][c] = strip_value<S16>(s, inner_row(z) ? scv[2] : scv[3], spr[h][c]);
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         const float sum = __builtin_fmaf(dx_[h][c], dtx, dz_[h][c] * dtz);
         float v = __builtin_fmaf(kk[h][c], sum, po[h][c]);   // kernel.cu:389-429
         bool wr = true;
         if (GEN) {
-          wr = inner_row(z) && inner_col(x + c);
-          if (strips && (qsp[h] >> c) & 17) {
-            v = store_value(s, (qsp[h] >> c) & 1 ? scv[2] : scv[3], spr[h][c]);   // kernel.cu:1348-1400
-            wr = true;
-          }
+          wr = inner_row(z) & inner_col(x + c);
           v = wr ? v : 0.0f;                           // cells the reconstruction does not hold
+          v = strip_p(z, x + c) ? spr[h][c] : v;       // kernel.cu:1348-1400
         }
         p[c] = v;
       }
@@ -817,12 +871,12 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
         const float wv = CCF(s.wav)[it];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-          const bool wr = !GEN || (inner_row(z) && inner_col(x + c)) || (strips && ((qsp[h] >> c) & 17));
+          const bool wr = !GEN | (inner_row(z) & inner_col(x + c)) | strip_p(z, x + c);
           if (wr && on && z >= s.sz0 && z <= s.sz1 && x + c >= s.sx0 && x + c <= s.sx1)
             p[c] = __builtin_fmaf(-GCF(s.sa)[(z - s.sz0) * (s.sx1 - s.sx0 + 1) + x + c - s.sx0], wv, p[c]);
         }
       }
-      bst4<Q::ST>(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+      bst4<Q::ST>(Rpn, p, pred_off(ooff, on & (!GEN | ((x < nxp) & (z < nzp)))), qsoff(h));
       continue;
     }
     f4 pu;
@@ -834,8 +888,8 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     } else {
       // the outer ring and the cells off the grid keep their value
 #pragma unroll
-      for (int c = 0; c < 4; c++) p[c] = inner_row(z) && inner_col(x + c) ? pu[c] : po[h][c];
-      if (any_lane(qsp[h] != 0 && on)) {               // split pair, p = p1 + p2 (kernel.cu:774-783)
+      for (int c = 0; c < 4; c++) p[c] = inner_row(z) & inner_col(x + c) ? pu[c] : po[h][c];
+      if (any_lane(split_q(z, x))) {                   // split pair, p = p1 + p2 (kernel.cu:774-783)
         const f4 ax = *(const gf4*)(GCF(s.ax) + x);
         const f4 bx = *(const gf4*)(GCF(s.bx) + x);
         const float az = GCF(s.az)[z], bz = GCF(s.bz)[z];
@@ -843,13 +897,13 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
 #pragma unroll
         for (int c = 0; c < 4; c++) {
           const float dxv = (dx_[h][c] * dtx) * kk[h][c], dzv = (dz_[h][c] * dtz) * kk[h][c];
-          const bool sp = (qsp[h] >> c) & 1;
+          const bool sp = split(z, x + c);
           q1[c] = sp ? __builtin_fmaf(ax[c], qa[h][c], -(dxv * bx[c])) : qa[h][c];   // (c1 q - d)/c2
           q2[c] = sp ? __builtin_fmaf(az, qb[h][c], -(dzv * bz)) : qb[h][c];
-          if (sp) p[c] = q1[c] + q2[c];
+          p[c] = sp ? q1[c] + q2[c] : p[c];
           if (on) nzb |= __float_as_uint(q1[c]) | __float_as_uint(q2[c]);
         }
-        const int o = pred_off(ooff, qsp[h] != 0 && on);
+        const int o = pred_off(ooff, split_q(z, x));
         bst4<Q::ST>(field_rsrc(s.q1, s), q1, o, qsoff(h));
         bst4<Q::ST>(field_rsrc(s.q2, s), q2, o, qsoff(h));
       }
@@ -880,20 +934,24 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
     if (on)
 #pragma unroll
       for (int c = 0; c < 4; c++) nzb |= __float_as_uint(p[c]);
-    if (save && on) {
-      const int lr = strip_row_lr(s, z), tb = strip_row_ptb(s, z);
-      const bool near = (x + 3 >= npml - RTM_R && x < npml) || (x + 3 >= nxp - npml && x < nxp - npml + RTM_R);
-      if ((lr >= 0 && near) || tb >= 0)
+    if (save) {
+      const rsrc_t R = strip_rsrc<S16>(s, it);
+      const int r = (z - npml) * RTM_R, tb = strip_row_ptb(s, z);
+      const bool in = on & inner_row(z);
+      if (hasL)
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const int pl = lr >= 0 ? strip_col_plr(s, x + c) : -1;
-          if (pl >= 0) put(2, lr + pl, p[c]);
-          else if (tb >= 0 && inner_col(x + c)) put(3, tb + x + c - npml, p[c]);
-        }
+        for (int c = 0; c < 4; c++) put(R, 2, blr + r + x + c - npml + RTM_R, p[c], in & left(x + c));
+      if (hasR)
+#pragma unroll
+        for (int c = 0; c < 4; c++) put(R, 2, blr + RTM_R * s.nzi + r + x + c - nxp + npml, p[c], in & rightp(x + c));
+      if (any_lane(tb >= 0))
+#pragma unroll
+        for (int c = 0; c < 4; c++) put(R, 3, tb + x + c - npml, p[c], on & (tb >= 0) & inner_col(x + c));
     }
-    bst4<Q::ST>(Rpn, p, pred_off(ooff, on && (!GEN || (x < nxp && z < nzp))), qsoff(h));
+    bst4<Q::ST>(Rpn, p, pred_off(ooff, on & (!GEN | ((x < nxp) & (z < nzp)))), qsoff(h));
   }
-  if (save == 2) {
+  }
+  if (S16 && save) {
 #pragma unroll
     for (int b = 0; b < 4; b++) {
       if (!any_lane(smax[b] > 0.0f)) continue;
@@ -917,7 +975,7 @@ template <class Q, int FK>
 __device__ __forceinline__ void field_step(float* __restrict__ lds, float* __restrict__ ctab, const ShotDev& s,
                                            const Tile& tl, int it, const float* pc, const float* vxc,
                                            const float* vzc, float* pn, float* vxn, float* vzn,
-                                           const float* pr = nullptr, bool img = false, int save = 0,
+                                           const float* pr = nullptr, bool img = false, bool save = false,
                                            unsigned char* actw = nullptr)
 {
   if (!(tl.kind & TF_GEN)) {
@@ -990,10 +1048,10 @@ __device__ __forceinline__ int snap_index(const ShotDev& s, int k)
 
 // ================================================================ kernels ==
 // forward time step of the source wavefield (modelling, recording, strips)
-template <int G, int RPT, bool C>
+template <int G, int RPT, bool C, bool S16>
 __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fwd(LaunchArgs a)
 {
-  using Q = Geo<G, RPT, C>;
+  using Q = Geo<G, RPT, C, S16>;
   __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];   // coefficient table (reduced radii near the edges)
   const int t = xcd_tile(a.ntiles);
@@ -1006,14 +1064,14 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) 
   const ShotDev& s = shot_of(a.shots, tl.slot);
   const int it = s.it_off + s.it_dir * a.step;
   if (track && skip_of(sw, it)) {                      // the forward field is +0 around the tile
-    if (a.save == 1 && (tl.kind & TF_SAVE)) save_zeros<Q>(s, tl, it);
+    if (!S16 && a.save && (tl.kind & TF_SAVE)) save_zeros<Q>(s, tl, it);
     return;
   }
   const bool odd = it & 1;                             // (a runtime index into s would spill it to scratch)
   unsigned char* actw = a.act ? (unsigned char*)(a.act + (size_t)((it + 1) & 1) * a.ntiles + t) : nullptr;
   field_step<Q, FK_SRC>(lds, ctab, s, tl, it, odd ? s.sp[1] : s.sp[0], odd ? s.svx[1] : s.svx[0],
                         odd ? s.svz[1] : s.svz[0], odd ? s.sp[0] : s.sp[1], odd ? s.svx[0] : s.svx[1],
-                        odd ? s.svz[0] : s.svz[1], nullptr, false, a.save, actw);
+                        odd ? s.svz[0] : s.svz[1], nullptr, false, a.save != 0, actw);
 }
 
 // tiles whose receiver halves, then reconstruction halves, follow each other
@@ -1030,10 +1088,10 @@ constexpr int RGRP = 16;
 // L2 from the other workgroup), so the two run at the same time; the last
 // step's products are added by k_image after the pass, those of a step whose
 // snapshot is restored by k_snap_load before it overwrites the field.
-template <int G, int RPT, bool C>
+template <int G, int RPT, bool C, bool S16>
 __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_rev(LaunchArgs a)
 {
-  using Q = Geo<G, RPT, C>;
+  using Q = Geo<G, RPT, C, S16>;
   __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];
   // XCD c's workgroups take its run of the table RGRP tiles at a time, their
@@ -1819,13 +1877,14 @@ template <int G, int RPT>
 static hipError_t launch_step_t(const LaunchArgs& a, int phase, hipStream_t st)
 {
   const dim3 b(64 * G), gf(grid8(a.ntiles)), gr(16 * (((a.ntiles + 7) / 8 + RGRP - 1) / RGRP * RGRP));
-  if (phase == PH_FWD) {
-    if (a.cached) hipLaunchKernelGGL((k_fwd<G, RPT, true>), gf, b, 0, st, a);
-    else hipLaunchKernelGGL((k_fwd<G, RPT, false>), gf, b, 0, st, a);
-  } else {
-    if (a.cached) hipLaunchKernelGGL((k_rev<G, RPT, true>), gr, b, 0, st, a);
-    else hipLaunchKernelGGL((k_rev<G, RPT, false>), gr, b, 0, st, a);
-  }
+  auto go = [&](auto cached, auto s16) {
+    if (phase == PH_FWD) hipLaunchKernelGGL((k_fwd<G, RPT, cached.value, s16.value>), gf, b, 0, st, a);
+    else hipLaunchKernelGGL((k_rev<G, RPT, cached.value, s16.value>), gr, b, 0, st, a);
+  };
+  if (a.cached && a.s16) go(std::true_type{}, std::true_type{});
+  else if (a.cached) go(std::true_type{}, std::false_type{});
+  else if (a.s16) go(std::false_type{}, std::true_type{});
+  else go(std::false_type{}, std::false_type{});
   return hipGetLastError();
 }
 

@@ -708,13 +708,15 @@ void Server::loop()
     if (err_) { cv_done_.notify_all(); std::this_thread::sleep_for(std::chrono::milliseconds(5)); continue; }
     if (ntf_ > 0) {
       LaunchArgs a{d_ds_, d_tf_, ntf_, (int)tick_};
-      a.save = opt_.store_fmt == ST_F32 ? 1 : 2;
+      a.save = 1;
+      a.s16 = opt_.store_fmt != ST_F32;
       if (rtm_launch_step(a, PH_FWD, opt_.tile_z, st_) != hipSuccess) fail("forward launch", hipGetLastError());
       if (nq_ > 0 && opt_.store_fmt != ST_F32) (void)rtm_launch_quant16(d_ds_, d_qs_, nq_, (int)tick_, st_);
       launches_ += 2;
     }
     if (ntr_ > 0) {
       LaunchArgs a{d_ds_, d_tr_, ntr_, (int)tick_};
+      a.s16 = opt_.store_fmt != ST_F32;
       if (rtm_launch_step(a, PH_REV, opt_.tile_z, st_) != hipSuccess) fail("reverse launch", hipGetLastError());
       launches_ += 2;
     }
