@@ -1428,157 +1428,383 @@ __global__ __launch_bounds__(NTHR) void k_gauss_smooth(const float* __restrict__
 // as updated -- until a sweep changes no cell by more than 5e-4 (relative)
 // or 1001 sweeps ran.  The in-place order is kept exactly:
 //   * left and right layers (columns 1..npml-1, rows 1..nz-2 in order, the
-//     reference's ix-outer / iz-inner loop): lane t of one wave owns column
-//     t+1 and runs one row behind lane t-1, which hands it the new value of
-//     its left neighbour by a lane shuffle; the cell above is the lane's own
-//     previous result; the cells right and below are not updated yet in this
-//     sweep and come from memory.  Left and right are independent (two waves).
+//     reference's ix-outer / iz-inner loop), one wave each (smooth_front);
 //   * top and bottom layers (rows 1..npml-1, columns 1..nx-2) the same with
-//     lanes over rows: the new value above from the lane before, the one on
-//     the left the lane's own.
+//     lanes over rows;
 //   * the edge columns and rows: four independent recurrences, one lane
-//     each, on copies staged in LDS; then the four corners.
+//     each, from sums formed beforehand; then the four corners.
 // Each sweep ends with the largest relative change over the layer ring (the
 // rest of the window never changes) and copies the ring back into w.  Sums
 // are formed in the reference's operand order, as floats, scaled by the
-// double literal 0.25.  Needs npml - 1 <= 64, nx, nz >= 3 npml (the
-// mirrors read only interior cells) and nx, nz <= RTM_SMOOTH_MAXN.
+// double literal 0.25 (a power of two: the float product is the same value).
+// What bounds it is the serial chain: about nz + nx + 2 npml dependent steps
+// a sweep and up to 1001 sweeps, on the few CUs that hold windows.  So a
+// step's operands are read ahead, its neighbours come by lane shifts in the
+// VALU, and the ring with one interior line beside it stays in LDS where it
+// fits (SMOOTH_LDS floats); a larger one is read through the caches.  The 16
+// waves are for the comparison of the ring (512 threads: within 10 % at rings
+// in LDS, 15 % slower in memory; 256: 50 % slower).  One window with its
+// transfers, against every operand loaded when needed and shuffled through
+// LDS: 265 x 320, npml 32, 20.0 -> 8.4 ms; 401 x 612, npml 50, 55.5 -> 25.2;
+// 2148 x 1124, npml 50, 162 -> 76.
+// Needs npml - 1 <= 64, nx, nz >= 3 npml (the mirrors read only interior
+// cells) and nx, nz <= RTM_SMOOTH_MAXN.
 #define RTM_SMOOTH_MAXN 4096
 struct SmoothWin { float* w; float* v; int nx, nz, npml, _pad; };
+constexpr int SMT = 1024, SMOOTH_LDS = 40000;
 
-__device__ __forceinline__ float avg4(float a, float b, float c, float d)
+__device__ __forceinline__ float avg4(float a, float b, float c, float d) { return 0.25f * (((a + b) + c) + d); }
+
+// where the cells of the ring are: the full window in memory ...
+struct RingMem {
+  gfloat* p;
+  int nx;
+  __device__ __forceinline__ int at(int r, int c) const { return r * nx + c; }
+  typedef __attribute__((address_space(1))) char gchar;
+  __device__ __forceinline__ gfloat* cell(int a) const { return (gfloat*)((gchar*)p + 4u * (unsigned)a); }
+  __device__ __forceinline__ float get(int a) const { return *cell(a); }
+  __device__ __forceinline__ void set(int a, float x) const { *cell(a) = x; }
+  // rows r0..r1 of a column are this far apart (0: not all the same)
+  __device__ __forceinline__ int row_step(int, int) const { return nx; }
+};
+// ... or the ring and one line beside it (m = npml + 1 deep) in LDS: the top
+// m rows and the bottom m rows in full (even pitch), the rows between as
+// their first and last m columns
+typedef __attribute__((address_space(3))) float lds_float_t;
+struct RingLds {
+  lds_float_t* p;
+  int nx, nz, m, P;
+  __device__ __forceinline__ int at(int r, int c) const
+  {
+    const int rows = imin(r, m) + imax(r - (nz - m), 0), mids = imin(imax(r - m, 0), nz - 2 * m);
+    const int narrow = c < m ? c : c - nx + 2 * m;
+    return rows * P + mids * 2 * m + ((r >= m) & (r < nz - m) ? narrow : c);
+  }
+  __device__ __forceinline__ float get(int a) const { return p[a]; }
+  __device__ __forceinline__ void set(int a, float x) const { p[a] = x; }
+  __device__ __forceinline__ int row_step(int r0, int r1) const { return r0 >= m && r1 < nz - m ? 2 * m : 0; }
+  static __device__ __forceinline__ int floats(int nx, int nz, int npml)
+  {
+    const int m = npml + 1, P = (nx + 1) & ~1;
+    return 2 * m * P + (nz - 2 * m) * 2 * m;
+  }
+};
+
+// lane l's value from lane l-1 (lane 0: `first`) and from lane l+1
+__device__ __forceinline__ float from_before(float first, float x)
 {
-  return (float)(0.25 * (double)(a + b + c + d));
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(x), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float from_after(float x)
+{
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x130, 0xf, 0xf, true));
 }
 
-// one side of the layer, one wave: lanes over `lanes` lines starting at
-// line0, positions 1..len along each line.  LR: lines are columns and
-// positions rows (sum E + W + S + N with W from the lane before, N the
-// lane's own); otherwise lines are rows and positions columns (W the lane's
-// own, N from the lane before).
-template <bool LR>
-__device__ void smooth_side(float* __restrict__ v, int nx, int line0, int lanes, int len)
+// One side of the layer, one wave: `lanes` lines from line0, positions 1..len
+// along each, as a front in which lane t (of line line0 + t) runs one position
+// behind lane t-1.  LR: lines are columns and positions rows; otherwise lines
+// are rows and positions columns.  A step of a lane at position j = 1 + k - t
+// needs four values: the old one at j+1 of its own line (read FB steps ahead:
+// no lane has updated it yet), the old one at j of the next line (what lane
+// t+1 reads in the same step; lane `lanes` reads the line beside for that, or,
+// FULL, the last lane does where all 64 are lines), the new one at j of the
+// line before (the result of lane t-1 in the step before; for lane 0 the line
+// beside) and its own result at j-1.  While every line is under way and no
+// address changes its stride (most of the front), a step is three adds, one
+// multiplication, two lane shifts, two reads and one write.
+template <bool LR, bool FULL, class A>
+__device__ __forceinline__ void smooth_front(const A acc, int line0, int lanes, int len)
 {
+  constexpr int FB = 8;
   const int t = threadIdx.x & 63;
-  float prev = 0.0f;                                 // the lane's new value at the previous position
-  for (int k = 0; k < len + lanes - 1; k++) {
-    const float before = __shfl_up(prev, 1, 64);     // lane t-1's new value at this lane's position
-    const int j = 1 + k - t;
-    if (t < lanes && j >= 1 && j <= len) {
-      const int ln = line0 + t;
-      const size_t c = LR ? (size_t)j * nx + ln : (size_t)ln * nx + j;
-      const float E = v[c + 1], S = v[c + nx];
-      float W, N;
-      if (LR) { W = t > 0 ? before : v[c - 1]; N = j > 1 ? prev : v[c - nx]; }
-      else { W = j > 1 ? prev : v[c - 1]; N = t > 0 ? before : v[c - nx]; }
-      prev = avg4(E, W, S, N);
-      v[c] = prev;
-    }
-  }
-}
-
-__global__ __launch_bounds__(NTHR) void k_pml_smooth(const SmoothWin* __restrict__ wins)
-{
-  __shared__ float ed[8 * RTM_SMOOTH_MAXN];          // col 0, 1, nx-1, nx-2 (nz each), row 0, 1, nz-1, nz-2 (nx each)
-  __shared__ float red[NTHR / 64];
-  __shared__ float err_s;
-  const SmoothWin sw = wins[blockIdx.x];
-  float* __restrict__ w = sw.w;
-  float* __restrict__ v = sw.v;
-  const int nx = sw.nx, nz = sw.nz, npml = sw.npml, tid = threadIdx.x, wave = tid >> 6;
-  // mirror the interior into the layer: columns (rows 1..nz-2), then rows
-  // (columns 1..nx-2, which include the mirrored columns)
-  for (int e = tid; e < npml * (nz - 2); e += NTHR) {
-    const int ix = e % npml, iz = 1 + e / npml;
-    w[(size_t)iz * nx + ix] = w[(size_t)iz * nx + 2 * npml - ix - 1];
-    w[(size_t)iz * nx + nx - npml + ix] = w[(size_t)iz * nx + nx - npml - ix - 1];
-  }
-  __syncthreads();
-  for (int e = tid; e < npml * (nx - 2); e += NTHR) {
-    const int iz = e / (nx - 2), ix = 1 + e % (nx - 2);
-    w[(size_t)iz * nx + ix] = w[(size_t)(2 * npml - iz - 1) * nx + ix];
-    w[(size_t)(nz - npml + iz) * nx + ix] = w[(size_t)(nz - npml - iz - 1) * nx + ix];
-  }
-  __syncthreads();
-  for (long long e = tid; e < (long long)nx * nz; e += NTHR) v[e] = w[e];
-  __syncthreads();
-  float* c0 = ed;
-  float* c1 = ed + nz;
-  float* cN = ed + 2 * nz;
-  float* cM = ed + 3 * nz;
-  float* r0 = ed + 4 * nz;
-  float* r1 = r0 + nx;
-  float* rN = r0 + 2 * nx;
-  float* rM = r0 + 3 * nx;
-  const int ring = 2 * npml * nx + 2 * npml * (nz - 2 * npml);
-  float err = 1.0f;
-  for (int num = 0; num <= 1000 && (double)err > 0.0005; num++) {
-    // left and right layers
-    if (wave == 0) smooth_side<true>(v, nx, 1, npml - 1, nz - 2);
-    else if (wave == 1) smooth_side<true>(v, nx, nx - npml, npml - 1, nz - 2);
-    __syncthreads();
-    // top and bottom layers
-    if (wave == 0) smooth_side<false>(v, nx, 1, npml - 1, nx - 2);
-    else if (wave == 1) smooth_side<false>(v, nx, nz - npml, npml - 1, nx - 2);
-    __syncthreads();
-    // edges: stage, four recurrences, corners, write back
-    for (int i = tid; i < nz; i += NTHR) {
-      c0[i] = v[(size_t)i * nx]; c1[i] = v[(size_t)i * nx + 1];
-      cN[i] = v[(size_t)i * nx + nx - 1]; cM[i] = v[(size_t)i * nx + nx - 2];
-    }
-    for (int i = tid; i < nx; i += NTHR) {
-      r0[i] = v[i]; r1[i] = v[nx + i];
-      rN[i] = v[(size_t)(nz - 1) * nx + i]; rM[i] = v[(size_t)(nz - 2) * nx + i];
-    }
-    __syncthreads();
-    if (tid == 0) {                                  // column 0: C + E + S + N
-      float up = c0[0];
-      for (int iz = 1; iz < nz - 1; iz++) { up = avg4(c0[iz], c1[iz], c0[iz + 1], up); c0[iz] = up; }
-    } else if (tid == 64) {                          // column nx-1
-      float up = cN[0];
-      for (int iz = 1; iz < nz - 1; iz++) { up = avg4(cN[iz], cM[iz], cN[iz + 1], up); cN[iz] = up; }
-    } else if (tid == 128) {                         // row 0: C + S + W + E
-      float lf = r0[0];
-      for (int ix = 1; ix < nx - 1; ix++) { lf = avg4(r0[ix], r1[ix], lf, r0[ix + 1]); r0[ix] = lf; }
-    } else if (tid == 192) {                         // row nz-1
-      float lf = rN[0];
-      for (int ix = 1; ix < nx - 1; ix++) { lf = avg4(rN[ix], rM[ix], lf, rN[ix + 1]); rN[ix] = lf; }
-    }
-    __syncthreads();
-    if (tid == 0) {                                  // corners (none reads another)
-      const float a = avg4(c0[0], c0[1], r0[1], c1[1]);
-      const float b = avg4(c0[nz - 1], c0[nz - 2], rN[1], c1[nz - 2]);
-      const float c = avg4(cN[0], r0[nx - 2], cN[1], cM[1]);
-      const float d = avg4(cN[nz - 1], cN[nz - 2], rN[nx - 2], cM[nz - 2]);
-      c0[0] = a; r0[0] = a; c0[nz - 1] = b; rN[0] = b; cN[0] = c; r0[nx - 1] = c; cN[nz - 1] = d; rN[nx - 1] = d;
-    }
-    __syncthreads();
-    for (int i = tid; i < nz; i += NTHR) { v[(size_t)i * nx] = c0[i]; v[(size_t)i * nx + nx - 1] = cN[i]; }
-    for (int i = tid; i < nx; i += NTHR) { v[i] = r0[i]; v[(size_t)(nz - 1) * nx + i] = rN[i]; }
-    __syncthreads();
-    // largest relative change over the ring, then the ring back into w
-    float m = -1.0e+5f;
-    for (int e = tid; e < ring; e += NTHR) {
-      int iz, ix;
-      if (e < 2 * npml * nx) { const int r = e / nx; iz = r < npml ? r : nz - 2 * npml + r; ix = e - r * nx; }
-      else { const int f = e - 2 * npml * nx, r = f / (2 * npml), c = f - r * 2 * npml;
-             iz = npml + r; ix = c < npml ? c : nx - 2 * npml + c; }
-      const size_t o = (size_t)iz * nx + ix;
-      const float a = w[o], b = v[o];
-      m = fmaxf(m, fabsf(a - b) / fabsf(a));
-      w[o] = b;
+  const int tl = imin(t, lanes), line = line0 + tl;
+  const bool real = t < lanes;
+  auto at = [&](int ln, int pos) {
+    const int q = imin(imax(pos, 0), len + 1);
+    return LR ? acc.at(q, ln) : acc.at(ln, q);
+  };
+  // operands of the steps k0 .. k0+FB-1: own line at 2 + k - t, the line
+  // before lane 0's at 1 + k, the line after the last one's at 2 + k - lanes;
+  // ad: the own line's addresses, the positions updated one step later
+  struct Block { float v[FB], first[FB], last[FB]; int ad[FB]; };
+  auto read = [&](int k0, Block& b) {
+    const int lo = 2 + k0 - lanes, hi = 1 + k0 + FB;
+    const int step = lo >= 0 && hi <= len + 1 ? (LR ? acc.row_step(lo, hi) : 1) : 0;
+    if (step) {
+      const int a = at(line, 2 + k0 - tl), f = at(line0 - 1, 1 + k0);
+#pragma unroll
+      for (int u = 0; u < FB; u++) {
+        b.ad[u] = LR ? a + u * step : a + u;
+        b.first[u] = acc.get(LR ? f + u * step : f + u);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < FB; u++) {
+        b.ad[u] = at(line, 2 + k0 + u - tl);
+        b.first[u] = acc.get(at(line0 - 1, 1 + k0 + u));
+      }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    if ((tid & 63) == 0) red[wave] = m;
+    for (int u = 0; u < FB; u++) b.v[u] = acc.get(b.ad[u]);
+    if (FULL)
+#pragma unroll
+      for (int u = 0; u < FB; u++) b.last[u] = acc.get(at(line0 + lanes, 2 + k0 + u - lanes));
+  };
+  int ab = at(line, 1 - t);                            // address of the position a lane updates
+  float prev = acc.get(at(line, 0));
+  const int K = len + lanes - 1;
+  auto steps = [&](int k0, const Block& cur) {
+    float after[FB];
+#pragma unroll
+    for (int u = 0; u < FB; u++) {
+      after[u] = from_after(cur.v[u]);
+      if (FULL) after[u] = t == 63 ? cur.last[u] : after[u];
+    }
+    auto step = [&](int u) {
+      const float c = from_before(cur.first[u], prev);
+      return LR ? avg4(after[u], c, cur.v[u], prev) : avg4(cur.v[u], prev, after[u], c);
+    };
+    if (k0 >= lanes - 1 && k0 + FB <= len) {           // every line under way for the whole block
+      if (FULL || real)
+#pragma unroll
+        for (int u = 0; u < FB; u++) {
+          prev = step(u);
+          acc.set(u ? cur.ad[u - 1] : ab, prev);
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < FB; u++) {
+        const float x = step(u);
+        const bool act = real & ((unsigned)(k0 + u - t) < (unsigned)len);
+        prev = act ? x : prev;
+        if (act) acc.set(u ? cur.ad[u - 1] : ab, x);
+      }
+    }
+    ab = cur.ad[FB - 1];
+  };
+  Block p, q;
+  read(0, p);
+  for (int k0 = 0; k0 < K; k0 += 2 * FB) {             // (a block past the end reads clamped positions)
+    read(k0 + FB, q);
+    steps(k0, p);
+    read(k0 + 2 * FB, p);
+    steps(k0 + FB, q);
+  }
+}
+
+// One edge line's recurrence, one lane: x(i) = ((s(i) + x(i-1)) [+ e(i)]) / 4
+// for i = 1..n-2 from x(0), in place of s
+template <bool COL, class E>
+__device__ void smooth_edge(lds_float_t* s, int n, float x, E e)
+{
+  constexpr int EB = 8;
+  float a[EB], b[EB];
+  auto read = [&](int i0) {
+#pragma unroll
+    for (int u = 0; u < EB; u++) {
+      a[u] = s[imin(i0 + u, n - 1)];
+      b[u] = COL ? 0.0f : e(imin(i0 + u, n - 2));
+    }
+  };
+  read(1);
+  for (int i0 = 1; i0 < n - 1; i0 += EB) {
+    float ca[EB], cb[EB];
+#pragma unroll
+    for (int u = 0; u < EB; u++) { ca[u] = a[u]; cb[u] = b[u]; }
+    read(i0 + EB);
+#pragma unroll
+    for (int u = 0; u < EB; u++) {
+      x = COL ? 0.25f * (ca[u] + x) : 0.25f * ((ca[u] + x) + cb[u]);
+      if (i0 + u < n - 1) s[i0 + u] = x;
+    }
+  }
+}
+
+// The change of one cell, a the value before the sweep and b after it.  The
+// reference's test is max |a-b| / |a| > 5e-4 in float division; a change
+// clearly past the bound is found by a multiplication (`far`), and only a
+// sweep without any divides.
+struct Change {
+  float far = -1.0e+5f, ratio = -1.0e+5f;
+  __device__ __forceinline__ void add(float a, float b) { far = fmaxf(far, __builtin_fmaf(-5.1e-4f, fabsf(a), fabsf(a - b))); }
+  __device__ __forceinline__ void divide(float a, float b) { ratio = fmaxf(ratio, fabsf(a - b) / fabsf(a)); }
+};
+__device__ __forceinline__ float block_max(float m, float* red)
+{
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  m = red[0];
+#pragma unroll
+  for (int i = 1; i < SMT / 64; i++) m = fmaxf(m, red[i]);
+  return m;
+}
+
+// the cells of the ring a thread compares: those of the LDS ring at tid + u
+// SMT (with the line beside, which never changes), kept in registers ...
+struct OldLds {
+  static constexpr int N = (SMOOTH_LDS + SMT - 1) / SMT;
+  lds_float_t* p;
+  int n;
+  float old[N];
+  __device__ __forceinline__ void take()
+  {
+#pragma unroll
+    for (int u = 0; u < N; u++) old[u] = (int)threadIdx.x + u * SMT < n ? p[threadIdx.x + u * SMT] : 0.0f;
+  }
+  template <bool DIVIDE>
+  __device__ __forceinline__ void compare(Change& c) const
+  {
+#pragma unroll
+    for (int u = 0; u < N; u++)
+      if ((int)threadIdx.x + u * SMT < n) {
+        const float b = p[threadIdx.x + u * SMT];
+        if (DIVIDE) c.divide(old[u], b);
+        else c.add(old[u], b);
+      }
+  }
+};
+// ... or the ring in memory against w: a wave per row, 4 loads in flight
+struct OldMem {
+  gfloat* v;
+  gfloat* w;
+  int nx, nz, npml;
+  template <class F>
+  __device__ __forceinline__ void rows(F f) const
+  {
+    for (int r = threadIdx.x >> 6; r < nz; r += SMT / 64) {
+      const bool mid = r >= npml && r < nz - npml;
+      const int n = mid ? 2 * npml : nx;
+      for (int c0 = threadIdx.x & 63; c0 < n; c0 += 4 * 64) {
+        int o[4];
+        float a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int c = c0 + 64 * u;
+          o[u] = c < n ? r * nx + (mid && c >= npml ? c + nx - 2 * npml : c) : -1;
+          a[u] = o[u] >= 0 ? w[o[u]] : 1.0f;
+          b[u] = o[u] >= 0 ? v[o[u]] : 1.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) f(o[u], a[u], b[u]);
+      }
+    }
+  }
+  __device__ __forceinline__ void take() { rows([&](int o, float, float b) { if (o >= 0) w[o] = b; }); }
+  template <bool DIVIDE>
+  __device__ __forceinline__ void compare(Change& c) const
+  {
+    rows([&](int, float a, float b) { if (DIVIDE) c.divide(a, b); else c.add(a, b); });
+  }
+};
+
+template <bool FULL, class A, class O>
+__device__ __forceinline__ void smooth_sweeps(const A acc, O& old, lds_float_t* T, float* red, int nx, int nz, int npml)
+{
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  lds_float_t* c0 = T;                                 // columns 0 and nx-1 (nz each), rows 0 and nz-1 (nx each)
+  lds_float_t* cN = T + nz;
+  lds_float_t* r0 = T + 2 * nz;
+  lds_float_t* rN = r0 + nx;
+  auto g = [&](int r, int c) { return acc.get(acc.at(r, c)); };
+  old.take();
+  for (int num = 0; num <= 1000; num++) {
+    // left and right layers, then top and bottom layers
+    if (wave < 2) smooth_front<true, FULL>(acc, wave ? nx - npml : 1, npml - 1, nz - 2);
     __syncthreads();
-    if (tid == 0) {
-      float x = red[0];
-      for (int i = 1; i < NTHR / 64; i++) x = fmaxf(x, red[i]);
-      err_s = x;
+    if (wave < 2) smooth_front<false, FULL>(acc, wave ? nz - npml : 1, npml - 1, nx - 2);
+    __syncthreads();
+    // edges.  Columns: C + E + S + N, rows: C + S + W + E, N and W being the
+    // recurrence's own last value
+    for (int i = 1 + tid; i < nz - 1; i += SMT) {
+      c0[i] = (g(i, 0) + g(i, 1)) + g(i + 1, 0);
+      cN[i] = (g(i, nx - 1) + g(i, nx - 2)) + g(i + 1, nx - 1);
+    }
+    for (int i = 1 + tid; i < nx - 1; i += SMT) {
+      r0[i] = g(0, i) + g(1, i);
+      rN[i] = g(nz - 1, i) + g(nz - 2, i);
     }
     __syncthreads();
-    err = err_s;
+    if (tid == 0) smooth_edge<true>(c0, nz, g(0, 0), [](int) { return 0.0f; });
+    else if (tid == 64) smooth_edge<true>(cN, nz, g(0, nx - 1), [](int) { return 0.0f; });
+    else if (tid == 128) smooth_edge<false>(r0, nx, g(0, 0), [&](int i) { return g(0, i + 1); });
+    else if (tid == 192) smooth_edge<false>(rN, nx, g(nz - 1, 0), [&](int i) { return g(nz - 1, i + 1); });
+    __syncthreads();
+    for (int i = 1 + tid; i < nz - 1; i += SMT) { acc.set(acc.at(i, 0), c0[i]); acc.set(acc.at(i, nx - 1), cN[i]); }
+    for (int i = 1 + tid; i < nx - 1; i += SMT) { acc.set(acc.at(0, i), r0[i]); acc.set(acc.at(nz - 1, i), rN[i]); }
+    __syncthreads();
+    if (tid == 0) {                                    // corners (none reads another)
+      const float a = avg4(g(0, 0), g(1, 0), g(0, 1), g(1, 1));
+      const float b = avg4(g(nz - 1, 0), g(nz - 2, 0), g(nz - 1, 1), g(nz - 2, 1));
+      const float c = avg4(g(0, nx - 1), g(0, nx - 2), g(1, nx - 1), g(1, nx - 2));
+      const float d = avg4(g(nz - 1, nx - 1), g(nz - 2, nx - 1), g(nz - 1, nx - 2), g(nz - 2, nx - 2));
+      acc.set(acc.at(0, 0), a); acc.set(acc.at(nz - 1, 0), b);
+      acc.set(acc.at(0, nx - 1), c); acc.set(acc.at(nz - 1, nx - 1), d);
+    }
+    __syncthreads();
+    // the largest change against the sweep before, whose values then go
+    Change ch;
+    old.template compare<false>(ch);
+    bool more = block_max(ch.far, red) > 0.0f;
+    if (!more) {
+      old.template compare<true>(ch);
+      more = (double)block_max(ch.ratio, red) > 0.0005;
+    }
+    old.take();
+    if (!more) break;
+    __syncthreads();
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(SMT) void k_pml_smooth(const SmoothWin* __restrict__ wins)
+{
+  __shared__ float S[SMOOTH_LDS];
+  __shared__ float red[SMT / 64];
+  const SmoothWin sw = wins[blockIdx.x];
+  gfloat* w = GF(sw.w);
+  const int nx = sw.nx, nz = sw.nz, npml = sw.npml, tid = threadIdx.x;
+  // mirror the interior into the layer: columns (rows 1..nz-2), then rows
+  // (columns 1..nx-2, which include the mirrored columns)
+  for (int e = tid; e < npml * (nz - 2); e += SMT) {
+    const int ix = e % npml, iz = 1 + e / npml;
+    w[iz * nx + ix] = w[iz * nx + 2 * npml - ix - 1];
+    w[iz * nx + nx - npml + ix] = w[iz * nx + nx - npml - ix - 1];
+  }
+  __syncthreads();
+  for (int e = tid; e < npml * (nx - 2); e += SMT) {
+    const int iz = e / (nx - 2), ix = 1 + e % (nx - 2);
+    w[iz * nx + ix] = w[(2 * npml - iz - 1) * nx + ix];
+    w[(nz - npml + iz) * nx + ix] = w[(nz - npml - iz - 1) * nx + ix];
+  }
+  __syncthreads();
+  lds_float_t* L = (lds_float_t*)S;
+  const int rf = RingLds::floats(nx, nz, npml);
+  if (rf + 2 * (nx + nz) <= SMOOTH_LDS && npml <= 64) {
+    const RingLds acc{L, nx, nz, npml + 1, (nx + 1) & ~1};
+    const int m = npml + 1;
+    for (int e = tid; e < nx * nz; e += SMT) {
+      const int r = e / nx, c = e - r * nx;
+      if (r < m || r >= nz - m || c < m || c >= nx - m) acc.set(acc.at(r, c), w[e]);
+    }
+    if (tid < 2 * m && acc.P > nx)                     // the pad of the full rows
+      L[(tid < m ? tid : tid - m) * acc.P + (tid < m ? 0 : m * acc.P + (nz - 2 * m) * 2 * m) + nx] = 1.0f;
+    __syncthreads();
+    OldLds old{L, rf};
+    smooth_sweeps<false>(acc, old, L + rf, red, nx, nz, npml);
+    for (int e = tid; e < nx * nz; e += SMT) {
+      const int r = e / nx, c = e - r * nx;
+      if (r < npml || r >= nz - npml || c < npml || c >= nx - npml) w[e] = acc.get(acc.at(r, c));
+    }
+  } else {
+    gfloat* v = GF(sw.v);
+    for (int e = tid; e < nx * nz; e += SMT) v[e] = w[e];
+    __syncthreads();
+    OldMem old{v, w, nx, nz, npml};
+    if (npml <= 64) smooth_sweeps<false>(RingMem{v, nx}, old, L, red, nx, nz, npml);
+    else smooth_sweeps<true>(RingMem{v, nx}, old, L, red, nx, nz, npml);
   }
 }
 
@@ -2021,7 +2247,7 @@ hipError_t rtm_launch_gauss_smooth(const float* in, float* out, int nz, int nx, 
 hipError_t rtm_launch_pml_smooth(const void* wins, int n, hipStream_t st)
 {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pml_smooth, dim3(n), dim3(NTHR), 0, st, (const SmoothWin*)wins);
+  hipLaunchKernelGGL(k_pml_smooth, dim3(n), dim3(SMT), 0, st, (const SmoothWin*)wins);
   return hipGetLastError();
 }
 
