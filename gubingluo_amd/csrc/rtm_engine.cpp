@@ -595,10 +595,35 @@ bool GraphKey::operator<(const GraphKey& o) const
   return slots < o.slots;
 }
 
+hipStream_t stream_beside(hipStream_t a)
+{
+  long long* t = nullptr;                              // start and end of the two launches
+  if (hipHostMalloc((void**)&t, 4 * sizeof(long long)) != hipSuccess) { (void)hipGetLastError(); t = nullptr; }
+  hipStream_t b = nullptr;
+  std::vector<hipStream_t> same;
+  for (int i = 0; i < 8; i++) {
+    if (b) same.push_back(b);                          // (kept until the end: its queue stays taken)
+    b = nullptr;
+    if (hipStreamCreateWithFlags(&b, hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); b = nullptr; break; }
+    if (!t) break;
+    // the first launches on a stream take longer to start
+    bool ok = rtm_launch_clock(t, 0, a) == hipSuccess && rtm_launch_clock(t + 2, 0, b) == hipSuccess &&
+              hipStreamSynchronize(a) == hipSuccess && hipStreamSynchronize(b) == hipSuccess &&
+              rtm_launch_clock(t, 20000, a) == hipSuccess && rtm_launch_clock(t + 2, 0, b) == hipSuccess &&
+              hipStreamSynchronize(a) == hipSuccess && hipStreamSynchronize(b) == hipSuccess;
+    if (!ok || t[2] < t[1]) break;
+  }
+  if (!b && !same.empty()) { b = same.back(); same.pop_back(); }
+  for (hipStream_t s : same) (void)hipStreamDestroy(s);
+  if (t) (void)hipHostFree(t);
+  return b;
+}
+
 Engine::Engine(int device) : device_(device)
 {
   (void)hipSetDevice(device_);
-  for (auto& l : lane_) (void)hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking);
+  (void)hipStreamCreateWithFlags(&lane_[0].st, hipStreamNonBlocking);
+  lane_[1].st = stream_beside(lane_[0].st);
   st_ = lane_[0].st;
 }
 

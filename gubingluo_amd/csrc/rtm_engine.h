@@ -55,6 +55,14 @@ void ricker(std::vector<float>& w, int nt, float fdom, float dt);
 // taper row (kernel.cu:1591-1604)
 void taper_row(std::vector<float>& t, int nxl, int nwin);
 
+// A new stream that runs beside `a` (null: none could be created).  Streams
+// share a few hardware queues per process (4 by default), and launches on one
+// queue do not overlap: two lanes on one queue served a mix of requests in 108
+// ms, on two in 83.  Which queue a new stream gets depends on the streams the
+// process has, so the overlap is tried: a later launch on the new stream has
+// to start before a 0.2 ms one on `a` ends.
+hipStream_t stream_beside(hipStream_t a);
+
 // ---- device memory pool ------------------------------------------------------
 // First-fit carving of one range [0, bytes) into blocks of whole 256-byte
 // units; put() merges a freed block with the free ranges either side of it.

@@ -2033,6 +2033,20 @@ __global__ __launch_bounds__(NTHR) void k_zero_f64(double* __restrict__ a, long 
   if (e < n) a[e] = 0.0;
 }
 
+// one wave that lasts `ticks` of the constant 100 MHz clock (and ends after a
+// bounded number of reads of it whatever the clock does): t[0], t[1] = its
+// start and end
+__global__ void k_clock(long long* __restrict__ t, long long ticks)
+{
+  const long long b = wall_clock64();
+  long long e = b;
+  for (int i = 0; i < 100000 && e - b < ticks; i++) e = wall_clock64();
+  if (threadIdx.x == 0) {
+    t[0] = b;
+    t[1] = e;
+  }
+}
+
 // Wavefield guard: the device form of the reference's max|p| print every
 // ntsnap steps (rtm_model.cu:271-273, 324, 415).  The largest |p| of each
 // listed slot's pressure as written by step `step` (it = it_off + it_dir *
@@ -2131,6 +2145,12 @@ hipError_t rtm_launch_step(const LaunchArgs& a, int phase, int tz, hipStream_t s
     case 64: return launch_step_t<8, 8>(a, phase, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t rtm_launch_clock(long long* t, long long ticks, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_clock, dim3(1), dim3(64), 0, st, t, ticks);
+  return hipGetLastError();
 }
 
 hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, int it, hipStream_t st)

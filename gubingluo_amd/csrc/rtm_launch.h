@@ -7,6 +7,8 @@
 // modelling) or PH_REV (reconstruction, receiver wavefield, imaging); tz the
 // tile height (16, 32 or 64)
 hipError_t rtm_launch_step(const LaunchArgs& a, int phase, int tz, hipStream_t st);
+// a wave of `ticks` (100 MHz): t[0], t[1] (host-visible) = its start and end
+hipError_t rtm_launch_clock(long long* t, long long ticks, hipStream_t st);
 // after the last reverse step `it` of the listed slots: its imaging products
 // (every other reverse step's are added by the step after it)
 hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, int it, hipStream_t st);
