@@ -951,7 +951,7 @@ int Engine::run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, 
           Group& g = groups[r.next];
           r.next += nl;
           r.g = &g;
-          r.left = nsteps - g.done;
+          r.left = nsteps;
           r.step = 0;
           const int nt = (int)g.tiles.size(), ns = (int)g.slots.size();
           HIPCHK(hipMemcpyAsync(L.tiles, d_tiles_ + g.tile0, nt * sizeof(Tile), hipMemcpyDeviceToDevice, L.st));
@@ -1315,10 +1315,9 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     return -1;
   }
   if (opt.tile_z != 0 && opt.tile_z != 16 && opt.tile_z != 32 && opt.tile_z != 64) {
-    set_error("tile_z must be 0 (autotuned), 16, 32 or 64");
+    set_error("tile_z must be 0 (by size), 16, 32 or 64");
     return -1;
   }
-  int tz = opt.tile_z > 0 ? opt.tile_z : 16;
   const Model* M = model(model_id);
   if (!M) { set_error("no such model"); return -1; }
   if (M->nx != P.nx || M->nz != P.nz) { set_error("model size differs from nx, nz"); return -1; }
@@ -1432,7 +1431,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
   hipEvent_t e0, e1, e2;
   HIPCHK(hipEventCreate(&e0)); HIPCHK(hipEventCreate(&e1)); HIPCHK(hipEventCreate(&e2));
   double fwd_ms = 0, rev_ms = 0, cells = 0, algb = 0, step_fwd = 0, step_rev = 0, fwdb = 0, revb = 0;
-  int last_tz = tz, last_tz_r = tz;
+  int last_tz = 0, last_tz_r = 0;
   if (stats) memset(stats, 0, sizeof(*stats));
   int nbatches = 0, maxb = 0;
   std::vector<double> img_tmp;  // for temp-image checkpoints
@@ -1461,27 +1460,6 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
       ds[j].record = (P.mode == 0) ? 1 : 0;
     }
     if (rc != 0) { for (void* p : mem) pool_.put(p); break; }
-    // tile height: given, cached for this geometry class, or tuned on the
-    // first forward steps of this batch (every candidate computes the same
-    // values, so the tuning steps are part of the pass)
-    int maxp = 0, maxz = 0;
-    for (int j = 0; j < nb; j++) { maxp = std::max(maxp, ds[j].nxp); maxz = std::max(maxz, ds[j].nzp); }
-    // the forward and reverse step kernels differ, so each pass has its own
-    // tile height (key bit 62: reverse)
-    const long long tkey = ((long long)(maxp / 64) << 40) | ((long long)(maxz / 32) << 20) | nb;
-    const long long rkey = tkey | (1LL << 62);
-    const int cands[3] = {16, 32, 64};
-    bool tune = false, tune_r = false;
-    int tz_r = tz;
-    if (opt.tile_z == 0) {
-      const bool can = nt >= 3 * kTuneSteps + 2 && !opt.profile;
-      auto ct = tuned_.find(tkey);
-      if (ct != tuned_.end()) tz = ct->second;
-      else tune = can;
-      auto cr = tuned_.find(rkey);
-      if (cr != tuned_.end()) tz_r = cr->second;
-      else tune_r = can;
-    }
     // groups of shots for each pass (one group when every launch is timed by
     // itself), and tables of any height for them (per-XCD runs are padded to
     // at most 1.25 x the even share)
@@ -1501,6 +1479,25 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
       return g;
     };
     std::vector<Group> gf = plan(PH_FWD, cached_f), gr = plan(PH_REV, cached_r);
+    // tile height of a pass: given, or by the 32-row tiles of the groups in
+    // flight.  Few tiles: 16 rows, whose workgroups' chains are the shortest;
+    // from 1000 forward, 1400 reverse, 32 rows, which do less halo work a cell
+    // and, forward, let the tiles the wavefield has not reached skip.  us per
+    // step with 16 / 32 rows, forward: 800 tiles 15.5 / 17.5, 896 14.9 / 16.2,
+    // 1120 16.8 / 15.5, 1428 19.2 / 16.2, 5980 (nt 3000) 97 / 76; reverse: 896
+    // 24.4 / 25.7, 1200 32.3 / 32.2, 1224 (one shot) 38.8 / 42.0, 1428 37.7 /
+    // 37.6, 1680 43.8 / 40.1, 2448 82.3 / 74.3.  64 rows were the fastest in
+    // none of them.  (Timing the heights on a pass's first steps chose 16 rows
+    // for forward passes that skip later, and cost those steps.)
+    auto height = [&](const std::vector<Group>& gs, int phase) {
+      if (opt.tile_z) return opt.tile_z;
+      double n = 0;                                    // (groups are of about equal size)
+      for (const Group& g : gs)
+        for (int k : g.slots) n += (double)((ds[k].nxp + 63) / 64) * ((ds[k].nzp + 31) / 32);
+      n *= std::min((double)kLanes / gs.size(), 1.0);
+      return n >= (phase == PH_FWD ? 1000 : 1400) ? 32 : 16;
+    };
+    const int tz = height(gf, PH_FWD), tz_r = height(gr, PH_REV);
     size_t tcap = 0;
     {
       std::vector<Tile> t;
@@ -1516,51 +1513,6 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
         layout_runs(g.tiles, phase);
         if (phase == PH_FWD) link_neighbours(g.tiles, h);
       }
-    };
-    // the first 3 x kTuneSteps steps of the groups that start a pass (as one
-    // launch, the load of the lanes together), kTuneSteps with each candidate
-    // height, timed with events after the height's first kWarmSteps; every
-    // candidate computes the same cells, so these are steps of the pass.
-    // Returns the fastest height.
-    auto tune_pass = [&](int phase, std::vector<Group>& gs, bool cached) -> int {
-      std::vector<int> sl;
-      for (size_t i = 0; i < gs.size() && i < (size_t)kLanes; i++) {
-        sl.insert(sl.end(), gs[i].slots.begin(), gs[i].slots.end());
-        gs[i].done = 3 * kTuneSteps;
-      }
-      std::vector<ShotDev> sub;
-      for (int j : sl) sub.push_back(ds[j]);
-      hipEvent_t te[6];
-      for (auto& e : te) HIPCHK(hipEventCreate(&e));
-      const Lane& L = lane_[0];
-      HIPCHK(hipMemcpyAsync(L.slots, sl.data(), sl.size() * 4, hipMemcpyHostToDevice, st_));
-      std::vector<Tile> tc[3];
-      for (int c = 0; c < 3; c++) {
-        build_tiles(sub, cands[c], tc[c], &sl);
-        layout_runs(tc[c], phase);
-        HIPCHK(hipMemcpyAsync(L.tiles, tc[c].data(), tc[c].size() * sizeof(Tile), hipMemcpyHostToDevice, st_));
-        LaunchArgs a{d_ds_, L.tiles, (int)tc[c].size(), 0};
-        a.cached = cached ? 1 : 0;
-        keep_strips(a, opt.store_fmt);
-        for (int s2 = 0; s2 < kTuneSteps; s2++) {
-          if (s2 == kWarmSteps) HIPCHK(hipEventRecord(te[2 * c], st_));
-          a.step = c * kTuneSteps + s2;
-          const int e = step_launches(a, phase, cands[c], opt.store_fmt, L, (int)sl.size());
-          if (e) return e;
-        }
-        HIPCHK(hipEventRecord(te[2 * c + 1], st_));
-      }
-      HIPCHK(rtm_launch_bump(d_ds_, L.slots, (int)sl.size(), 3 * kTuneSteps, st_));
-      HIPCHK(hipEventSynchronize(te[5]));
-      float best = 1e30f;
-      int pick = cands[0];
-      for (int c = 0; c < 3; c++) {
-        float m = 0;
-        HIPCHK(hipEventElapsedTime(&m, te[2 * c], te[2 * c + 1]));
-        if (m < best) { best = m; pick = cands[c]; }
-      }
-      for (auto& e : te) (void)hipEventDestroy(e);
-      return pick;
     };
     if (ensure_cb(nb, tcap) != 0) { for (void* p : mem) pool_.put(p); rc = -3; break; }
     ShotDev* d_ds = d_ds_;
@@ -1580,11 +1532,6 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     // ---- forward pass: propagation + record + boundary strips
     if (guard_clear() != 0) { for (void* p : mem) pool_.put(p); rc = -10; break; }
     HIPCHK(hipEventRecord(e0, st_));
-    if (tune) {
-      tz = tune_pass(PH_FWD, gf, cached_f);
-      if (tz < 0) { for (void* p : mem) pool_.put(p); rc = tz; break; }
-      tuned_[tkey] = tz;
-    }
     tables(gf, PH_FWD, tz);
     rc = prof ? profile_pass(PH_FWD, nt, gf[0], tz, opt.store_fmt, stats, fwd_skip_ok(tz))
               : run_pass(PH_FWD, nt, gf, tz, opt.store_fmt, opt.graph_chunk, cached_f, guard_every, fwd_skip_ok(tz));
@@ -1693,11 +1640,6 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     if (opt.verbose) printf("source wavefiled prepared over...\nBegin backward......\n");
     if (guard_clear() != 0) { for (void* p : mem) pool_.put(p); rc = -10; break; }
     HIPCHK(hipEventRecord(e1, st_));
-    if (tune_r) {
-      tz_r = tune_pass(PH_REV, gr, cached_r);
-      if (tz_r < 0) { for (void* p : mem) pool_.put(p); rc = tz_r; break; }
-      tuned_[rkey] = tz_r;
-    }
     tables(gr, PH_REV, tz_r);
     rc = prof ? profile_pass(PH_REV, nt - 1, gr[0], tz_r, opt.store_fmt, stats, false)
               : run_pass(PH_REV, nt - 1, gr, tz_r, opt.store_fmt, opt.graph_chunk, cached_r, guard_every, false);

@@ -277,19 +277,16 @@ class Engine {
   Lane lane_[kLanes];
   std::vector<Tile> stage_tiles_;       // host copies of a pass's uploads (kept until the next pass)
   std::vector<int> stage_slots_;
-  // the shots of one group: indices into the batch, its tile table, the steps
-  // it has taken (the autotuner's), its place in the uploaded tables
+  // the shots of one group: indices into the batch, its tile table, its place
+  // in the uploaded tables
   struct Group {
     std::vector<int> slots;
     std::vector<Tile> tiles;
-    int done = 0;
     size_t tile0 = 0, slot0 = 0;
   };
   DevPool pool_;
   std::map<GraphKey, hipGraphExec_t> graphs_;
   std::map<int, Model> models_;
-  std::map<long long, int> tuned_;      // geometry class -> tile height
-  static constexpr int kTuneSteps = 12, kWarmSteps = 4;
   mutable std::mutex models_mu_;
   int next_model_ = 1;
   // persistent control block: captured graphs reference these addresses

@@ -104,7 +104,7 @@ typedef struct rtmh_options {
   int batch;          /* shots per launch; 0 = as many as fit the memory budget  */
   int store_fmt;      /* boundary store: RTMH_STORE_F32 / _F16 / _BF16           */
   int graph_chunk;    /* time steps per captured hipGraph; 0 = plain launches    */
-  int tile_z;         /* tile height 16/32/64; 0 = autotuned                     */
+  int tile_z;         /* tile height 16/32/64; 0 = by the size of the launches   */
   int write_files;    /* reproduce the reference's file side effects             */
   int verbose;        /* 0 silent, 1 per-shot lines as the reference prints       */
   double mem_budget;  /* bytes of HBM for shot slots; 0 = 80% of free memory      */
