@@ -74,6 +74,19 @@ __device__ __forceinline__ const ShotDev& shot_of(const ShotDev* shots, int slot
   return *(const ShotDev*)((const_shot_t*)shots + slot);
 }
 
+// The descriptor's cache lines, all fetched at once: its members are read a
+// few at a time all along a step, and each line's first read would wait for
+// memory by itself.
+__device__ __forceinline__ void fetch_shot(const ShotDev* __restrict__ shots, int slot)
+{
+  typedef const __attribute__((address_space(4))) int const_int_t;
+  constexpr int N = (sizeof(ShotDev) + 63) / 64;
+  static_assert(N == 8, "one word of each line");
+  const_int_t* p = (const_int_t*)((const_shot_t*)shots + slot);
+  const int a = p[0], b = p[16], c = p[32], d = p[48], e = p[64], f = p[80], g = p[96], h = p[112];
+  asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d), "s"(e), "s"(f), "s"(g), "s"(h));
+}
+
 // blockIdx -> tile: workgroups are dealt to the 8 XCDs round-robin, so give
 // each XCD a contiguous run of the tile table (neighbouring tiles of one shot
 // share their halos through that XCD's L2).
@@ -143,6 +156,7 @@ struct Geo {
   static constexpr bool S16 = S16_;                    // the boundary store is 16-bit
   static constexpr int ST = CACHED ? 0 : 2;            // cache policy of the field stores (bst)
   static constexpr int TZ = G * RPT;                   // tile rows
+  static constexpr int SPLIT = TZ < 16 ? 16 / TZ : 1;  // workgroups that share a tile of the table (16 rows or more)
   static constexpr int NT = 64 * G;                    // threads
   static constexpr int PW = 108;                       // p row: column x at float x - x0 + 21 (x0-20..x0+83 held):
                                                        // a quad's window x-9..x+14 starts on 16 bytes
@@ -156,7 +170,8 @@ struct Geo {
   static constexpr int LDS_A = PZR * PW;               // p rows z0-19..
   static constexpr int LDS_B = 4 + TZ * VXW + ZR * 64; // new vx | new vz
   static constexpr int LDS = LDS_A > LDS_B ? LDS_A : LDS_B;
-  static constexpr int LDS_D = 2 * VXW;                // vx damping of the tile's columns (after LDS)
+  static constexpr int LDS_D = 2 * VXW + 128 + 2 * TZ; // damping factors (after LDS): of vx at columns x0-12..x0+75,
+                                                       // of p at the tile's columns and rows
   static_assert(RPT == 2 || RPT % 4 == 0, "own quads fill whole waves, or half of one");
 };
 
@@ -291,6 +306,12 @@ __device__ __forceinline__ void part() { __builtin_amdgcn_sched_barrier(0); }
 // would otherwise be computed there, and its whole window held until then
 __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 
+// lane k's value (k < 64 known at compile time) as a scalar
+__device__ __forceinline__ float lane_value(float v, int k)
+{
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+}
+
 // sum of the staggered differences w[h + i] - w[h + 1 - i], i = 1..10, as the
 // reference loops (kernel.cu:459-460), one fused multiply-add a tap
 template <class W, class Cf>
@@ -308,18 +329,32 @@ __device__ __forceinline__ float taps(const W& w, int h, const Cf& c)
 // are finite cells of the staged halo or the zero margins), and row 9 gives
 // the radius-10 sum bit for bit.
 constexpr int CTW = 12;
+struct CoefRow {
+  f4 a, b;
+  f2 d;
+  __device__ __forceinline__ CoefRow(const float* ctab, int r)
+  {
+    const f4* cr = (const f4*)(ctab + (r - 1) * CTW);
+    a = cr[0];
+    b = cr[1];
+    d = *(const f2*)(cr + 2);
+  }
+};
 template <class W>
-__device__ __forceinline__ float taps_r(const W& w, int h, const float* ctab, int r)
+__device__ __forceinline__ float taps_r(const W& w, int h, const CoefRow& r)
 {
-  const f4* cr = (const f4*)(ctab + (r - 1) * CTW);
-  const f4 a = cr[0], b = cr[1], d = cr[2];
-  const float c[RTM_R] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, d.x, d.y};
+  const float c[RTM_R] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w, r.d.x, r.d.y};
   // (the difference as -(b - a), the same value: the compiler would hoist the
   // differences it shares with the full-radius branch and hold them)
   float acc = 0.0f;
 #pragma unroll
   for (int i = 1; i <= RTM_R; i++) acc = __builtin_fmaf(c[i - 1], -(w[h + 1 - i] - w[h + i]), acc);
   return acc;
+}
+template <class W>
+__device__ __forceinline__ float taps_r(const W& w, int h, const float* ctab, int r)
+{
+  return taps_r(w, h, CoefRow(ctab, r));
 }
 // entry t of that table
 __device__ __forceinline__ float ctab_entry(const ShotDev& s, int t)
@@ -378,6 +413,8 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   unsigned int nzb = 0u;
   float* PS = lds;                                     // p rows z0-19.., columns x0-20..x0+83 from float 1 of a row
   float* DMP = lds + Q::LDS;                           // a, b of vx at columns x0-12.. (88 each)
+  float* DPX = DMP + 2 * VXW;                          // a, b of p at the tile's columns (64 each)
+  float* DPZ = DPX + 128;                              // a, b of p at the tile's rows
   float* VXL = lds + 4;                                // (after the pressure is consumed) column x at x - x0 + 10
   float* VZL = lds + 4 + TZ * VXW;                     // new vz rows z0-10.., 64 columns
   const int lane = threadIdx.x & 63;
@@ -419,10 +456,6 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
   const bool edge_x = EDGE && (x0 - 12 <= 9 || x0 + 75 >= nxp - 10);
   const bool mfree = !GEN || (x0 - 12 >= s.mxs && x0 + 76 <= s.mxs + s.mxn);
   const bool inner_cols = !GEN || (x0 >= npml && x0 + 64 <= nxp - npml);
-  float c10[RTM_R];
-#pragma unroll
-  for (int i = 0; i < RTM_R; i++) c10[i] = CCF(s.coef)[90 + i];
-
   // ---- 1. the pressure and its halo into LDS (buffer loads with the lds
   //         modifier: lane i of a wave writes its dword to base + 4 i): tile
   //         rows as two full-wave loads (x0-20..x0+43, x0+20..x0+83; the
@@ -449,6 +482,10 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       }
     }
   }
+  part();                                              // (nothing waits before these loads are on their way)
+  float c10[RTM_R];
+#pragma unroll
+  for (int i = 0; i < RTM_R; i++) c10[i] = CCF(s.coef)[90 + i];
   // rows of the z phase that exist for every wave need no test
   auto zrow = [&](int k) { return k < ZR - (G - 1) * KZ || g * KZ + k < ZR; };
   const int mcol = model_col(s, ix);
@@ -495,6 +532,19 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       ((f4*)DMP)[t] = *(const gf4*)(GCF(s.axv) + x0 - 12 + 4 * t);
       ((f4*)DMP)[22 + t] = *(const gf4*)(GCF(s.bxv) + x0 - 12 + 4 * t);
     }
+    for (int t = threadIdx.x; t < 128 + 2 * TZ; t += 64 * G) {
+      const gfloat* src = t < 64 ? GCF(s.ax) + x0 : t < 128 ? GCF(s.bx) + x0 - 64
+                         : t < 128 + TZ ? GCF(s.az) + z0 - 128 : GCF(s.bz) + z0 - 128 - TZ;
+      DPX[t] = src[t];
+    }
+  }
+  // (damping of the wave's vz rows: lane k holds row k's, so that a row reads
+  // it as a scalar with no memory access)
+  float azl = 1.0f, bzl = 0.0f;
+  if (!RCN && GEN) {
+    const int r = z0 - 10 + imin(g * KZ + lane, ZR - 1);
+    azl = GCF(s.azv)[r];
+    bzl = GCF(s.bzv)[r];
   }
   __builtin_amdgcn_s_waitcnt(0);                       // the LDS writes of the staging loads
   __syncthreads();                                     // p staged
@@ -581,7 +631,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
             sum = taps(cw, k + 9, c10);
           }
           const float u = (sum * dtz) * ibz[k];
-          vzn_[k] = GEN ? __builtin_fmaf(CCF(s.azv)[iz], vzo[k], -(u * CCF(s.bzv)[iz])) : vzo[k] - u;
+          vzn_[k] = GEN ? __builtin_fmaf(lane_value(azl, k), vzo[k], -(u * lane_value(bzl, k))) : vzo[k] - u;
         }
       }
       pin(vzn_[k]);
@@ -763,7 +813,7 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
       w[4 * m] = v.x; w[4 * m + 1] = v.y; w[4 * m + 2] = v.z; w[4 * m + 3] = v.w;
     }
     int rad[4] = {RTM_R, RTM_R, RTM_R, RTM_R};
-    bool red = false;
+    bool red = false, mixed = false;
     if (EDGE && !RCN) {
 #pragma unroll
       for (int c = 0; c < 4; c++) {
@@ -771,16 +821,28 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
         if (((unsigned)(z - 1) < (unsigned)(nzp - 2)) & ((unsigned)(x - 1) < (unsigned)(nxp - 2)))
           rad[c] = imin(imin(RTM_R, imin(x, nxp - 1 - x)), imin(z, nzp - 1 - z));
         red = red | (rad[c] != RTM_R);
+        mixed = mixed | (rad[c] != rad[0]);
       }
       red = any_lane(red);
+      mixed = any_lane(mixed);
     }
+    if (EDGE && !RCN && red && !mixed) {               // (away from the left and right edge: one row of coefficients)
+      const CoefRow cr(ctab, rad[0]);
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-      float v;
-      if (EDGE && !RCN && red) v = taps_r(w, 9 + c, ctab, rad[c]);
-      else v = taps(w, 9 + c, c10);
-      pin(v);
-      dx_[h][c] = v;
+      for (int c = 0; c < 4; c++) {
+        float v = taps_r(w, 9 + c, cr);
+        pin(v);
+        dx_[h][c] = v;
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        float v;
+        if (EDGE && !RCN && red) v = taps_r(w, 9 + c, ctab, rad[c]);
+        else v = taps(w, 9 + c, c10);
+        pin(v);
+        dx_[h][c] = v;
+      }
     }
   }
   part();
@@ -890,9 +952,9 @@ __device__ __forceinline__ void tile_step(float* __restrict__ lds, const float* 
 #pragma unroll
       for (int c = 0; c < 4; c++) p[c] = inner_row(z) & inner_col(x + c) ? pu[c] : po[h][c];
       if (any_lane(split_q(z, x))) {                   // split pair, p = p1 + p2 (kernel.cu:774-783)
-        const f4 ax = *(const gf4*)(GCF(s.ax) + x);
-        const f4 bx = *(const gf4*)(GCF(s.bx) + x);
-        const float az = GCF(s.az)[z], bz = GCF(s.bz)[z];
+        const f4 ax = *(const f4*)(DPX + (oq ? ocol : 0));
+        const f4 bx = *(const f4*)(DPX + 64 + (oq ? ocol : 0));
+        const float az = DPZ[g * RPT + qrow(h)], bz = DPZ[TZ + g * RPT + qrow(h)];
         f4 q1, q2;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -1054,13 +1116,16 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) 
   using Q = Geo<G, RPT, C, S16>;
   __shared__ __attribute__((aligned(16))) float lds[Q::LDS + Q::LDS_D];
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];   // coefficient table (reduced radii near the edges)
-  const int t = xcd_tile(a.ntiles);
-  if (t < 0) return;
-  const Tile tl = a.tiles[t];
+  const int v = xcd_tile(a.ntiles * Q::SPLIT);
+  if (v < 0) return;
+  const int t = v / Q::SPLIT;
+  Tile tl = a.tiles[t];
   if (tl.slot < 0) return;                             // padding of a shorter XCD run
+  tl.z0 += v % Q::SPLIT * Q::TZ;
   const bool track = a.act && !(tl.kind & (TF_SRC | TF_REC));
   SkipWords sw{};
   if (track) sw = skip_words(a.act, a.ntiles, t, tl);
+  fetch_shot(a.shots, tl.slot);
   const ShotDev& s = shot_of(a.shots, tl.slot);
   const int it = s.it_off + s.it_dir * a.step;
   if (track && skip_of(sw, it)) {                      // the forward field is +0 around the tile
@@ -1096,13 +1161,15 @@ __global__ __launch_bounds__(64 * G) __attribute__((amdgpu_waves_per_eu(4, 8))) 
   __shared__ __attribute__((aligned(16))) float ctab[RTM_R * CTW];
   // XCD c's workgroups take its run of the table RGRP tiles at a time, their
   // receiver halves and then their reconstruction halves
-  const int per = (a.ntiles + 7) >> 3, b = blockIdx.x >> 3, r = b % (2 * RGRP);
+  const int n = a.ntiles * Q::SPLIT, per = (n + 7) >> 3, b = blockIdx.x >> 3, r = b % (2 * RGRP);
   const int i = b / (2 * RGRP) * RGRP + r % RGRP;
   if (i >= per) return;
-  const int t = (blockIdx.x & 7) * per + i;
-  if (t >= a.ntiles) return;
-  const Tile tl = a.tiles[t];
+  const int v = (blockIdx.x & 7) * per + i;
+  if (v >= n) return;
+  Tile tl = a.tiles[v / Q::SPLIT];
   if (tl.slot < 0) return;                             // padding of a shorter XCD run
+  tl.z0 += v % Q::SPLIT * Q::TZ;
+  fetch_shot(a.shots, tl.slot);
   const ShotDev& s = shot_of(a.shots, tl.slot);
   const int it = s.it_off + s.it_dir * a.step;
   const bool odd = it & 1;
@@ -2116,7 +2183,8 @@ static inline int grid8(int ntiles) { return ((ntiles + 7) / 8) * 8; }
 template <int G, int RPT>
 static hipError_t launch_step_t(const LaunchArgs& a, int phase, hipStream_t st)
 {
-  const dim3 b(64 * G), gf(grid8(a.ntiles)), gr(16 * (((a.ntiles + 7) / 8 + RGRP - 1) / RGRP * RGRP));
+  const int n = a.ntiles * Geo<G, RPT, false, false>::SPLIT;
+  const dim3 b(64 * G), gf(grid8(n)), gr(16 * (((n + 7) / 8 + RGRP - 1) / RGRP * RGRP));
   auto go = [&](auto cached, auto s16) {
     if (phase == PH_FWD) hipLaunchKernelGGL((k_fwd<G, RPT, cached.value, s16.value>), gf, b, 0, st, a);
     else hipLaunchKernelGGL((k_rev<G, RPT, cached.value, s16.value>), gr, b, 0, st, a);
@@ -2132,15 +2200,20 @@ hipError_t rtm_launch_step(const LaunchArgs& a, int phase, int tz, hipStream_t s
 {
   if (a.ntiles <= 0) return hipSuccess;
   switch (tz) {
-    // 16 rows are the height of the smallest launches.  Up to one and a half
-    // tiles per CU the time is a workgroup's own chain of phases, which 8
-    // waves of 2 rows shorten; past that the 4 x 4 form does less halo work a
-    // wave.  us per forward (with its strip save) / reverse step, 8 x 2
-    // against 4 x 4: one 184 x 124 window (24 tiles) 10.3 / 9.5 against 11.4 /
-    // 11.6, 480 x 280 (144) 11.5 / 12.5 against 12.6 / 13.0, 401 x 612 (273)
-    // 14.3 / 10.9 against 15.4 / 12.3, two of them (546) 15.9 / 18.2 against
-    // 16.0 / 15.1, four 24.4 / 29.9 against 22.2 / 24.9
-    case 16: return a.ntiles <= 384 ? launch_step_t<8, 2>(a, phase, st) : launch_step_t<4, 4>(a, phase, st);
+    // 16 rows are the height of the smallest launches, whose time is a
+    // workgroup's own chain of phases (about 6 of 8 us a step).  Up to one
+    // tile per CU two workgroups of 8 rows share a tile: a reverse step has two
+    // fields, so whole tiles leave some CUs with two workgroups and others idle.
+    // Up to one and a half, 8 waves of 2 rows; past that the 4 x 4 form does
+    // less halo work a wave.  us per forward / reverse step, halves against 8 x
+    // 2: one 184 x 124 window (24 tiles) 7.5 / 7.7 against 7.8 / 8.3, 480 x 280
+    // (144) 7.8 / 10.4 against 8.0 / 11.8, two of 265 x 320 a launch (200) 9.0 /
+    // 11.7 against 8.9 / 13.2, 401 x 612 (273) 8.6 / 11.2 against 8.4 / 10.7;
+    // 8 x 2 against 4 x 4 (with a strip save of its own): 273 tiles 14.3 /
+    // 10.9 against 15.4 / 12.3, 546 15.9 / 18.2 against 16.0 / 15.1
+    case 16:
+      if (a.ntiles <= 256) return launch_step_t<4, 2>(a, phase, st);
+      return a.ntiles <= 384 ? launch_step_t<8, 2>(a, phase, st) : launch_step_t<4, 4>(a, phase, st);
     case 32: return launch_step_t<4, 8>(a, phase, st);
     case 64: return launch_step_t<8, 8>(a, phase, st);
     default: return hipErrorInvalidValue;
