@@ -1512,8 +1512,8 @@ __global__ __launch_bounds__(NTHR) void k_gauss_smooth(const float* __restrict__
 // waves are for the comparison of the ring (512 threads: within 10 % at rings
 // in LDS, 15 % slower in memory; 256: 50 % slower).  One window with its
 // transfers, against every operand loaded when needed and shuffled through
-// LDS: 265 x 320, npml 32, 20.0 -> 8.4 ms; 401 x 612, npml 50, 55.5 -> 25.2;
-// 2148 x 1124, npml 50, 162 -> 76.
+// LDS: 265 x 320, npml 32, 20.0 -> 7.0 ms; 401 x 612, npml 50, 55.5 -> 24.8;
+// 2148 x 1124, npml 50, 162 -> 74.5.
 // Needs npml - 1 <= 64, nx, nz >= 3 npml (the mirrors read only interior
 // cells) and nx, nz <= RTM_SMOOTH_MAXN.
 #define RTM_SMOOTH_MAXN 4096
@@ -1522,38 +1522,51 @@ constexpr int SMT = 1024, SMOOTH_LDS = 40000;
 
 __device__ __forceinline__ float avg4(float a, float b, float c, float d) { return 0.25f * (((a + b) + c) + d); }
 
-// where the cells of the ring are: the full window in memory ...
+// Where the cells of the ring are (byte offsets).  A line of a front is a
+// column, at base + row * pitch, or a row, whose columns start at l, c and r in
+// the left layer, the centre and the right layer (less the column itself).
+struct RowAt { int l, c, r; };
+// the full window in memory ...
 struct RingMem {
+  typedef __attribute__((address_space(1))) char gchar;
   gfloat* p;
   int nx;
-  __device__ __forceinline__ int at(int r, int c) const { return r * nx + c; }
-  typedef __attribute__((address_space(1))) char gchar;
-  __device__ __forceinline__ gfloat* cell(int a) const { return (gfloat*)((gchar*)p + 4u * (unsigned)a); }
+  __device__ __forceinline__ gfloat* cell(int a) const { return (gfloat*)((gchar*)p + (unsigned)a); }
   __device__ __forceinline__ float get(int a) const { return *cell(a); }
   __device__ __forceinline__ void set(int a, float x) const { *cell(a) = x; }
-  // rows r0..r1 of a column are this far apart (0: not all the same)
-  __device__ __forceinline__ int row_step(int, int) const { return nx; }
+  __device__ __forceinline__ int pitch() const { return 4 * nx; }
+  __device__ __forceinline__ int column(int c) const { return 4 * c; }
+  __device__ __forceinline__ RowAt row(int r) const { return RowAt{4 * r * nx, 4 * r * nx, 4 * r * nx}; }
+  __device__ __forceinline__ int in_row(const RowAt& w, int c) const { return w.c + 4 * c; }
+  __device__ __forceinline__ bool straight(int, int) const { return true; }
+  __device__ __forceinline__ int at(int r, int c) const { return 4 * (r * nx + c); }
 };
-// ... or the ring and one line beside it (m = npml + 1 deep) in LDS: the top
-// m rows and the bottom m rows in full (even pitch), the rows between as
-// their first and last m columns
+// ... or the ring and one line beside it (m = npml + 1 deep) in LDS: the first
+// and last m columns of every row, 2 m to a row, then the centre columns of
+// the first and last m rows.  Both pitches are even, so that a front, whose
+// lanes are a pitch less one apart, meets every bank.
 typedef __attribute__((address_space(3))) float lds_float_t;
+typedef __attribute__((address_space(3))) char lds_char_t;
 struct RingLds {
   lds_float_t* p;
-  int nx, nz, m, P;
-  __device__ __forceinline__ int at(int r, int c) const
+  int nx, nz, m, P;                                    // P: pitch of the centre columns
+  __device__ __forceinline__ lds_float_t* cell(int a) const { return (lds_float_t*)((lds_char_t*)p + a); }
+  __device__ __forceinline__ float get(int a) const { return *cell(a); }
+  __device__ __forceinline__ void set(int a, float x) const { *cell(a) = x; }
+  __device__ __forceinline__ int pitch() const { return 8 * m; }
+  __device__ __forceinline__ int column(int c) const { return 4 * (c < m ? c : c - nx + 2 * m); }
+  __device__ __forceinline__ RowAt row(int r) const
   {
-    const int rows = imin(r, m) + imax(r - (nz - m), 0), mids = imin(imax(r - m, 0), nz - 2 * m);
-    const int narrow = c < m ? c : c - nx + 2 * m;
-    return rows * P + mids * 2 * m + ((r >= m) & (r < nz - m) ? narrow : c);
+    const int k = r < m ? r : r - nz + 2 * m;          // its place among the first and last m rows
+    return RowAt{8 * r * m, 4 * (2 * nz * m + k * P - m), 4 * (2 * r * m - nx + 2 * m)};
   }
-  __device__ __forceinline__ float get(int a) const { return p[a]; }
-  __device__ __forceinline__ void set(int a, float x) const { p[a] = x; }
-  __device__ __forceinline__ int row_step(int r0, int r1) const { return r0 >= m && r1 < nz - m ? 2 * m : 0; }
+  __device__ __forceinline__ int in_row(const RowAt& w, int c) const { return 4 * c + (c < m ? w.l : c < nx - m ? w.c : w.r); }
+  __device__ __forceinline__ bool straight(int c0, int c1) const { return c0 >= m && c1 < nx - m; }
+  __device__ __forceinline__ int at(int r, int c) const { return in_row(row(r), c); }
   static __device__ __forceinline__ int floats(int nx, int nz, int npml)
   {
-    const int m = npml + 1, P = (nx + 1) & ~1;
-    return 2 * m * P + (nz - 2 * m) * 2 * m;
+    const int m = npml + 1, P = (nx - 2 * m + 1) & ~1;
+    return 2 * m * (nz + P);
   }
 };
 
@@ -1584,41 +1597,45 @@ __device__ __forceinline__ void smooth_front(const A acc, int line0, int lanes, 
 {
   constexpr int FB = 8;
   const int t = threadIdx.x & 63;
-  const int tl = imin(t, lanes), line = line0 + tl;
+  const int tl = imin(t, lanes);
   const bool real = t < lanes;
-  auto at = [&](int ln, int pos) {
+  // a line's place, and the address of a position (0..len+1) on it
+  struct Line { int base; RowAt row; };
+  auto line_of = [&](int ln) { return LR ? Line{acc.column(ln), RowAt{}} : Line{0, acc.row(ln)}; };
+  auto at = [&](const Line& ln, int pos) {
     const int q = imin(imax(pos, 0), len + 1);
-    return LR ? acc.at(q, ln) : acc.at(ln, q);
+    return LR ? ln.base + q * acc.pitch() : acc.in_row(ln.row, q);
   };
+  const Line own = line_of(line0 + tl), before = line_of(line0 - 1), beside = line_of(line0 + lanes);
   // operands of the steps k0 .. k0+FB-1: own line at 2 + k - t, the line
   // before lane 0's at 1 + k, the line after the last one's at 2 + k - lanes;
   // ad: the own line's addresses, the positions updated one step later
   struct Block { float v[FB], first[FB], last[FB]; int ad[FB]; };
   auto read = [&](int k0, Block& b) {
-    const int lo = 2 + k0 - lanes, hi = 1 + k0 + FB;
-    const int step = lo >= 0 && hi <= len + 1 ? (LR ? acc.row_step(lo, hi) : 1) : 0;
-    if (step) {
-      const int a = at(line, 2 + k0 - tl), f = at(line0 - 1, 1 + k0);
+    const int lo = 2 + k0 - lanes, hi = 1 + k0 + FB;   // positions of all lanes
+    if (lo >= 0 && hi <= len + 1 && (LR || acc.straight(lo, hi))) {
+      const int step = LR ? acc.pitch() : 4;
+      const int a = at(own, 2 + k0 - tl), f = at(before, 1 + k0);
 #pragma unroll
       for (int u = 0; u < FB; u++) {
-        b.ad[u] = LR ? a + u * step : a + u;
-        b.first[u] = acc.get(LR ? f + u * step : f + u);
+        b.ad[u] = LR ? a + u * step : a + 4 * u;
+        b.first[u] = acc.get(LR ? f + u * step : f + 4 * u);
       }
     } else {
 #pragma unroll
       for (int u = 0; u < FB; u++) {
-        b.ad[u] = at(line, 2 + k0 + u - tl);
-        b.first[u] = acc.get(at(line0 - 1, 1 + k0 + u));
+        b.ad[u] = at(own, 2 + k0 + u - tl);
+        b.first[u] = acc.get(at(before, 1 + k0 + u));
       }
     }
 #pragma unroll
     for (int u = 0; u < FB; u++) b.v[u] = acc.get(b.ad[u]);
     if (FULL)
 #pragma unroll
-      for (int u = 0; u < FB; u++) b.last[u] = acc.get(at(line0 + lanes, 2 + k0 + u - lanes));
+      for (int u = 0; u < FB; u++) b.last[u] = acc.get(at(beside, 2 + k0 + u - lanes));
   };
-  int ab = at(line, 1 - t);                            // address of the position a lane updates
-  float prev = acc.get(at(line, 0));
+  int ab = at(own, 1 - t);                             // address of the position a lane updates
+  float prev = acc.get(at(own, 0));
   const int K = len + lanes - 1;
   auto steps = [&](int k0, const Block& cur) {
     float after[FB];
@@ -1850,14 +1867,13 @@ __global__ __launch_bounds__(SMT) void k_pml_smooth(const SmoothWin* __restrict_
   lds_float_t* L = (lds_float_t*)S;
   const int rf = RingLds::floats(nx, nz, npml);
   if (rf + 2 * (nx + nz) <= SMOOTH_LDS && npml <= 64) {
-    const RingLds acc{L, nx, nz, npml + 1, (nx + 1) & ~1};
     const int m = npml + 1;
+    const RingLds acc{L, nx, nz, m, (nx - 2 * m + 1) & ~1};
     for (int e = tid; e < nx * nz; e += SMT) {
       const int r = e / nx, c = e - r * nx;
       if (r < m || r >= nz - m || c < m || c >= nx - m) acc.set(acc.at(r, c), w[e]);
     }
-    if (tid < 2 * m && acc.P > nx)                     // the pad of the full rows
-      L[(tid < m ? tid : tid - m) * acc.P + (tid < m ? 0 : m * acc.P + (nz - 2 * m) * 2 * m) + nx] = 1.0f;
+    if (tid < 2 * m && acc.P > nx - 2 * m) L[2 * nz * m + tid * acc.P + nx - 2 * m] = 1.0f;   // the centre's pad
     __syncthreads();
     OldLds old{L, rf};
     smooth_sweeps<false>(acc, old, L + rf, red, nx, nz, npml);
