@@ -873,7 +873,7 @@ std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int ph
 
 int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt, rtmh_stats* prof, bool skip)
 {
-  // every step kernel (and the strip save after it) bracketed by its own
+  // every step kernel (and what follows it in the step) bracketed by its own
   // event pair on the launch stream
   const Lane& L = lane_[0];
   const int ntiles = (int)g.tiles.size(), nslots = (int)g.slots.size();

@@ -170,14 +170,14 @@ struct SlotMem {
 };
 
 // Everything a captured chunk bakes in by value: the launch shapes (tiles,
-// tile height, slots: k_save's and k_ic's grids and k_bump's count), the
+// tile height, slots: k_quant16's and k_ic's grids and k_bump's count), the
 // kernels chosen (phase, store format, imaging conditions, guard) and the
 // control-block addresses.  Descriptors and tiles are read from the control
 // block at replay, so batches that agree on all of these share a graph.
 struct GraphKey {
-  int ntiles, tz, phase, save, fmt, k;     // save: strip save after every (forward) step, fmt its store format
+  int ntiles, tz, phase, save, fmt, k;     // save: a forward step keeps its strips, fmt their store format
   int ic;                                  // cells of the other imaging conditions after every reverse step (0: off)
-  int nslots;                              // slots of the batch (k_save / k_ic grids, k_bump count)
+  int nslots;                              // slots of the batch (k_quant16 / k_ic grids, k_bump count)
   int guard;                               // wavefield guard after the chunk
   int snap;                                // snapshot launches after every step: 0 off, else 1 + format
   int skip;                                // zero-tile skip of the step kernels

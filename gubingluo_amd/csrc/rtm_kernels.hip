@@ -18,11 +18,12 @@
 //
 // LDS: the pressure of the tile and its halo (columns x0-20..x0+83 of the
 // tile rows, rows z0-19..z0+TZ+18 of the tile columns), then -- reusing the
-// same bytes -- the new velocities (vx: columns x0-10..x0+73; vz: rows
-// z0-10..z0+TZ+8).  x-derivatives read LDS rows; z-derivatives read a
-// register window of the thread's own column.  The reverse step runs the
-// source reconstruction and then the receiver wavefield through the same
-// LDS; the imaging products use the reconstructed pressure from registers.
+// same bytes -- the new velocities (vx: columns x0-12..x0+75; vz: rows
+// z0-10..z0+TZ+8).  x-derivatives are taken four columns a lane from 16-byte
+// LDS reads, z-derivatives from a register window of a lane's column.  In the
+// reverse step a tile's receiver field and its source reconstruction are two
+// workgroups; the reconstruction adds the imaging products of the step
+// before, whose pressures both fields still read.
 //
 // Arithmetic follows the reference operation order with explicit fused
 // multiply-adds (the oracle's canonical FP32 form), so every cell matches the

@@ -12,8 +12,8 @@ hipError_t rtm_launch_clock(long long* t, long long ticks, hipStream_t st);
 // after the last reverse step `it` of the listed slots: its imaging products
 // (every other reverse step's are added by the step after it)
 hipError_t rtm_launch_image(const ShotDev* shots, const int* slots, int nslots, int it, hipStream_t st);
-// after a forward step with LaunchArgs::save = 2: its boundary strips into the
-// 16-bit store of the listed slots, with a scale per block
+// after a forward step with LaunchArgs::save and s16: its boundary strips into
+// the 16-bit store of the listed slots, with a scale per block
 hipError_t rtm_launch_quant16(const ShotDev* shots, const int* slots, int nslots, int step, hipStream_t st);
 hipError_t rtm_launch_phase_init(const ShotDev* shots, int slot, int phase, int nblocks, hipStream_t st);
 // 1/rho and rho v^2 of n model cells (ib = 1/rho, kk = rho v^2, each rounded once)

@@ -171,8 +171,8 @@ typedef struct rtmh_stats {
   double cell_updates;      /* 2*nt*nxp*nzp + (nt-1)*nz*nxl summed over shots     */
   int nshots, batches, tile_z, batch;
   double hbm_bytes_alg;     /* algorithmic bytes of the propagation passes        */
-  /* profile=1 only: per kernel (0 forward step, 1 strip save after it,
-   * 2 reverse step, 3 unused) summed launch time and launch count */
+  /* profile=1 only: per kernel (0 forward step, 1 what follows it: the 16-bit
+   * store's quantisation and snapshots, 2 reverse step, 3 unused) summed launch time and launch count */
   double kern_ms[4];
   int kern_calls[4];
   double step_bytes_fwd;    /* algorithmic bytes of one forward step of the batch */
