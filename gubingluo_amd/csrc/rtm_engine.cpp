@@ -847,7 +847,7 @@ std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int ph
   int n = 1;
   if (nb > 1) {
     n = 2;
-    if (most <= half && phase == PH_REV) n = 2 * std::max(1, (int)std::ceil(total / kCacheBytes));
+    if (most <= half && phase == PH_REV && total > kPairBytes) n = 2 * (int)std::ceil(total / kCacheBytes);
     n = std::min(n, nb);
   }
   std::vector<std::vector<int>> g(n);

@@ -323,19 +323,29 @@ class Engine {
 // groups in flight (two at a time) fit the 256 MB Infinity Cache.  Two lanes
 // in turn fill each other's launch tails, and in the reverse pass a group's
 // fields stay in the cache from step to step: a reverse step works on
-// `live_bytes` of a slot, a group takes at most half of kCacheBytes of them,
-// groups are of about equal size and even in number, so that both lanes are
-// busy to the end.  A forward pass, and shots too large for that, run as two
-// halves: a forward launch of few shots is short while the wavefield is still
-// small and its fixed costs then weigh more than the cache gives.  Measured,
-// ms of the forward and the reverse pass as one group / two halves / cached
-// groups: 48 survey shots (nt 3000) 260, 555 / 222, - / 245, 437; 160 (nt
-// 1000) 174, 638 / 160, - / 201, 531; 16 ragged windows of 400-1600 columns
-// 38, 176 / 34, - / 50, 155; 4 shots of 2148 x 1124 (nt 1200) 52, 194 / 51,
-// 187 / 95, -.
-// The bound itself, ms of 48 survey shots / 16 with every imaging condition at
-// 200, 235, 270 and 320 MB: 674 / 104, 674 / 101, 675 / 101, 772 / 100.
-constexpr double kCacheBytes = 235e6;
+// `live_bytes` of a slot, and a batch is cut into an even number of groups (or
+// one a shot) of about equal size, so that two of them hold kCacheBytes or
+// less; a cut falls between shots, so that a pair may hold one shot more.
+// `cached` allows a pair 15 % over the bound (230 MB).  A forward pass, and
+// shots larger than half the bound, run as two halves: a forward launch of few
+// shots is short while the wavefield is still small and its fixed costs then
+// weigh more than the cache gives.  Measured, ms of the forward and the
+// reverse pass as one group / two halves / cached groups: 48 survey shots (nt
+// 3000) 260, 555 / 222, - / 245, 437; 160 (nt 1000) 174, 638 / 160, - / 201,
+// 531; 16 ragged windows of 400-1600 columns 38, 176 / 34, - / 50, 155; 4
+// shots of 2148 x 1124 (nt 1200) 52, 194 / 51, 187 / 95, -.
+// The bound: strips, model and images come on top of the fields.  us per
+// reverse step of survey shots at 200 / 235 MB where the plans differ, their
+// largest pairs in brackets: 32 shots 108 (151 MB) / 111 (220), 34 113 (165) /
+// 126 (234), 64 210 (179) / 225 (220), 100 333 (206) / 370 (234), 160 529
+// (206) / 555 (220), 200 644 (193) / 682 (224).
+// A batch that is one pair keeps a little more, since nothing else goes
+// through the cache and four groups would be launches of half the size.  us
+// per reverse step as two groups / as four, 13.7 MB survey shots and others:
+// 206 MB 52 / 56, 214 MB 66 / 67, 216 MB 54 / 58, 220 MB 57 / 56, 227 MB 75 /
+// 71, 234 MB 66 / 62; with every imaging condition 206 MB 76 / 83, 220 MB 80 /
+// 86, 234 MB 85 / 91.
+constexpr double kCacheBytes = 200e6, kPairBytes = 225e6;
 double live_bytes(const ShotDev& d, int phase);
 std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int phase, bool& cached);
 

@@ -1,0 +1,107 @@
+// host_plan.cpp -- CPU checks of how a pass is cut into groups of shots
+// (rtm::plan_groups), over batches of equal, growing and random windows.
+// Built and run by tests/test_host_plan.py; prints one line per check and
+// exits non-zero if one fails.
+#include <stdio.h>
+#include <string.h>
+
+#include <algorithm>
+#include <random>
+#include <vector>
+
+#include "rtm_engine.h"
+
+static int g_fail = 0;
+#define CHECK(c, ...)                                                  \
+  do {                                                                 \
+    if (!(c)) {                                                        \
+      printf("FAIL %s:%d: %s -- ", __FILE__, __LINE__, #c);            \
+      printf(__VA_ARGS__);                                             \
+      printf("\n");                                                    \
+      g_fail = 1;                                                      \
+    }                                                                  \
+  } while (0)
+
+static ShotDev window(int nxl, int nzi, int npml)
+{
+  ShotDev d;
+  memset(&d, 0, sizeof(d));
+  d.nxl = nxl; d.nzi = nzi; d.npml = npml;
+  d.nxp = nxl + 2 * npml; d.nzp = nzi + 2 * npml;
+  return d;
+}
+
+struct Plan { std::vector<std::vector<int>> g; bool cached; double total = 0, most = 0, pair = 0; };
+static Plan plan(const std::vector<ShotDev>& ds, int phase)
+{
+  Plan p;
+  p.g = rtm::plan_groups(ds, phase, p.cached);
+  double prev = 0;
+  for (auto& v : p.g) {
+    double b = 0;
+    for (int j : v) {
+      const double x = rtm::live_bytes(ds[j], phase);
+      b += x;
+      p.most = std::max(p.most, x);
+    }
+    p.total += b;
+    p.pair = std::max(p.pair, prev + b);
+    prev = b;
+  }
+  return p;
+}
+
+// every shot once and in order, no empty group
+static bool whole(const Plan& p, int n)
+{
+  int at = 0;
+  for (auto& v : p.g) {
+    if (v.empty()) return false;
+    for (int j : v)
+      if (j != at++) return false;
+  }
+  return at == n;
+}
+
+// the reverse pass: two neighbouring groups hold at most 200 MB and one shot
+// (the cuts fall between shots), or are the whole pass and hold at most 225 MB
+static void reverse_bound(const char* name, const std::vector<ShotDev>& ds)
+{
+  const Plan p = plan(ds, PH_REV);
+  const int nb = (int)ds.size(), n = (int)p.g.size();
+  CHECK(whole(p, nb), "%s: %d shots, %d groups", name, nb, n);
+  CHECK(nb == 1 ? n == 1 : n % 2 == 0 || n == nb, "%s: %d groups of %d shots", name, n, nb);
+  if (p.most <= 100e6) {
+    const double bound = n == 2 && p.total <= 225e6 ? 225e6 : 200e6 + p.most;
+    CHECK(p.pair <= bound, "%s: %d shots in %d groups, a pair holds %.0f MB of at most %.0f", name, nb, n, p.pair / 1e6,
+          bound / 1e6);
+  } else {
+    CHECK(n == std::min(2, nb), "%s: %d groups of large shots", name, n);
+  }
+  // 256 MB of cache
+  CHECK(!p.cached || p.pair <= 230e6, "%s: %d shots count as cached with %.0f MB", name, nb, p.pair / 1e6);
+  CHECK(p.cached || p.pair > 225e6, "%s: %d shots do not count as cached with %.0f MB", name, nb, p.pair / 1e6);
+}
+
+int main()
+{
+  for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
+    reverse_bound("survey", std::vector<ShotDev>(n, window(301, 512, 50)));
+  for (int n : {5, 31, 33, 70, 119}) reverse_bound("narrow", std::vector<ShotDev>(n, window(60 + n, 300, 32)));
+  for (int n : {2, 3, 4, 9}) reverse_bound("wide", std::vector<ShotDev>(n, window(1200, 768, 50)));
+  for (int n : {1, 2, 4, 5}) reverse_bound("large", std::vector<ShotDev>(n, window(2048, 1024, 50)));
+  std::mt19937 rng(7);
+  for (int k = 0; k < 300; k++) {
+    std::vector<ShotDev> ds;
+    const int n = 1 + rng() % 120, nz = 60 + rng() % 700;
+    for (int j = 0; j < n; j++) ds.push_back(window(40 + rng() % 900, nz, 32));
+    const Plan p = plan(ds, PH_REV);
+    CHECK(whole(p, n), "random %d: %d shots", k, n);
+    const Plan f = plan(ds, PH_FWD);
+    CHECK(whole(f, n) && (int)f.g.size() == std::min(2, n), "random %d: forward in %d groups", k, (int)f.g.size());
+    reverse_bound("random", ds);
+  }
+  printf("ok groups of a pass\n");
+  if (!g_fail) printf("all plan checks passed\n");
+  return g_fail;
+}
