@@ -1274,26 +1274,46 @@ int Engine::run(const rtmh_params& P, const float* vp0, const float* rho0, const
 // entries) large enough; graphs captured against the old block are dropped
 int Engine::ensure_cb(int nslots, size_t ntiles)
 {
-  if (nslots <= cb_slots_ && ntiles <= cb_tiles_) return 0;
+  if (cb_ && nslots <= cb_slots_ && ntiles <= cb_tiles_) return 0;
   drop_graphs();
+  const int ns = std::max(64, std::max(nslots, cb_slots_));
+  const size_t nt = ntiles > cb_tiles_ ? ntiles * 2 : cb_tiles_;
+  // the old block goes back before the new one is taken; until that is there
+  // the engine has none (a job that cannot get it leaves nothing to launch on)
   if (cb_) (void)hipFree(cb_);
   cb_ = nullptr;
-  cb_slots_ = nslots > cb_slots_ ? nslots : cb_slots_;
-  if (cb_slots_ < 64) cb_slots_ = 64;
-  cb_tiles_ = ntiles > cb_tiles_ ? ntiles * 2 : cb_tiles_;
+  cb_slots_ = 0;
+  cb_tiles_ = 0;
+  d_ds_ = nullptr;
+  d_tiles_ = nullptr;
+  d_slots_ = nullptr;
+  d_stk_ = nullptr;
+  d_flag_ = nullptr;
+  for (auto& l : lane_) { l.tiles = nullptr; l.slots = nullptr; l.act = nullptr; }
   // descriptors | the batch's tile tables, slot lists, stack entries | guard
   // flag | per lane: table, slot list, skip words
-  const size_t bt = align256(cb_tiles_ * sizeof(Tile)), bs = align256(cb_slots_ * 4),
-               ba = align256(2 * cb_tiles_ * sizeof(unsigned long long));
-  const size_t bytes = align256(cb_slots_ * sizeof(ShotDev)) + bt + bs + align256(cb_slots_ * sizeof(StackShotHost)) + 256 +
-                       kLanes * (bt + bs + ba);
-  HIPCHK(hipMalloc(&cb_, bytes));
+  const size_t bd = align256(ns * sizeof(ShotDev)), bt = align256(nt * sizeof(Tile)), bs = align256((size_t)ns * 4),
+               bk = align256(ns * sizeof(StackShotHost)), ba = align256(2 * nt * sizeof(unsigned long long));
+  const size_t bytes = bd + bt + bs + bk + 256 + kLanes * (bt + bs + ba);
+  void* mem = nullptr;
+  if (hipMalloc(&mem, bytes) != hipSuccess) {
+    pool_.trim();                                      // memory that earlier jobs left cached
+    if (hipMalloc(&mem, bytes) != hipSuccess) {
+      (void)hipGetLastError();                         // reported here, not by the next launch
+      set_error("out of device memory (control block)");
+      return -3;
+    }
+    (void)hipGetLastError();
+  }
+  cb_ = mem;
+  cb_slots_ = ns;
+  cb_tiles_ = nt;
   char* p = (char*)cb_;
   auto take = [&](size_t n) { char* q = p; p += n; return q; };
-  d_ds_ = (ShotDev*)take(align256(cb_slots_ * sizeof(ShotDev)));
+  d_ds_ = (ShotDev*)take(bd);
   d_tiles_ = (Tile*)take(bt);
   d_slots_ = (int*)take(bs);
-  d_stk_ = (StackShotHost*)take(align256(cb_slots_ * sizeof(StackShotHost)));
+  d_stk_ = (StackShotHost*)take(bk);
   d_flag_ = (unsigned int*)take(256);
   for (auto& l : lane_) {
     l.tiles = (Tile*)take(bt);

@@ -1,15 +1,25 @@
-// host_plan.cpp -- CPU checks of how a pass is cut into groups of shots
-// (rtm::plan_groups), over batches of equal, growing and random windows.
+// host_plan.cpp -- CPU checks of how the engine plans and prepares a pass: how
+// it is cut into groups of shots (rtm::plan_groups), over batches of equal,
+// growing and random windows, and the control block whose allocation fails.
 // Built and run by tests/test_host_plan.py; prints one line per check and
 // exits non-zero if one fails.
 #include <stdio.h>
 #include <string.h>
 
 #include <algorithm>
+#include <condition_variable>
+#include <functional>
+#include <map>
+#include <mutex>
 #include <random>
+#include <string>
 #include <vector>
 
+#include <hip/hip_runtime.h>
+
+#define private public   // the engine's control block
 #include "rtm_engine.h"
+#undef private
 
 static int g_fail = 0;
 #define CHECK(c, ...)                                                  \
@@ -83,8 +93,27 @@ static void reverse_bound(const char* name, const std::vector<ShotDev>& ds)
   CHECK(p.cached || p.pair > 225e6, "%s: %d shots do not count as cached with %.0f MB", name, nb, p.pair / 1e6);
 }
 
+// A control block that cannot be allocated (here: there is no GPU) is not
+// counted as there by the next job, which would launch on its addresses; with
+// a GPU both calls succeed.
+static void control_block()
+{
+  rtm::Engine e(0);
+  const int gpus = [] { int n = 0; return hipGetDeviceCount(&n) == hipSuccess ? n : 0; }();
+  for (int call = 0; call < 3; call++) {
+    const int rc = e.ensure_cb(10, 100 + 10 * (call == 2));
+    CHECK((rc == 0) == (gpus > 0), "call %d returns %d with %d GPUs", call, rc, gpus);
+    CHECK((rc == 0) == (e.cb_ != nullptr), "call %d returns %d, block %p", call, rc, e.cb_);
+    CHECK(e.cb_ || (!e.d_ds_ && !e.d_tiles_ && !e.d_slots_ && !e.d_stk_ && !e.d_flag_ && !e.lane_[0].tiles &&
+                    !e.lane_[1].act), "call %d leaves addresses of no block", call);
+    CHECK(hipGetLastError() != hipErrorOutOfMemory, "call %d leaves its error for the next launch", call);
+  }
+  printf("ok control block\n");
+}
+
 int main()
 {
+  control_block();
   for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
     reverse_bound("survey", std::vector<ShotDev>(n, window(301, 512, 50)));
   for (int n : {5, 31, 33, 70, 119}) reverse_bound("narrow", std::vector<ShotDev>(n, window(60 + n, 300, 32)));

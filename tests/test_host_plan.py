@@ -1,4 +1,4 @@
-"""How a pass is cut into groups of shots, on the CPU: a small C++ program
+"""How the engine plans and prepares a pass, on the CPU: a small C++ program
 (tests/host_plan.cpp) linked against the library."""
 import os
 import subprocess
