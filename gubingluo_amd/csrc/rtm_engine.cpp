@@ -623,8 +623,10 @@ Engine::Engine(int device) : device_(device)
 {
   (void)hipSetDevice(device_);
   (void)hipStreamCreateWithFlags(&lane_[0].st, hipStreamNonBlocking);
-  lane_[1].st = stream_beside(lane_[0].st);
   st_ = lane_[0].st;
+  // without a second stream (or a first: st_ is then the default one, which
+  // cannot be captured beside) every batch runs as one group
+  if (st_ && (lane_[1].st = stream_beside(st_))) nlanes_ = kLanes;
 }
 
 Engine::~Engine()
@@ -871,6 +873,21 @@ std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int ph
   return g;
 }
 
+std::vector<Engine::Group> Engine::groups_of(const std::vector<ShotDev>& ds, int phase, bool timed, bool& cached) const
+{
+  std::vector<std::vector<int>> v;
+  if (timed || nlanes_ < kLanes) {
+    v.resize(1);
+    for (int j = 0; j < (int)ds.size(); j++) v[0].push_back(j);
+    cached = false;
+  } else {
+    v = plan_groups(ds, phase, cached);
+  }
+  std::vector<Group> g(v.size());
+  for (size_t i = 0; i < v.size(); i++) g[i].slots = std::move(v[i]);
+  return g;
+}
+
 int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt, rtmh_stats* prof, bool skip)
 {
   // every step kernel (and what follows it in the step) bracketed by its own
@@ -931,7 +948,7 @@ int Engine::run_pass(int phase, int nsteps, std::vector<Group>& groups, int tz, 
     int left = 0, step = 0;                            // steps left of the group; plain steps taken since its last chunk
     hipGraphExec_t ex = nullptr;
   } run[kLanes];
-  const int nl = std::min<int>(kLanes, (int)groups.size());
+  const int nl = std::min(nlanes_, (int)groups.size());
   hipEvent_t ev;
   HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc = 0;
@@ -1486,20 +1503,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
     // at most 1.25 x the even share)
     const bool prof = opt.profile && stats;
     bool cached_f = false, cached_r = false;
-    auto plan = [&](int phase, bool& cached) {
-      std::vector<std::vector<int>> v;
-      if (prof) {
-        v.resize(1);
-        for (int j = 0; j < nb; j++) v[0].push_back(j);
-        cached = false;
-      } else {
-        v = plan_groups(ds, phase, cached);
-      }
-      std::vector<Group> g(v.size());
-      for (size_t i = 0; i < v.size(); i++) g[i].slots = v[i];
-      return g;
-    };
-    std::vector<Group> gf = plan(PH_FWD, cached_f), gr = plan(PH_REV, cached_r);
+    std::vector<Group> gf = groups_of(ds, PH_FWD, prof, cached_f), gr = groups_of(ds, PH_REV, prof, cached_r);
     // tile height of a pass: given, or by the 32-row tiles of the groups in
     // flight.  Few tiles: 16 rows, whose workgroups' chains are the shortest;
     // from 1000 forward, 1400 reverse, 32 rows, which do less halo work a cell

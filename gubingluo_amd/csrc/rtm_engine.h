@@ -275,6 +275,7 @@ class Engine {
   };
   static constexpr int kLanes = 2;
   Lane lane_[kLanes];
+  int nlanes_ = 1;                      // lanes that have a stream of their own
   std::vector<Tile> stage_tiles_;       // host copies of a pass's uploads (kept until the next pass)
   std::vector<int> stage_slots_;
   // the shots of one group: indices into the batch, its tile table, its place
@@ -302,6 +303,9 @@ class Engine {
   SnapPlan snap_;                       // snapshots of the running job
   int ensure_cb(int nslots, size_t ntiles);
 
+  // the groups a batch runs in (plan_groups); one group of all where there is
+  // one lane only or every launch is timed by itself
+  std::vector<Group> groups_of(const std::vector<ShotDev>& ds, int phase, bool timed, bool& cached) const;
   // All steps of a pass on every group, the groups dealt to the lanes in
   // turn.  guard_every > 0: the wavefield guard after every guard_every steps
   // (plain launches) or after every replayed chunk, and after the last step.

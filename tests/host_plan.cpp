@@ -1,6 +1,7 @@
 // host_plan.cpp -- CPU checks of how the engine plans and prepares a pass: how
 // it is cut into groups of shots (rtm::plan_groups), over batches of equal,
-// growing and random windows, and the control block whose allocation fails.
+// growing and random windows, how with one stream only, and the control block
+// whose allocation fails.
 // Built and run by tests/test_host_plan.py; prints one line per check and
 // exits non-zero if one fails.
 #include <stdio.h>
@@ -111,8 +112,27 @@ static void control_block()
   printf("ok control block\n");
 }
 
+// without a second stream (here: there is no GPU) a batch is one group on the
+// engine's own: a lane of its own would be the default stream
+static void one_lane()
+{
+  rtm::Engine e(0);
+  const std::vector<ShotDev> ds(40, window(301, 512, 50));
+  for (int phase : {PH_FWD, PH_REV}) {
+    bool cached = true;
+    const size_t n = e.groups_of(ds, phase, false, cached).size();
+    CHECK((n == 1) == (e.lane_[0].st == nullptr || e.lane_[1].st == nullptr), "%zu groups with streams %p, %p", n,
+          (void*)e.lane_[0].st, (void*)e.lane_[1].st);
+    CHECK(n > 1 || !cached, "phase %d: all shots at once count as cached", phase);
+    const auto t = e.groups_of(ds, phase, true, cached);
+    CHECK(t.size() == 1 && t[0].slots.size() == 40 && !cached, "timed launches in %zu groups", t.size());
+  }
+  printf("ok one lane\n");
+}
+
 int main()
 {
+  one_lane();
   control_block();
   for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
     reverse_bound("survey", std::vector<ShotDev>(n, window(301, 512, 50)));
