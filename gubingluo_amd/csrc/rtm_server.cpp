@@ -790,15 +790,18 @@ void Server::loop()
       if (L.ntf > 0) {
         a.save = 1;
         if (rtm_launch_step(a, PH_FWD, opt_.tile_z, st) != hipSuccess) fail("forward launch", hipGetLastError());
-        if (opt_.store_fmt != ST_F32) (void)rtm_launch_quant16(d_ds_, d_qs_ + L.qs, L.nq, (int)tick_, st);
-        launches_ += 2;
+        launches_ += 1;
+        if (opt_.store_fmt != ST_F32) {
+          (void)rtm_launch_quant16(d_ds_, d_qs_ + L.qs, L.nq, (int)tick_, st);
+          launches_ += 1;
+        }
       }
       if (L.ntr > 0) {
         a.save = 0;
         a.tiles = d_tiles_ + L.tr;
         a.ntiles = L.ntr;
         if (rtm_launch_step(a, PH_REV, opt_.tile_z, st) != hipSuccess) fail("reverse launch", hipGetLastError());
-        launches_ += 2;
+        launches_ += 1;
       }
     }
     // wavefield guard of every resident shot (the shots' own ntsnap differ;

@@ -376,7 +376,8 @@ int rtmh_server_request_bytes(rtmh_server *srv, int model_id, const rtmh_params 
  * the request failed (-3 memory, -7 its wavefield blew up), or the server did */
 int rtmh_server_wait(rtmh_server *srv, int request_id, double timeout_s, rtmh_outputs *out,
                      rtmh_request_stats *stats);
-/* server-wide counters: ticks, launches, peak resident shots, busy seconds,
+/* server-wide counters: ticks, launches (the ticks' steps and the 16-bit
+ * store's quantisation after a forward one), peak resident shots, busy seconds,
  * the HBM budget the server admits against (bytes), and the device
  * allocations it made (count, host seconds in hipMalloc/hipFree; 1 and the
  * time of the reservation when the budget was taken at start) */
