@@ -645,8 +645,22 @@ Engine::~Engine()
 
 void Engine::drop_graphs()
 {
-  for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : graphs_) (void)hipGraphExecDestroy(kv.second.ex);
   graphs_.clear();
+}
+
+void Engine::trim_graphs()
+{
+  if (graphs_.size() <= kMaxGraphs) return;
+  std::vector<unsigned long long> used;
+  for (auto& kv : graphs_) used.push_back(kv.second.used);
+  auto oldest_kept = used.end() - kMaxGraphs;          // (every use has a time of its own)
+  std::nth_element(used.begin(), oldest_kept, used.end());
+  for (auto it = graphs_.begin(); it != graphs_.end();) {
+    if (it->second.used >= *oldest_kept) { ++it; continue; }
+    (void)hipGraphExecDestroy(it->second.ex);
+    it = graphs_.erase(it);
+  }
 }
 
 static size_t store_elem(int fmt) { return fmt == ST_F32 ? 4 : 2; }
@@ -806,7 +820,10 @@ static void keep_strips(LaunchArgs& a, int fmt) { a.save = 1; a.s16 = fmt != ST_
 hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
 {
   auto it = graphs_.find(k);
-  if (it != graphs_.end()) return it->second;
+  if (it != graphs_.end()) {
+    it->second.used = ++graph_clock_;
+    return it->second.ex;
+  }
   hipGraph_t g = nullptr;
   if (hipStreamBeginCapture(L.st, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
   LaunchArgs a{d_ds_, L.tiles, k.ntiles, 0};
@@ -824,7 +841,7 @@ hipGraphExec_t Engine::graph_for(const GraphKey& k, const Lane& L)
   hipGraphExec_t ex = nullptr;
   if (hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) != hipSuccess) ex = nullptr;
   (void)hipGraphDestroy(g);
-  if (ex) graphs_[k] = ex;
+  if (ex) graphs_[k] = Graph{ex, ++graph_clock_};
   return ex;
 }
 
@@ -1540,6 +1557,7 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
       }
     };
     if (ensure_cb(nb, tcap) != 0) { for (void* p : mem) pool_.put(p); rc = -3; break; }
+    trim_graphs();                                     // (the passes before this batch have ended, also failed ones)
     ShotDev* d_ds = d_ds_;
     StackShotHost* d_stk = d_stk_;
     for (auto& u : uploads) HIPCHK(hipMemcpyAsync(u.first, u.second.data(), u.second.size(), hipMemcpyHostToDevice, st_));

@@ -286,7 +286,13 @@ class Engine {
     size_t tile0 = 0, slot0 = 0;
   };
   DevPool pool_;
-  std::map<GraphKey, hipGraphExec_t> graphs_;
+  // captured chunks, kept for the batches after this one: the kMaxGraphs used
+  // last.  A batch takes one for each pass and group shape (2 to about 30); a
+  // process with varied jobs would otherwise keep every shape it ever ran
+  static constexpr size_t kMaxGraphs = 128;
+  struct Graph { hipGraphExec_t ex = nullptr; unsigned long long used = 0; };
+  std::map<GraphKey, Graph> graphs_;
+  unsigned long long graph_clock_ = 0;
   std::map<int, Model> models_;
   mutable std::mutex models_mu_;
   int next_model_ = 1;
@@ -321,6 +327,8 @@ class Engine {
   int guard_check(const std::vector<ShotDev>& ds, const std::vector<int>& shots, int k0, const char* pass);
   hipGraphExec_t graph_for(const GraphKey& k, const Lane& L);
   void drop_graphs();
+  // back to kMaxGraphs, the longest unused ones first; no replay may be running
+  void trim_graphs();
 };
 
 // Groups of consecutive slots that a pass steps together, and whether the

@@ -1,7 +1,7 @@
 // host_plan.cpp -- CPU checks of how the engine plans and prepares a pass: how
 // it is cut into groups of shots (rtm::plan_groups), over batches of equal,
-// growing and random windows, how with one stream only, and the control block
-// whose allocation fails.
+// growing and random windows, how with one stream only, the control block
+// whose allocation fails, and the bound of the captured chunks that are kept.
 // Built and run by tests/test_host_plan.py; prints one line per check and
 // exits non-zero if one fails.
 #include <stdio.h>
@@ -130,8 +130,36 @@ static void one_lane()
   printf("ok one lane\n");
 }
 
+// the captured chunks that an engine keeps are bounded, the longest unused go
+// first (the entries here hold no graph)
+static void kept_graphs()
+{
+  rtm::Engine e(0);
+  const int cap = (int)rtm::Engine::kMaxGraphs, n = 3 * cap;
+  auto key = [](int i) {
+    rtm::GraphKey k;
+    memset(&k, 0, sizeof(k));
+    k.ntiles = i;
+    return k;
+  };
+  for (int i = 0; i < cap; i++) e.graphs_[key(i)] = {nullptr, ++e.graph_clock_};
+  e.trim_graphs();
+  CHECK((int)e.graphs_.size() == cap, "%zu of %d kept", e.graphs_.size(), cap);
+  for (int i = cap; i < n; i++) e.graphs_[key(i)] = {nullptr, ++e.graph_clock_};
+  for (int i = 0; i < 10; i++) e.graphs_[key(7 * i)].used = ++e.graph_clock_;   // old ones used again
+  e.trim_graphs();
+  CHECK((int)e.graphs_.size() == cap, "%zu of %d kept", e.graphs_.size(), n);
+  for (int i = 0; i < n; i++) {
+    const bool want = (i % 7 == 0 && i < 70) || i >= n - (cap - 10);
+    CHECK((e.graphs_.count(key(i)) == 1) == want, "entry %d of %d", i, n);
+  }
+  (void)hipGetLastError();
+  printf("ok kept graphs\n");
+}
+
 int main()
 {
+  kept_graphs();
   one_lane();
   control_block();
   for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
