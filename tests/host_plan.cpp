@@ -94,6 +94,22 @@ static void reverse_bound(const char* name, const std::vector<ShotDev>& ds)
   CHECK(p.cached || p.pair > 225e6, "%s: %d shots do not count as cached with %.0f MB", name, nb, p.pair / 1e6);
 }
 
+// the batches of tests/test_gpu_lane_groups.py, which are there for a stream's
+// second and third group
+static void lane_group_jobs()
+{
+  std::vector<ShotDev> ragged;
+  for (int k = 0; k < 121; k++) ragged.push_back(window(61 + 2 * (37 * k % 120), 300, 32));
+  for (const auto& ds : {std::vector<ShotDev>(75, window(301, 300, 32)), ragged}) {
+    const Plan p = plan(ds, PH_REV);
+    bool equal = true;
+    for (auto& g : p.g) equal &= g.size() == p.g[0].size();
+    CHECK(p.g.size() >= 6, "%zu shots in %zu groups", ds.size(), p.g.size());
+    CHECK(!equal, "%zu shots in groups of the same size", ds.size());
+  }
+  printf("ok several groups a stream\n");
+}
+
 // A control block that cannot be allocated (here: there is no GPU) is not
 // counted as there by the next job, which would launch on its addresses; with
 // a GPU both calls succeed.
@@ -162,6 +178,7 @@ int main()
   kept_graphs();
   one_lane();
   control_block();
+  lane_group_jobs();
   for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
     reverse_bound("survey", std::vector<ShotDev>(n, window(301, 512, 50)));
   for (int n : {5, 31, 33, 70, 119}) reverse_bound("narrow", std::vector<ShotDev>(n, window(60 + n, 300, 32)));
