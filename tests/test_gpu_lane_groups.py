@@ -30,8 +30,9 @@ def _job(nshot, ragged, **kw):
     (75, False, 45, dict(graph_chunk=0)),
     (121, True, 55, dict(graph_chunk=20)),
     (121, True, 41, dict(graph_chunk=0)),
-    (75, False, 64, dict(graph_chunk=25, store_fmt=G.STORE_F16, snap_every=20)),
-    (75, False, 45, dict(graph_chunk=0, store_fmt=G.STORE_BF16, snap_every=10, snap_fmt=G.STORE_BF16)),
+    # (snapshots start 4 / (fdom dt) = 160 steps in)
+    (75, False, 231, dict(graph_chunk=50, store_fmt=G.STORE_F16, snap_every=20)),
+    (75, False, 193, dict(graph_chunk=0, store_fmt=G.STORE_BF16, snap_every=10, snap_fmt=G.STORE_BF16)),
     (75, False, 48, dict(graph_chunk=16, ic_extra=True)),
 ])
 def test_several_groups_a_stream(gpu_ctx, nshot, ragged, nt, kw):
