@@ -922,6 +922,7 @@ int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt,
   hipEvent_t ev[3];
   for (auto& e : ev) HIPCHK(hipEventCreate(&e));
   const int kb = phase == PH_FWD ? 0 : 2;
+  const bool after = phase == PH_FWD && (store_fmt != ST_F32 || snap_.on());   // a forward step has launches after it
   for (int s = 0; s < nsteps; s++) {
     a.step = s;
     HIPCHK(hipEventRecord(ev[0], st_));
@@ -936,7 +937,7 @@ int Engine::profile_pass(int phase, int nsteps, Group& g, int tz, int store_fmt,
     HIPCHK(hipEventElapsedTime(&m0, ev[0], ev[1]));
     HIPCHK(hipEventElapsedTime(&m1, ev[1], ev[2]));
     prof->kern_ms[kb] += m0; prof->kern_calls[kb]++;
-    if (phase == PH_FWD) { prof->kern_ms[kb + 1] += m1; prof->kern_calls[kb + 1]++; }
+    if (after) { prof->kern_ms[kb + 1] += m1; prof->kern_calls[kb + 1]++; }
   }
   for (auto& e : ev) (void)hipEventDestroy(e);
   return 0;

@@ -108,7 +108,13 @@ typedef struct rtmh_options {
   int write_files;    /* reproduce the reference's file side effects             */
   int verbose;        /* 0 silent, 1 per-shot lines as the reference prints       */
   double mem_budget;  /* bytes of HBM for shot slots; 0 = 80% of free memory      */
-  int profile;        /* 1: plain launches timed one by one with HIP events       */
+  int profile;        /* 1: every step's launches timed by themselves with HIP
+                         events (rtmh_stats.kern_ms).  Each pass then is one
+                         launch of all shots of a batch per step, on one stream,
+                         with non-temporal field stores and a tile height for
+                         launches of that size: not the groups of shots on two
+                         streams that a pass without it runs in, so the times
+                         are those of the kernels and not parts of such a pass */
   const float *shot_offsetmax; /* per shot (job order) aperture overriding offsetmax
                                   (ragged windows); NULL: offsetmax for every shot */
   /* Checkpoint / resume (no counterpart in the reference, whose temp images
@@ -171,8 +177,9 @@ typedef struct rtmh_stats {
   double cell_updates;      /* 2*nt*nxp*nzp + (nt-1)*nz*nxl summed over shots     */
   int nshots, batches, tile_z, batch;
   double hbm_bytes_alg;     /* algorithmic bytes of the propagation passes        */
-  /* profile=1 only: per kernel (0 forward step, 1 what follows it: the 16-bit
-   * store's quantisation and snapshots, 2 reverse step, 3 unused) summed launch time and launch count */
+  /* profile=1 only: per kernel (0 forward step, 1 what follows it where
+   * something does: the 16-bit store's quantisation and snapshots, 2 reverse
+   * step, 3 unused) summed time and number of steps */
   double kern_ms[4];
   int kern_calls[4];
   double step_bytes_fwd;    /* algorithmic bytes of one forward step of the batch */

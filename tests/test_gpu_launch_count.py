@@ -1,5 +1,6 @@
 """The counters of launches count the launches that are made: a served tick's
-steps, one more after a forward step of a 16-bit store."""
+steps, one more after a forward step of a 16-bit store; a timed pass's forward
+steps, what follows them where something does, and its reverse steps."""
 import numpy as np
 import pytest
 
@@ -31,3 +32,17 @@ def test_served_launches(gpu_ctx, store, forward):
             assert q.launches == forward * nt + (nt - 1)
     finally:
         gpu_ctx.model_destroy(mid)
+
+
+# snapshots start 4 / (fdom dt) = 200 steps in: none is due in 83 steps
+@pytest.mark.parametrize("store,snap,nt,follows", [(G.STORE_F32, 0, 83, False), (G.STORE_F32, 20, 83, False),
+                                                   (G.STORE_F32, 20, 300, True), (G.STORE_F16, 0, 83, True)])
+def test_timed_steps(gpu_ctx, store, snap, nt, follows):
+    P, vp, rho = _job(nt)
+    print(f"[launches] timed, store {store}, snapshots {snap}, nt={nt}", flush=True)
+    r = gpu_ctx.run(P, vp, rho, profile=True, store_fmt=store, snap_every=snap)
+    assert list(r.stats.kern_calls) == [nt, nt if follows else 0, nt - 1, 0]
+    assert (r.stats.kern_ms[1] > 0) == follows
+    assert r.stats.kern_ms[0] > 0 and r.stats.kern_ms[2] > 0 and r.stats.kern_ms[3] == 0
+    ref = gpu_ctx.run(P, vp, rho, store_fmt=store, snap_every=snap)
+    assert np.array_equal(r.image1, ref.image1) and np.array_equal(r.illum, ref.illum)
