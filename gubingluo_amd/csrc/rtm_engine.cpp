@@ -853,20 +853,25 @@ double live_bytes(const ShotDev& d, int phase)
   return phase == PH_FWD ? 4 * (6 * cells + 2 * (cells - in)) : 4 * (12 * cells + 2 * (cells - in) + 2 * in);
 }
 
+static double tiles32(const ShotDev& d) { return (double)((d.nxp + RTM_TX - 1) / RTM_TX) * ((d.nzp + 31) / 32); }
+
 std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int phase, bool& cached)
 {
   const int nb = (int)ds.size();
-  double total = 0, most = 0;
+  double total = 0, most = 0, tiles = 0;
   for (const ShotDev& d : ds) {
     const double b = live_bytes(d, phase);
     total += b;
     most = std::max(most, b);
+    tiles += tiles32(d);
   }
-  const double half = kCacheBytes / 2;
   int n = 1;
   if (nb > 1) {
     n = 2;
-    if (most <= half && phase == PH_REV && total > kPairBytes) n = 2 * (int)std::ceil(total / kCacheBytes);
+    if (phase == PH_REV && most <= kPairMost / 2) {
+      n = 2 * (int)std::ceil(total / kPairBytes);
+      if (most > kPairBytes / 2 || 2 * tiles / n < kRevTall) n = 2 * (int)std::ceil(total / kPairMost);
+    }
     n = std::min(n, nb);
   }
   std::vector<std::vector<int>> g(n);
@@ -886,7 +891,7 @@ std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int ph
     worst = std::max(worst, prev + b);
     prev = b;
   }
-  cached = worst <= 1.15 * kCacheBytes;
+  cached = worst <= kCachedBytes;
   return g;
 }
 
@@ -1536,9 +1541,9 @@ int Engine::run_model(int model_id, const rtmh_params& P, const float* coef, con
       if (opt.tile_z) return opt.tile_z;
       double n = 0;                                    // (groups are of about equal size)
       for (const Group& g : gs)
-        for (int k : g.slots) n += (double)((ds[k].nxp + 63) / 64) * ((ds[k].nzp + 31) / 32);
+        for (int k : g.slots) n += tiles32(ds[k]);
       n *= std::min((double)kLanes / gs.size(), 1.0);
-      return n >= (phase == PH_FWD ? 1000 : 1400) ? 32 : 16;
+      return n >= (phase == PH_FWD ? kFwdTall : kRevTall) ? 32 : 16;
     };
     const int tz = height(gf, PH_FWD), tz_r = height(gr, PH_REV);
     size_t tcap = 0;

@@ -336,28 +336,38 @@ class Engine {
 // in turn fill each other's launch tails, and in the reverse pass a group's
 // fields stay in the cache from step to step: a reverse step works on
 // `live_bytes` of a slot, and a batch is cut into an even number of groups (or
-// one a shot) of about equal size, so that two of them hold kCacheBytes or
-// less; a cut falls between shots, so that a pair may hold one shot more.
-// `cached` allows a pair 15 % over the bound (230 MB).  A forward pass, and
-// shots larger than half the bound, run as two halves: a forward launch of few
-// shots is short while the wavefield is still small and its fixed costs then
-// weigh more than the cache gives.  Measured, ms of the forward and the
-// reverse pass as one group / two halves / cached groups: 48 survey shots (nt
-// 3000) 260, 555 / 222, - / 245, 437; 160 (nt 1000) 174, 638 / 160, - / 201,
-// 531; 16 ragged windows of 400-1600 columns 38, 176 / 34, - / 50, 155; 4
-// shots of 2148 x 1124 (nt 1200) 52, 194 / 51, 187 / 95, -.
-// The bound: strips, model and images come on top of the fields.  us per
-// reverse step of survey shots at 200 / 235 MB where the plans differ, their
-// largest pairs in brackets: 32 shots 108 (151 MB) / 111 (220), 34 113 (165) /
-// 126 (234), 64 210 (179) / 225 (220), 100 333 (206) / 370 (234), 160 529
-// (206) / 555 (220), 200 644 (193) / 682 (224).
-// A batch that is one pair keeps a little more, since nothing else goes
-// through the cache and four groups would be launches of half the size.  us
-// per reverse step as two groups / as four, 13.7 MB survey shots and others:
-// 206 MB 52 / 56, 214 MB 66 / 67, 216 MB 54 / 58, 220 MB 57 / 56, 227 MB 75 /
-// 71, 234 MB 66 / 62; with every imaging condition 206 MB 76 / 83, 220 MB 80 /
-// 86, 234 MB 85 / 91.
-constexpr double kCacheBytes = 200e6, kPairBytes = 225e6;
+// one a shot) of about equal size, so that two of them hold kPairBytes or less
+// on average; a cut falls between shots, so that a pair may hold one shot more.
+// A forward pass, and shots too large for that, run as two halves: a forward
+// launch of few shots is short while the wavefield is still small and its
+// fixed costs then weigh more than the cache gives.  Measured, ms of the
+// forward and the reverse pass as one group / two halves / cached groups: 48
+// survey shots (nt 3000) 260, 555 / 222, - / 245, 437; 160 (nt 1000) 174, 638 /
+// 160, - / 201, 531; 16 ragged windows of 400-1600 columns 38, 176 / 34, - /
+// 50, 155; 4 shots of 2148 x 1124 (nt 1200) 52, 194 / 51, 187 / 95, -.
+// kPairBytes: strips, model and images come on top of the fields.  us per
+// reverse step of survey shots with pairs of 200 / 235 MB where the plans
+// differ, their largest pairs in brackets: 32 shots 108 (151 MB) / 111 (220),
+// 34 113 (165) / 126 (234), 64 210 (179) / 225 (220), 100 333 (206) / 370
+// (234), 160 529 (206) / 555 (220), 200 644 (193) / 682 (224).
+// kPairMost: a pair holds more where the other plan is worse still, which is
+// where it would leave fewer tiles in flight than 32-row tiles need (kRevTall),
+// or where a shot is larger than half of kPairBytes and the other plan is two
+// halves past the cache.  ms of reverse passes of nt 600 at 200 / 235 MB, fewer
+// tiles: 4 shots, 227 MB in all 37.4 / 30.9, 3 of 76 MB 40.2 / 37.5, 23 ragged,
+// 415 MB 63.8 / 59.4, 29, 425 MB 71.5 / 68.4, 22 with every imaging condition,
+// 230 MB 58.3 / 55.1; large shots: 4 of 112 MB 75.1 / 68.3, 3 of 103 MB 58.4 /
+// 52.5.  With enough tiles the smaller pairs won there too: 32 shots, 447 MB
+// 66.0 / 73.2, 40, 466 MB 66.9 / 72.6, 33, 461 MB 63.7 / 67.8.
+// kCachedBytes: `cached`, ordinary stores, up to that in two neighbours (the
+// lanes go on by themselves, but through groups of about equal size).  ms of
+// forward passes of nt 600 as halves of 232-268 MB together, ordinary stores /
+// with the hint: 13 shots 16.1 / 17.5, 23 15.6 / 17.7, 28 19.0 / 23.0, 64 28.9 /
+// 32.0.
+constexpr double kPairBytes = 200e6, kPairMost = 235e6, kCachedBytes = 270e6;
+// 32-row tiles in flight from which a forward / a reverse pass takes 32 rows
+// (Engine::run_model says what was measured)
+constexpr int kFwdTall = 1000, kRevTall = 1400;
 double live_bytes(const ShotDev& d, int phase);
 std::vector<std::vector<int>> plan_groups(const std::vector<ShotDev>& ds, int phase, bool& cached);
 

@@ -554,8 +554,8 @@ void Server::rebuild_tiles()
   join();                                            // steps in flight read the tables
   qslots_.clear();
   aslots_.clear();
-  // ordinary stores while everything resident fits the Infinity Cache (the
-  // batch engine's bound for its groups): six requests of up to nine shots on
+  // ordinary stores while everything resident fits the Infinity Cache (what a
+  // pair of the batch engine's groups holds at most): six requests of up to nine shots on
   // three models of 512 x 384 and less took 92 ms with the non-temporal hint,
   // 82 without
   double live = 0, total = 0;
@@ -568,7 +568,7 @@ void Server::rebuild_tiles()
       live += live_bytes(hds_[i], slots_[i].phase);
       total += work(i);
     }
-  fits_ = live <= kCacheBytes;
+  fits_ = live <= kPairMost;
   std::stable_partition(aslots_.begin(), aslots_.end(), [&](int i) { return slots_[i].phase == PH_FWD; });
   tiles_.clear();
   double done = 0;

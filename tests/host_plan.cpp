@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <condition_variable>
 #include <functional>
 #include <map>
@@ -74,24 +75,51 @@ static bool whole(const Plan& p, int n)
   return at == n;
 }
 
-// the reverse pass: two neighbouring groups hold at most 200 MB and one shot
-// (the cuts fall between shots), or are the whole pass and hold at most 225 MB
+// The reverse pass.  Two neighbouring groups hold 200 MB on average, or 235
+// where 200 would leave fewer than 1400 32-row tiles in flight or a shot is
+// larger than 100 MB; with one shot more where a cut falls between shots.
 static void reverse_bound(const char* name, const std::vector<ShotDev>& ds)
 {
   const Plan p = plan(ds, PH_REV);
   const int nb = (int)ds.size(), n = (int)p.g.size();
   CHECK(whole(p, nb), "%s: %d shots, %d groups", name, nb, n);
   CHECK(nb == 1 ? n == 1 : n % 2 == 0 || n == nb, "%s: %d groups of %d shots", name, n, nb);
-  if (p.most <= 100e6) {
-    const double bound = n == 2 && p.total <= 225e6 ? 225e6 : 200e6 + p.most;
-    CHECK(p.pair <= bound, "%s: %d shots in %d groups, a pair holds %.0f MB of at most %.0f", name, nb, n, p.pair / 1e6,
-          bound / 1e6);
+  double tiles = 0;
+  for (const ShotDev& d : ds) tiles += (double)((d.nxp + 63) / 64) * ((d.nzp + 31) / 32);
+  auto groups = [&](double bound) { return std::min(nb, 2 * (int)std::ceil(p.total / bound)); };
+  if (nb > 1 && p.most <= 117.5e6) {
+    const bool few = 2 * tiles / (2 * std::ceil(p.total / 200e6)) < 1400 || p.most > 100e6;
+    CHECK(n == groups(few ? 235e6 : 200e6), "%s: %d shots of %.0f MB, %.0f tiles, in %d groups", name, nb, p.total / 1e6,
+          tiles, n);
+    CHECK(p.pair <= (few ? 235e6 : 200e6) + p.most, "%s: %d shots in %d groups, a pair holds %.0f MB", name, nb, n,
+          p.pair / 1e6);
   } else {
     CHECK(n == std::min(2, nb), "%s: %d groups of large shots", name, n);
   }
-  // 256 MB of cache
-  CHECK(!p.cached || p.pair <= 230e6, "%s: %d shots count as cached with %.0f MB", name, nb, p.pair / 1e6);
-  CHECK(p.cached || p.pair > 225e6, "%s: %d shots do not count as cached with %.0f MB", name, nb, p.pair / 1e6);
+  CHECK(p.cached == (p.pair <= 270e6), "%s: %d shots, %.0f MB, cached %d", name, nb, p.pair / 1e6, (int)p.cached);
+}
+
+// Plans on both sides of each of these lines: equal windows, their number and
+// the groups that were the faster ones (rtm_engine.h).
+static void known_plans()
+{
+  struct { int nxl, nzi, npml, shots, groups; } t[] = {
+    {301, 512, 50, 16, 2},  {301, 512, 50, 32, 6},   {301, 512, 50, 34, 6},  {301, 512, 50, 64, 10},
+    {301, 512, 50, 100, 14}, {301, 512, 50, 160, 22}, {301, 512, 50, 200, 28},
+    {1431, 562, 50, 4, 2},  {1764, 970, 50, 4, 4},   {1953, 792, 50, 3, 3},  {2048, 1024, 50, 4, 2},
+  };
+  for (auto& k : t) {
+    const Plan p = plan(std::vector<ShotDev>(k.shots, window(k.nxl, k.nzi, k.npml)), PH_REV);
+    CHECK((int)p.g.size() == k.groups, "%d shots of %d x %d (%.0f MB): %zu groups, not %d", k.shots, k.nxl, k.nzi,
+          p.total / 1e6, p.g.size(), k.groups);
+  }
+  // forward halves keep ordinary stores up to 270 MB together
+  for (int n : {20, 40, 60}) {
+    const Plan f = plan(std::vector<ShotDev>(n, window(301, 512, 50)), PH_FWD);
+    CHECK(f.g.size() == 2 && f.cached == (f.total <= 270e6), "%d shots forward, %.0f MB, cached %d", n, f.total / 1e6,
+          (int)f.cached);
+  }
+  printf("ok known plans\n");
 }
 
 // the batches of tests/test_gpu_lane_groups.py, which are there for a stream's
@@ -179,6 +207,7 @@ int main()
   one_lane();
   control_block();
   lane_group_jobs();
+  known_plans();
   for (int n : {1, 2, 3, 15, 16, 17, 20, 32, 33, 34, 64, 100, 128, 160, 200, 256})
     reverse_bound("survey", std::vector<ShotDev>(n, window(301, 512, 50)));
   for (int n : {5, 31, 33, 70, 119}) reverse_bound("narrow", std::vector<ShotDev>(n, window(60 + n, 300, 32)));
