@@ -36,7 +36,7 @@ single-shot configuration (400x200, nt 2000) and on survey shots.
 Other workloads (one JSON line each, same keys):
   --workload batched    2048x768, 256 shots with per-shot aperture windows
                         U[400,1600] columns, 64 shots per launch, hipGraph
-                        time loop, autotuned tile height
+                        time loop, tile heights by size
   --workload precision  2048x1024 dx=7.5 m nt=6000 25 Hz: throughput with
                         FP32 / FP16 / BF16 boundary stores, and the image
                         error of each against the FP64 CPU oracle
@@ -148,8 +148,9 @@ def cpu_baseline(P_full, vp, rho, synth, quick=False, keep=None):
 
 
 def traffic_ratio(kernel):
-    """HBM bytes / algorithmic bytes of a step kernel, measured offline with
-    rocprofv3 FETCH_SIZE / WRITE_SIZE (profiles/step_kernel_traffic.json)."""
+    """Bytes past the L2s / algorithmic bytes of a step kernel, measured offline
+    with rocprofv3 FETCH_SIZE / WRITE_SIZE (profiles/step_kernel_traffic.json).
+    Reads that the Infinity Cache serves are among them: not HBM bytes."""
     try:
         with open(os.path.join(ROOT, "profiles", "step_kernel_traffic.json")) as f:
             return float(json.load(f)[kernel]["traffic_over_algorithmic"])
@@ -158,12 +159,14 @@ def traffic_ratio(kernel):
 
 
 def roofline_of(recs, P, copy_gbs=None):
-    """Dominant kernel: the reverse time step k_rev (one launch per step:
-    reconstruction, receiver wavefield, imaging), timed by HIP events on the
-    engine's stream around every reverse pass of the timed region; the
-    algorithmic bytes come from the per-cell figures (engine stats
-    rev_bytes_alg: all reverse steps of all batches), so a launch's average
-    is exact also when the batches of a step differ in size."""
+    """Dominant kernel: the reverse time step k_rev (reconstruction, receiver
+    wavefield, imaging), timed by HIP events on the engine's stream around
+    every reverse pass of the timed region.  A step is the launches of all its
+    groups of shots, two at a time on two streams.  The algorithmic bytes come
+    from the per-cell figures (engine stats rev_bytes_alg: all reverse steps of
+    all batches), so a step's average is exact also when batches differ in
+    size.  `achieved` is that work per time: the groups in flight keep their
+    fields in the Infinity Cache, so less than it moves through HBM."""
     rev_steps = sum(s.batches * (P.nt - 1) for s, _, _ in recs)
     rev_ms = sum(s.rev_ms for s, _, _ in recs)
     # totals over every batch of every step (batches may differ in size)
@@ -178,14 +181,15 @@ def roofline_of(recs, P, copy_gbs=None):
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": None if ratio is None else round(ratio * step_bytes),
             "traffic_source": None if ratio is None else
-            f"HBM/algorithmic bytes {ratio} of k_rev from rocprofv3 FETCH_SIZE+WRITE_SIZE "
-            "(profiles/k_fwd_k_rev_survey200_traffic.md) times this run's algorithmic bytes",
+            f"bytes past the L2s (Infinity Cache hits included) / algorithmic bytes {ratio} of a k_rev step from "
+            "rocprofv3 FETCH_SIZE+WRITE_SIZE (profiles/k_fwd_k_rev_survey200_traffic.md) times this run's "
+            "algorithmic bytes",
             "copy_gbs": None if copy_gbs is None else round(copy_gbs, 1),
             "kernel": "k_rev (reverse time step: reconstruction + receiver wavefield + imaging)",
-            "avg_launch_us": round(avg_step_s * 1e6, 2), "alg_bytes_per_launch": step_bytes,
+            "avg_step_us": round(avg_step_s * 1e6, 2), "alg_bytes_per_step": step_bytes,
             "forward_step": {"kernel": "k_fwd", "achieved": round(fwd_bytes / (fwd_ms * 1e-3 / fwd_steps) / 1e9, 1),
-                             "avg_launch_us": round(fwd_ms * 1e3 / fwd_steps, 2),
-                             "alg_bytes_per_launch": fwd_bytes,
+                             "avg_step_us": round(fwd_ms * 1e3 / fwd_steps, 2),
+                             "alg_bytes_per_step": fwd_bytes,
                              "note": "bytes of every tile of the step; tiles whose forward field is still +0 "
                                      "around them skip the step and move none of theirs, so this rate is the "
                                      "step's work per time, not an HBM rate"}}
@@ -283,8 +287,8 @@ def run_survey(args, G, synth):
 # ------------------------------------------------------ configuration subs --
 def batched_sub(args, G, synth, ctx):
     """One 64-shot launch batch of the ragged 2048x768 survey (windows drawn
-    from 400-1600 columns), graph chunk 50, autotuned tile heights: one
-    untimed batch (it tunes), then one timed."""
+    from 400-1600 columns), graph chunk 50, tile heights by size: one
+    untimed batch (it captures the graphs), then one timed."""
     P, vp, rho, om = synth.batched_ragged()
     if args.nt:
         P.nt = args.nt
@@ -300,7 +304,7 @@ def batched_sub(args, G, synth, ctx):
     widths = [int(np.floor(om[i] / P.dx + 1)) for i in range(64)]
     out = {"workload": f"batched RTM, 2048x768 dx=10 m, shots 1-64 of 256 every 80 m, windows U[400,1600] "
                        f"columns (drawn {min(widths)}..{max(widths)}, clipped at the edges), nt={P.nt}, "
-                       f"64 shots per launch batch, graph chunk {args.chunk}, autotuned tile heights",
+                       f"64 shots per launch batch, graph chunk {args.chunk}, tile heights by size",
            "value": round(r.stats.cell_updates / dt / 1e9, 3), "unit": "Gcell/s", "seconds": round(dt, 3),
            "shots_per_hour": round(64 / dt * 3600.0, 1), "tile_z": r.stats.tile_z, "tile_z_rev": r.stats.tile_z_rev,
            "k_rev_achieved_gbs": roof["achieved"], "k_rev_frac": roof["frac"]}
@@ -312,7 +316,7 @@ def single_sub(args, G, synth, ctx):
     """The reference's CPU-runnable case on the GPU: one shot of the
     single-shot anomaly model (400x200, npml 40, nt 2000), as the plain form
     (one shot per launch, per-step launches, FP32 boundaries, 16-row tiles)
-    and as the default engine (graph chunk, autotuned tile heights); one
+    and as the default engine (graph chunk, tile heights by size); one
     untimed run of each, then one timed."""
     P, vp, rho = synth.single_shot_anomaly()
     mid = ctx.model_create(vp, rho)
@@ -713,7 +717,7 @@ def main():
     ap.add_argument("--batch", type=int, default=0, help="shots per launch (0: all shots of the step)")
     ap.add_argument("--store", default="f32", choices=["f32", "f16", "bf16"])
     ap.add_argument("--chunk", type=int, default=50, help="time steps per replayed hipGraph (0: plain launches)")
-    ap.add_argument("--tz", type=int, default=0, help="tile height 16/32/64 (0: autotuned)")
+    ap.add_argument("--tz", type=int, default=0, help="tile height 16/32/64 (0: by size)")
     ap.add_argument("--nt", type=int, default=0, help="override nt (shorter runs)")
     ap.add_argument("--requests", type=int, default=50, help="serve: requests in the stream")
     ap.add_argument("--plain-requests", type=int, default=8,
